@@ -106,20 +106,23 @@ __global__ __launch_bounds__(256) void embed_bwd_chain_kernel(float *__restrict_
 // rows of D <= 2048 floats.  Per-row sums go through a fixed-order block reduction.
 constexpr int RMS_NT = 256, RMS_VPT = 2;
 
-// Sum over the block of one value per thread: wave sums, then the 4 wave totals in wave order.
-// `red` alternates between two slots by row parity so consecutive rows need one barrier each.
-__device__ __forceinline__ float block_sum_row(float v, float (*red)[RMS_NT / 64], int slot) {
+// Sum over a row group (the RMS_NT threads that own a row; a block holds RG of them) of one value
+// per thread: wave sums, then the 4 wave totals in wave order.  `red` alternates between two slots
+// by row parity so consecutive rows need one barrier each.
+template <int RG = 1>
+__device__ __forceinline__ float block_sum_row(float v, float (*red)[RG * RMS_NT / 64], int slot) {
   v = wave_sum(v);
   if ((threadIdx.x & 63) == 0) red[slot][threadIdx.x >> 6] = v;
   lds_barrier();  // waits for the LDS writes only: global loads issued earlier stay in flight
-  return red[slot][0] + red[slot][1] + red[slot][2] + red[slot][3];
+  const float *r = &red[slot][RG > 1 ? (threadIdx.x / RMS_NT) * (RMS_NT / 64) : 0];
+  return r[0] + r[1] + r[2] + r[3];
 }
 
 // Row `row` of a split-K result, columns t and t + 256 (as float4): base + alpha * sum_z part[z].
 // The partials are added in z order (the GEMM's own reduction order) with the loads of four
 // consecutive z issued together.
 __device__ __forceinline__ void split_row(const SplitIn &sp, long row, int D, float4 (&o)[RMS_VPT]) {
-  const int D4 = D / 4, t = threadIdx.x;
+  const int D4 = D / 4, t = threadIdx.x % RMS_NT;
   const float4 *p = (const float4 *)(sp.part + row * D);
   const long sl = sp.slice / 4;
 #pragma unroll
@@ -213,18 +216,25 @@ __global__ __launch_bounds__(RMS_NT) void rmsnorm_fwd_kernel(float *__restrict__
 // Replaces TD/cpu_ops.h:108-261 (rmsnorm_bwd / rmsnorm_bwd_add).  With REF the
 // reference's own formula is used instead, dx = (dy - x*r^2*sum(dy*x*g)/D)*r*g
 // (TD/cpu_ops.h:146-153, 188-189, 255-256), whose projection term carries one more
-// factor g than the exact gradient; both agree while every gain is 1.  A block walks
-// rows_per_block rows; each thread keeps the gain-gradient sums of its own columns and
-// writes them as the block's partial row (or adds them atomically without `part`).  With
-// split-K partials (sp.n > 0) dy is formed from them.
-template <typename HT, bool REF>
-__global__ __launch_bounds__(RMS_NT) void rmsnorm_bwd_kernel(
+// factor g than the exact gradient; both agree while every gain is 1.  A block holds RG row
+// groups of RMS_NT threads and walks rows_per_block rows, RG at a time; each thread keeps the
+// gain-gradient sums of its own columns.  With `part` they are the block's partial row (RG = 1),
+// reduced in block order by colsum_kernel.  Without it (the kernel entry point has no scratch)
+// the groups' sums meet in LDS in group order and the block adds its D sums to dg with atomics:
+// those are what bounds that form, about 22 ns for each operation on a 128-byte line, one
+// after the other whatever block issues them.  So few blocks (RG = 4, at most 256 of them) and
+// consecutive lanes on consecutive columns: one operation per line and block instead of 4 (one
+// float of each lane's float4 at a time) from 1024 blocks.  Entry point, D = 1024: 16,384 rows
+// 135 -> 49 us (302 MB: 6.1 TB/s), 2048 rows 105 -> 14 us, 256 rows 27 -> 4.7 us.  With split-K partials
+// (sp.n > 0) dy is formed from them.
+template <typename HT, bool REF, int RG>
+__global__ __launch_bounds__(RG * RMS_NT) void rmsnorm_bwd_kernel(
     const float *__restrict__ dy, const float *__restrict__ x, const float *__restrict__ g,
     const float *__restrict__ rr, const float *__restrict__ resid, float *__restrict__ dx,
     h16_t *__restrict__ dxb, float bscale, float *__restrict__ dg, float dg_scale, int T, int D,
     int rows_per_block, int *ovf, float *__restrict__ part, SplitIn sp) {
-  __shared__ float red[2][RMS_NT / 64];
-  const int t = threadIdx.x, D4 = D / 4;
+  __shared__ float red[2][RG * RMS_NT / 64];
+  const int t = threadIdx.x % RMS_NT, grp = threadIdx.x / RMS_NT, D4 = D / 4;
   float4 acc[RMS_VPT], gw[RMS_VPT];
   const float4 *gv = (const float4 *)g;
 #pragma unroll
@@ -258,8 +268,11 @@ __global__ __launch_bounds__(RMS_NT) void rmsnorm_bwd_kernel(
     }
     ro = rr[row];
   };
-  if (r0 < r1) load_row(r0, dyv, xv, rsv, r);
-  for (int row = r0; row < r1; row++) {
+  // every group takes every step (the row sums share a barrier); a group past the last row (RG > 1)
+  // repeats that row and stores nothing
+  if (r0 < r1) load_row(min(r0 + grp, r1 - 1), dyv, xv, rsv, r);
+  for (int row0 = r0, step = 0; row0 < r1; row0 += RG, step++) {
+    const int row = row0 + grp;
     float dot = 0.f;
 #pragma unroll
     for (int j = 0; j < RMS_VPT; j++)
@@ -267,15 +280,16 @@ __global__ __launch_bounds__(RMS_NT) void rmsnorm_bwd_kernel(
              dyv[j].w * xv[j].w * gw[j].w;
     float4 dyn[RMS_VPT], xn[RMS_VPT], rsn[RMS_VPT];
     float rn = 0.f;
-    if (row + 1 < r1) load_row(row + 1, dyn, xn, rsn, rn);
-    dot = block_sum_row(dot, red, row & 1);
+    const bool more = row0 + RG < r1;
+    if (more) load_row(min(row + RG, r1 - 1), dyn, xn, rsn, rn);
+    dot = block_sum_row<RG>(dot, red, step & 1);
     const float c = REF ? r * r * dot * invD : r * r * r * dot * invD;
     float4 *dxr = (float4 *)(dx + (long)row * D);
     u16x4 *dbr = dxb ? (u16x4 *)(dxb + (long)row * D) : nullptr;
 #pragma unroll
     for (int j = 0; j < RMS_VPT; j++) {
       const int i = t + RMS_NT * j;
-      if (i < D4) {
+      if (i < D4 && (RG == 1 || row < r1)) {
         const float4 w = gw[j];
         float4 o;
         if (REF) {
@@ -308,7 +322,7 @@ __global__ __launch_bounds__(RMS_NT) void rmsnorm_bwd_kernel(
         acc[j].w += dyv[j].w * xv[j].w * r;
       }
     }
-    if (row + 1 < r1) {
+    if (more) {
 #pragma unroll
       for (int j = 0; j < RMS_VPT; j++) {
         dyv[j] = dyn[j];
@@ -319,19 +333,26 @@ __global__ __launch_bounds__(RMS_NT) void rmsnorm_bwd_kernel(
     }
   }
   flag_overflow(ovf, bad);
+  if constexpr (RG == 1) {
 #pragma unroll
-  for (int j = 0; j < RMS_VPT; j++) {
-    const int i = t + RMS_NT * j;
-    if (i < D4) {
-      const float4 v = make_float4(dg_scale * acc[j].x, dg_scale * acc[j].y, dg_scale * acc[j].z, dg_scale * acc[j].w);
-      if (part) {
-        *(float4 *)(part + (long)blockIdx.x * D + 4 * i) = v;  // reduced in block order by colsum_kernel
-      } else {
-        atomicAdd(dg + 4 * i, v.x);
-        atomicAdd(dg + 4 * i + 1, v.y);
-        atomicAdd(dg + 4 * i + 2, v.z);
-        atomicAdd(dg + 4 * i + 3, v.w);
-      }
+    for (int j = 0; j < RMS_VPT; j++) {
+      const int i = t + RMS_NT * j;
+      if (i < D4)
+        *(float4 *)(part + (long)blockIdx.x * D + 4 * i) =
+            make_float4(dg_scale * acc[j].x, dg_scale * acc[j].y, dg_scale * acc[j].z, dg_scale * acc[j].w);
+    }
+  } else {
+    constexpr int DMAX = 4 * RMS_NT * RMS_VPT;
+    __shared__ __attribute__((aligned(16))) float comb[RG][DMAX];
+#pragma unroll
+    for (int j = 0; j < RMS_VPT; j++)
+      if (t + RMS_NT * j < D4) *(float4 *)&comb[grp][4 * (t + RMS_NT * j)] = acc[j];
+    __syncthreads();
+    for (int i = threadIdx.x; i < D; i += RG * RMS_NT) {
+      float v = comb[0][i];
+#pragma unroll
+      for (int k = 1; k < RG; k++) v += comb[k][i];
+      atomicAdd(dg + i, dg_scale * v);
     }
   }
 }
@@ -535,108 +556,171 @@ __global__ __launch_bounds__(256) void qk_prep_fwd_kernel(h16_t *__restrict__ qk
   flag_overflow(ovf_qkv, bad);
 }
 
-// Backward of qk_prep: inverse rotation (TD/cpu_ops.h:510-537), then the exact
-// per-head RMSNorm backward; gain gradients reduced per block, one atomic per channel.
-// Block = 256 threads = 256/(HD/2) token rows of one head slot; grid.y = head slot.
-template <typename HT, bool QKN>
+// Backward of qk_prep: inverse rotation (TD/cpu_ops.h:510-537), then the exact per-head RMSNorm
+// backward.  HBM-bound: reads dq, dk (fp32) and the q and k columns of qkv, writes their
+// columns of dqkv.  A head slot (one head of one token) is HD/8 consecutive lanes owning 8
+// elements each, so every access is 16 bytes; a block takes tok_per_block tokens and its slots run
+// over the (token, head) items of those, so a lane meets the same 8 columns of a head every time
+// and keeps their q- and k-gain sums in registers for the whole block: they meet in LDS once, at its
+// end, and leave as one partial row of q and one of k per block (reduced by colsum_kernel) or,
+// without `part` (the kernel entry point has no scratch), as one atomic per channel and block.
+// Before (one head per block, 8-byte accesses, the atomics of every head's blocks on the same
+// lines, about 22 ns each, one after the other) the entry point took 171 us for 16,384 tokens of
+// 16 + 8 heads of 128, 697 us for 3,264 tokens and 53 us for 256; now 96 (408 MB: 4.2 TB/s), 25 and
+// 8.5 us.  In a training step (partial rows, no atomics) 256 tokens take the same 5.9 us.
+// With kvpart (per-query-head dK/dV partials, [2][T, NH*HD]) a k slot sums its query heads'
+// dK partials in head order, and NKV further slots per token sum dV into dqkv's v columns.
+template <typename HT, bool QKN, int HD>
 __global__ __launch_bounds__(256) void qk_prep_bwd_kernel(
     const float *__restrict__ dq, const float *__restrict__ dk, const h16_t *__restrict__ qkv, long ld,
     const float *__restrict__ cosb, const float *__restrict__ sinb, const float *__restrict__ gq,
     const float *__restrict__ gk, const float *__restrict__ rq, const float *__restrict__ rk,
     h16_t *__restrict__ dqkv, float *__restrict__ dgq, float *__restrict__ dgk, float dg_scale, int T,
-    int S, int NH, int NKV, int HD, int tok_per_block, int *ovf, float *__restrict__ part,
+    int S, int NH, int NKV, int tok_per_block, int *ovf, float *__restrict__ part,
     const float *__restrict__ kvpart, int *ovf_v) {
-  bool bad = false;
-  __shared__ float red[256 * 2];
-  const int half = HD / 2;
-  const int i = threadIdx.x % half;
-  const int sub = threadIdx.x / half, nsub = 256 / half;
-  const int h = blockIdx.y;
+  constexpr int TPH = HD / 8, HALF = HD / 2, SPB = 256 / TPH;  // lanes per slot, slots per block
+  const int j = threadIdx.x % TPH;
   const int ratio = NH / NKV;
-  if (h >= NH + NKV) {
-    // dV of kv head h - NH - NKV: the head-order sum of its query heads' partials (kvpart's
-    // second half), rounded to 16 bits into dqkv's v columns
-    const int kvh = h - NH - NKV;
-    const float *pv = kvpart + (long)T * NH * HD;
-    const long t0 = (long)blockIdx.x * tok_per_block, t1 = min((long)T, t0 + tok_per_block);
-    for (long t = t0 + sub; t < t1; t += nsub) {
-      float2 sv = make_float2(0.f, 0.f);
-      for (int r = 0; r < ratio; r++) {
-        const float2 y = *(const float2 *)(pv + t * NH * HD + (long)(kvh * ratio + r) * HD + 2 * i);
-        sv.x += y.x; sv.y += y.y;
-      }
-      const h16_t o0 = HT::h(sv.x), o1 = HT::h(sv.y);
-      bad |= HT::bad(o0) | HT::bad(o1);
-      *(uint32_t *)(dqkv + t * ld + (long)(NH + NKV) * HD + (long)kvh * HD + 2 * i) = (uint32_t)o0 | ((uint32_t)o1 << 16);
-    }
-    flag_overflow(ovf_v, bad);
-    return;
+  const int slots = kvpart ? NH + 2 * NKV : NH + NKV;
+  const int t0 = blockIdx.x * tok_per_block, nt = min(tok_per_block, T - t0);
+  bool bad = false, bad_v = false;
+  float gqv[8], gkv[8], aq[8], ak[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    aq[e] = ak[e] = 0.f;
+    gqv[e] = QKN ? gq[8 * j + e] : 0.f;
+    gkv[e] = QKN ? gk[8 * j + e] : 0.f;
   }
-  const bool isq = h < NH;
-  const int hh = isq ? h : h - NH;
-  const long col = (isq ? 0 : (long)NH * HD) + (long)hh * HD + 2 * i;
-  const float *gg = isq ? gq : gk;
-  float g0 = 0.f, g1 = 0.f;
-  if (QKN) {
-    g0 = gg[2 * i];
-    g1 = gg[2 * i + 1];
-  }
-  float a0 = 0.f, a1 = 0.f;
-  const long t0 = (long)blockIdx.x * tok_per_block;
-  const long t1 = min((long)T, t0 + tok_per_block);
-  for (long t = t0 + sub; t < t1; t += nsub) {
-    float2 dd;
-    if (isq) {
-      dd = *(const float2 *)(dq + t * (long)NH * HD + (long)hh * HD + 2 * i);
-    } else if (kvpart) {  // dK: the head-order sum of the query heads' partials
-      dd = make_float2(0.f, 0.f);
-      for (int r = 0; r < ratio; r++) {
-        const float2 y = *(const float2 *)(kvpart + t * (long)NH * HD + (long)(hh * ratio + r) * HD + 2 * i);
-        dd.x += y.x; dd.y += y.y;
-      }
+  // An item's loads are issued before the item before it is worked on: two items, and for GQA
+  // partials two query heads of each, are in flight per lane.
+  struct Item {
+    float4 d[2][2];  // dq / dk, or the partials of the first two query heads
+    float4 c4, s4;
+    u16x8 pr;
+    float r;
+  };
+  const int n = nt * slots;
+  auto place = [&](int w, long &t, int &h, int &hh, long &col) {
+    t = t0 + w / slots;
+    h = w % slots;
+    hh = h < NH ? h : h < NH + NKV ? h - NH : h - NH - NKV;
+    col = (h < NH ? 0 : h < NH + NKV ? (long)NH * HD : (long)(NH + NKV) * HD) + (long)hh * HD + 8 * j;
+  };
+  auto partials = [&](long t, int h, int hh) {
+    return kvpart + (h >= NH + NKV ? (long)T * NH * HD : 0) + t * (long)NH * HD + (long)hh * ratio * HD + 8 * j;
+  };
+  auto load = [&](int w, Item &it) {
+    long t, col;
+    int h, hh;
+    place(w, t, h, hh, col);
+    const bool isq = h < NH;
+    const float *p = isq      ? dq + t * (long)NH * HD + (long)hh * HD + 8 * j
+                     : kvpart ? partials(t, h, hh)
+                              : dk + t * (long)NKV * HD + (long)hh * HD + 8 * j;
+    it.d[0][0] = *(const float4 *)p;
+    it.d[0][1] = *(const float4 *)(p + 4);
+    if (!isq && kvpart && ratio > 1) {
+      it.d[1][0] = *(const float4 *)(p + HD);
+      it.d[1][1] = *(const float4 *)(p + HD + 4);
     } else {
-      dd = *(const float2 *)(dk + t * (long)NKV * HD + (long)hh * HD + 2 * i);
+      it.d[1][0] = it.d[1][1] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    const int pos = t % S;
-    const float c = cosb[pos * half + i], s = sinb[pos * half + i];
-    float d0 = dd.x * c + dd.y * s;
-    float d1 = dd.y * c - dd.x * s;
+    if (h >= NH + NKV) return;
+    const long pos = t % S;
+    it.c4 = *(const float4 *)(cosb + pos * HALF + 4 * j);
+    it.s4 = *(const float4 *)(sinb + pos * HALF + 4 * j);
     if (QKN) {
-      const uint32_t pr = *(const uint32_t *)(qkv + t * ld + col);
-      const float x0 = HT::f((h16_t)(pr & 0xFFFF)), x1 = HT::f((h16_t)(pr >> 16));
-      const float r = isq ? rq[t * NH + hh] : rk[t * NKV + hh];
-      float dot = d0 * x0 * g0 + d1 * x1 * g1;
-      dot = half == 64 ? group_sum<64>(dot) : group_sum<32>(dot);  // HD = 128 or 64
-      const float cc = r * r * r * dot / (float)HD;
-      a0 += d0 * x0 * r;
-      a1 += d1 * x1 * r;
-      d0 = r * g0 * d0 - x0 * cc;
-      d1 = r * g1 * d1 - x1 * cc;
+      it.pr = *(const u16x8 *)(qkv + t * ld + col);
+      it.r = isq ? rq[t * NH + hh] : rk[t * NKV + hh];
     }
-    const h16_t o0 = HT::h(d0), o1 = HT::h(d1);
-    bad |= HT::bad(o0) | HT::bad(o1);
-    *(uint32_t *)(dqkv + t * ld + col) = (uint32_t)o0 | ((uint32_t)o1 << 16);
+  };
+  // whole head slots are active or idle together, so the sums below stay within a slot
+  auto finish = [&](int w, const Item &it) {
+    long t, col;
+    int h, hh;
+    place(w, t, h, hh, col);
+    const bool isq = h < NH;
+    float d[8] = {it.d[0][0].x + it.d[1][0].x, it.d[0][0].y + it.d[1][0].y, it.d[0][0].z + it.d[1][0].z,
+                  it.d[0][0].w + it.d[1][0].w, it.d[0][1].x + it.d[1][1].x, it.d[0][1].y + it.d[1][1].y,
+                  it.d[0][1].z + it.d[1][1].z, it.d[0][1].w + it.d[1][1].w};
+    if (!isq && kvpart)
+      for (int r = 2; r < ratio; r++) {
+        const float *p = partials(t, h, hh) + (long)r * HD;
+        const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 4);
+        d[0] += a.x; d[1] += a.y; d[2] += a.z; d[3] += a.w;
+        d[4] += b.x; d[5] += b.y; d[6] += b.z; d[7] += b.w;
+      }
+    u16x8 o;
+    if (h >= NH + NKV) {
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        o[e] = HT::h(d[e]);
+        bad_v |= HT::bad(o[e]);
+      }
+      *(u16x8 *)(dqkv + t * ld + col) = o;
+      return;
+    }
+    const float cv[4] = {it.c4.x, it.c4.y, it.c4.z, it.c4.w}, sv[4] = {it.s4.x, it.s4.y, it.s4.z, it.s4.w};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const float d0 = d[2 * q] * cv[q] + d[2 * q + 1] * sv[q];
+      const float d1 = d[2 * q + 1] * cv[q] - d[2 * q] * sv[q];
+      d[2 * q] = d0;
+      d[2 * q + 1] = d1;
+    }
+    if (QKN) {
+      const float r = it.r;
+      float x[8], dot = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        x[e] = HT::f(it.pr[e]);
+        dot += d[e] * x[e] * (isq ? gqv[e] : gkv[e]);
+      }
+      dot = group_sum<TPH>(dot);
+      const float cc = r * r * r * dot / (float)HD;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const float a = d[e] * x[e] * r;
+        aq[e] += isq ? a : 0.f;
+        ak[e] += isq ? 0.f : a;
+        d[e] = r * (isq ? gqv[e] : gkv[e]) * d[e] - x[e] * cc;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      o[e] = HT::h(d[e]);
+      bad |= HT::bad(o[e]);
+    }
+    *(u16x8 *)(dqkv + t * ld + col) = o;
+  };
+  int w = threadIdx.x / TPH;
+  Item ia, ib;
+  if (w < n) load(w, ia);
+  for (; w < n; w += 2 * SPB) {
+    if (w + SPB < n) load(w + SPB, ib);
+    finish(w, ia);
+    if (w + 2 * SPB < n) load(w + 2 * SPB, ia);
+    if (w + SPB < n) finish(w + SPB, ib);
   }
   flag_overflow(ovf, bad);
-  if (QKN) {
-    red[threadIdx.x * 2] = a0;
-    red[threadIdx.x * 2 + 1] = a1;
+  flag_overflow(ovf_v, bad_v);
+  if constexpr (QKN) {
+    __shared__ float comb[SPB][2 * HD];
+    const int sb = threadIdx.x / TPH;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      comb[sb][8 * j + e] = aq[e];
+      comb[sb][HD + 8 * j + e] = ak[e];
+    }
     __syncthreads();
-    if (sub == 0) {
-      float s0 = 0.f, s1 = 0.f;
-      for (int k = 0; k < nsub; k++) {
-        s0 += red[(k * half + i) * 2];
-        s1 += red[(k * half + i) * 2 + 1];
-      }
-      if (part) {  // layout [head slot][token block][HD], reduced by colsum_kernel
-        float *pp = part + ((long)h * gridDim.x + blockIdx.x) * HD;
-        pp[2 * i] = dg_scale * s0;
-        pp[2 * i + 1] = dg_scale * s1;
-      } else {
-        float *dg = isq ? dgq : dgk;
-        atomicAdd(dg + 2 * i, dg_scale * s0);
-        atomicAdd(dg + 2 * i + 1, dg_scale * s1);
-      }
+    const int i = threadIdx.x;  // channel i of q (i < HD) or i - HD of k
+    if (i < 2 * HD) {
+      float v = 0.f;
+#pragma unroll
+      for (int k = 0; k < SPB; k++) v += comb[k][i];
+      v *= dg_scale;
+      if (part) part[i < HD ? (long)blockIdx.x * HD + i : ((long)gridDim.x + blockIdx.x) * HD + i - HD] = v;
+      else atomicAdd(i < HD ? dgq + i : dgk + i - HD, v);
     }
   }
 }
@@ -681,18 +765,21 @@ int launch_rmsnorm_fwd(int dt, const float *x, const float *g, h16_t *y, float *
 
 namespace {
 int rms_rows(int T) { return std::max(1, (T + 1023) / 1024); }  // rows per block: <= 1024 blocks
-// Tokens per block of the QK-prep backward: on short steps one per thread group (HD/2 threads a
-// token), so a block runs one pass and there are 4x-8x more blocks (256 tokens: 10.3 us with
-// 16 tokens a block, four passes of dependent loads); 128 on long steps.
-int qk_tpb(int T, int HD) { return T <= 4096 ? 512 / HD : 128; }
+// Rows per block of the form that adds its gain sums with atomics: <= 256 blocks of 4 row groups.
+int rms_rows_atomic(int T) { return 4 * std::max(1, (T + 1023) / 1024); }
+// Tokens per block of the QK-prep backward: as few as one on short steps (a block is a chain of
+// dependent loads per 16 or 32 head slots), at most 1024 blocks on long ones; at most 512 where
+// every block ends in atomics on the same lines.
+int qk_tpb(int T, bool atomics) {
+  const int most = atomics ? 512 : 1024;
+  return std::max(atomics ? 2 : 1, (T + most - 1) / most);
+}
 }  // namespace
 
 long rmsnorm_bwd_part_elems(int T, int D) { return (long)((T + rms_rows(T) - 1) / rms_rows(T)) * D; }
 int rmsnorm_bwd_part_rows(int T) { return (T + rms_rows(T) - 1) / rms_rows(T); }
-void qk_prep_bwd_part_rows(int T, int NH, int NKV, int HD, int *rows_q, int *rows_k) {
-  const int nbx = (T + qk_tpb(T, HD) - 1) / qk_tpb(T, HD);
-  *rows_q = NH * nbx;
-  *rows_k = NKV * nbx;
+void qk_prep_bwd_part_rows(int T, int *rows_q, int *rows_k) {
+  *rows_q = *rows_k = (T + qk_tpb(T, false) - 1) / qk_tpb(T, false);
 }
 
 int launch_colsum_batch(const ColsumJob *jobs_dev, int njobs, int max_n, hipStream_t s) {
@@ -701,8 +788,8 @@ int launch_colsum_batch(const ColsumJob *jobs_dev, int njobs, int max_n, hipStre
                      s, jobs_dev);
   return ne_hip_status(hipGetLastError(), "colsum_batch");
 }
-long qk_prep_bwd_part_elems(int T, int NH, int NKV, int HD) {
-  return (long)((T + qk_tpb(T, HD) - 1) / qk_tpb(T, HD)) * (NH + NKV) * HD;
+long qk_prep_bwd_part_elems(int T, int HD) {
+  return (long)((T + qk_tpb(T, false) - 1) / qk_tpb(T, false)) * 2 * HD;
 }
 
 int launch_rmsnorm_bwd(int dt, const float *dy, const float *x, const float *g, const float *r,
@@ -712,12 +799,13 @@ int launch_rmsnorm_bwd(int dt, const float *dy, const float *x, const float *g, 
   if (D % 4 || D > 4 * RMS_NT * RMS_VPT)
     return ne_fail(NE_ERR_ARG, "rmsnorm_bwd: D=%d must be a multiple of 4 <= 2048", D);
   if (T <= 0) return 0;
-  const int rows = rms_rows(T);
+  const int rows = part ? rms_rows(T) : rms_rows_atomic(T);
   const int nb = (T + rows - 1) / rows;
   NE_CHECK(DISPATCH_H16(dt, [&] {
-    auto kernel = ref_formula ? rmsnorm_bwd_kernel<HT, true> : rmsnorm_bwd_kernel<HT, false>;
-    hipLaunchKernelGGL(kernel, dim3(nb), dim3(RMS_NT), 0, s, dy, x, g, r, resid, dx, dxb, bscale, dg, dg_scale, T, D,
-                       rows, ovf, part, sp);
+    auto kernel = part ? (ref_formula ? rmsnorm_bwd_kernel<HT, true, 1> : rmsnorm_bwd_kernel<HT, false, 1>)
+                       : (ref_formula ? rmsnorm_bwd_kernel<HT, true, 4> : rmsnorm_bwd_kernel<HT, false, 4>);
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(part ? RMS_NT : 4 * RMS_NT), 0, s, dy, x, g, r, resid, dx, dxb, bscale,
+                       dg, dg_scale, T, D, rows, ovf, part, sp);
     return ne_hip_status(hipGetLastError(), "rmsnorm_bwd");
   }()));
   if (part && !defer_colsum) {
@@ -770,18 +858,28 @@ int launch_qk_prep_bwd(int dt, const float *dq, const float *dk, const h16_t *qk
                        int T, int S, int NH, int NKV, int HD, int *ovf, float *part, hipStream_t s,
                        bool defer_colsum, const float *kvpart, int *ovf_v) {
   if (HD != 64 && HD != 128) return ne_fail(NE_ERR_ARG, "qk_prep: head_dim %d not in {64,128}", HD);
-  if (kvpart && (ld % 2 || NH % NKV)) return ne_fail(NE_ERR_ARG, "qk_prep: bad layout for the dK/dV partials");
-  const int tpb = qk_tpb(T, HD);
+  if (kvpart && NH % NKV) return ne_fail(NE_ERR_ARG, "qk_prep: bad layout for the dK/dV partials");
+  if (T <= 0) return 0;
+  const bool atomics = gq && !part;
+  const int tpb = qk_tpb(T, atomics);
   const int nbx = (T + tpb - 1) / tpb;
-  dim3 grid(nbx, NH + NKV + (kvpart ? NKV : 0));
   NE_CHECK(DISPATCH_H16(dt, [&] {
-    if (gq) hipLaunchKernelGGL((qk_prep_bwd_kernel<HT, true>), grid, dim3(256), 0, s, dq, dk, qkv, ld, cosb, sinb, gq, gk, rq, rk, dqkv, dgq, dgk, dg_scale, T, S, NH, NKV, HD, tpb, ovf, part, kvpart, ovf_v);
-    else hipLaunchKernelGGL((qk_prep_bwd_kernel<HT, false>), grid, dim3(256), 0, s, dq, dk, qkv, ld, cosb, sinb, gq, gk, rq, rk, dqkv, dgq, dgk, dg_scale, T, S, NH, NKV, HD, tpb, ovf, part, kvpart, ovf_v);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(nbx), dim3(256), 0, s, dq, dk, qkv, ld, cosb, sinb, gq, gk, rq, rk, dqkv, dgq,
+                         dgk, dg_scale, T, S, NH, NKV, tpb, ovf, part, kvpart, ovf_v);
+    };
+    if (HD == 128) {
+      if (gq) go(qk_prep_bwd_kernel<HT, true, 128>);
+      else go(qk_prep_bwd_kernel<HT, false, 128>);
+    } else {
+      if (gq) go(qk_prep_bwd_kernel<HT, true, 64>);
+      else go(qk_prep_bwd_kernel<HT, false, 64>);
+    }
     return ne_hip_status(hipGetLastError(), "qk_prep_bwd");
   }()));
   if (gq && part && !defer_colsum) {
     hipLaunchKernelGGL(colsum_kernel, dim3((HD + CS_COLS - 1) / CS_COLS, 2), dim3(CS_COLS * CS_GROUPS), 0, s, part,
-                       NH * nbx, dgq, part + (long)NH * nbx * HD, NKV * nbx, dgk, HD);
+                       nbx, dgq, part + (long)nbx * HD, nbx, dgk, HD);
     NE_HIP(hipGetLastError());
   }
   return 0;

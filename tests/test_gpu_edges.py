@@ -1,0 +1,80 @@
+"""Kernel entry points at the sizes where their launch rules change: remainders of blocks, the
+smallest and largest of a range, row pitches that are not multiples of a wide access.  Against
+float64 numpy; tolerances from the fp32 sums (a sum of n terms in any order: about sqrt(n) * 2^-24
+of its terms' norm) and one 16-bit rounding of the outputs."""
+import numpy as np
+import pytest
+
+from gpu_util import FMT, _release_device_tensors, call, dev, host, need_gpu, ptr, rel_l2, torch, zeros  # noqa: F401
+import ne
+from oracle import model as om
+
+pytestmark = pytest.mark.gpu
+L = None
+
+
+@pytest.fixture(autouse=True)
+def _gpu():
+    need_gpu()
+    global L
+    L = ne.lib()
+
+
+# 4 row groups a block, at most 256 blocks: one row, a partial group, one row past a block, the last
+# block partly empty, several rows a group; D below, at and above one float4 per thread
+@pytest.mark.parametrize("T,D", [(1, 64), (3, 768), (5, 2048), (1024, 832), (1025, 1028), (2051, 128)])
+def test_rmsnorm_bwd_gain_sums(T, D):
+    dt, tdt, _, u = FMT["fp16"]
+    rng = np.random.default_rng(T + D)
+    x, dy, res = (rng.standard_normal((T, D)).astype(np.float32) for _ in range(3))
+    g = (1 + 0.2 * rng.standard_normal(D)).astype(np.float32)
+    r = (1.0 / np.sqrt((x.astype(np.float64) ** 2).mean(1) + 1e-5)).astype(np.float32)
+    dx, dxb = zeros((T + 1, D)), zeros((T + 1, D), tdt)
+    dg = dev(np.ones(D, np.float32))  # accumulates
+    call(L.ne_k_rmsnorm_bwd, dt, ptr(dev(dy)), ptr(dev(x)), ptr(dev(g)), ptr(dev(r)), ptr(dev(res)), ptr(dx),
+         ptr(dxb), 0.5, ptr(dg), 2.0, T, D, None)
+    X, DY, R = x.astype(np.float64), dy.astype(np.float64), r.astype(np.float64)[:, None]
+    ref = R * g * DY - X * R ** 3 * (DY * X * g).sum(1, keepdims=True) / D + res
+    got = host(dx)
+    assert rel_l2(got[:T], ref) < 1e-6 and not got[T].any() and not host(dxb)[T].any()
+    assert rel_l2(host(dxb)[:T], 0.5 * ref) < u
+    assert rel_l2(host(dg), 1 + 2 * (DY * X * R).sum(0)) < 1e-5
+
+
+# tokens a block: 2 on short steps, ceil(T / 512) above; a last block with one token; heads whose slots
+# leave lanes of the last pass idle; a pitch of 2 elements more than a row (4-byte aligned rows)
+@pytest.mark.parametrize("fmt", ["fp16", "bf16"])
+@pytest.mark.parametrize("T,S,NH,NKV,HD,pad,qk", [(64, 64, 2, 1, 64, 0, True), (192, 64, 3, 3, 128, 2, True),
+                                                  (1088, 1088, 10, 5, 64, 0, True), (1088, 64, 5, 1, 128, 2, True),
+                                                  (192, 192, 5, 5, 64, 2, False)])
+def test_qk_prep_bwd_edges(fmt, T, S, NH, NKV, HD, pad, qk):
+    dt, tdt, rnd, u = FMT[fmt]
+    Q, KV = NH * HD, NKV * HD
+    QKV = Q + 2 * KV
+    ld = QKV + pad
+    rng = np.random.default_rng(T + HD + pad)
+    qkv = rnd(rng.standard_normal((T, ld)).astype(np.float32))
+    gq, gk = ((1 + 0.3 * rng.standard_normal(HD)).astype(np.float32) for _ in range(2))
+    cos, sin = om.rope_tables(S, HD, 1e4)
+    dq, dk = rng.standard_normal((T, Q)).astype(np.float32), rng.standard_normal((T, KV)).astype(np.float32)
+    B = T // S
+    q, k = qkv[:, :Q].reshape(B, S, NH, HD), qkv[:, Q:Q + KV].reshape(B, S, NKV, HD)
+    dqn, dkn = om.rope_bwd(dq.reshape(B, S, NH, HD), cos, sin), om.rope_bwd(dk.reshape(B, S, NKV, HD), cos, sin)
+    rq = rk = None
+    if qk:
+        rq, rk = om.rmsnorm(q, gq, 1e-5)[1], om.rmsnorm(k, gk, 1e-5)[1]
+        (dqn, dgqr), (dkn, dgkr) = om.rmsnorm_bwd(dqn, q, gq, rq), om.rmsnorm_bwd(dkn, k, gk, rk)
+    dqkv = zeros((T, ld), tdt)
+    o = np.ones(HD, np.float32)
+    dgq, dgk = (dev(o), dev(o)) if qk else (None, None)
+    P = lambda a: ptr(dev(a)) if a is not None else None  # noqa: E731
+    call(L.ne_k_qk_prep_bwd, dt, P(dq), P(dk), ptr(dev(qkv, tdt)), ld,
+         P(cos.astype(np.float32)), P(sin.astype(np.float32)), P(gq) if qk else None, P(gk) if qk else None,
+         P(rq.reshape(T, NH)) if qk else None, P(rk.reshape(T, NKV)) if qk else None, ptr(dqkv), ptr(dgq), ptr(dgk),
+         2.0, T, S, NH, NKV, HD, None)
+    got = host(dqkv)
+    assert rel_l2(got[:, :Q], dqn.reshape(T, Q)) < u
+    assert rel_l2(got[:, Q:Q + KV], dkn.reshape(T, KV)) < u
+    assert not got[:, Q + KV:].any()  # the v columns and the padding are not this call's
+    if qk:
+        assert rel_l2(host(dgq), 1 + 2 * dgqr) < 1e-4 and rel_l2(host(dgk), 1 + 2 * dgkr) < 1e-4
