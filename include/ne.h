@@ -106,7 +106,7 @@ int ne_train_step(ne_ctx *ctx, const int32_t *tokens, float loss_scale, float *l
  * the step's graph is used only while ne_overlap_weight_grads is off and per-kernel
  * profiling is disabled: the two-stream step runs faster from eager launches).  The step's graph is
  * captured on first use per (fresh accumulation, loss_scale, internal gradient scale), the
- * decode graphs per (batch size, greedy or sampling); they replace the reference's
+ * decode graphs per (batch size; greedy, sampling, sampling with top-p); they replace the reference's
  * per-kernel ANE dispatch (TD/io.h:190-229).  Off: every kernel is launched eagerly. */
 int ne_use_graphs(ne_ctx *ctx, int on);
 /* Run the step's weight-gradient GEMMs (and the embedding gradient of the classifier) on a

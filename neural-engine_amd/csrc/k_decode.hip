@@ -31,6 +31,9 @@ struct DecState {
   float top_p;
 };
 
+// How a position's token is chosen: the first maximum, or sampled without or with a top-p mask.
+enum { PICK_GREEDY = 0, PICK_SAMPLE = 1, PICK_TOPP = 2 };
+
 constexpr int VB = 4;            // largest batch of the VALU GEMV path
 constexpr int BIG_ARGMAX = 256;  // argmax partials per sequence on the MFMA path
 
@@ -50,10 +53,15 @@ struct Dec {
   int32_t *out;           // [Bp, ctx] generated tokens
   int32_t *prompt;        // [Bp, ctx]
   double *unif;           // [Bp, ctx]
+  int sg, schunk;         // sampling: chunks per row of logits, columns per chunk
+  float *spmax;           // sampling partials (SampArgs)
+  double *spsum;
+  unsigned long long *shist, *smass, *sabove;
+  uint32_t *spre;
   float *cosb, *sinb;     // [ctx, HD/2]
   DecState *st;
   void *arena;
-  struct Graph { int B; bool greedy; hipGraphExec_t pre, gen; };
+  struct Graph { int B, mode; hipGraphExec_t pre, gen; };  // mode: PICK_*
   std::vector<Graph> graphs;
 };
 
@@ -696,26 +704,6 @@ __global__ __launch_bounds__(256) void dec_attn_kernel(const float *__restrict__
   }
 }
 
-// Block-wide helpers for the sampler (1024 threads).
-__device__ float block_max(float v, float *red) {
-  v = wave_max(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  float m = red[0];
-  for (int i = 1; i < (int)(blockDim.x >> 6); i++) m = fmaxf(m, red[i]);
-  return m;
-}
-__device__ double block_sum_d(double v, double *red) {
-  v = wave_sum_d(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  double s = 0.0;
-  for (int i = 0; i < (int)(blockDim.x >> 6); i++) s += red[i];
-  return s;
-}
-
 __device__ __forceinline__ int gen_step(const DecState *st) { return st->pos - (st->P - 1); }
 
 // Greedy from per-block partials: first index of the maximum logit (np.argmax).  One block
@@ -781,87 +769,341 @@ __global__ __launch_bounds__(256) void dec_argmax_part_kernel(const float *__res
   }
 }
 
-// Sampling: p = softmax(logits/T) in fp32, optional top-p mask, then the first index whose
-// fp64 cumulative mass exceeds u * total (np.random.choice: cdf.searchsorted(u,
-// side='right')).  One block (1024 threads) per sequence.
-__global__ __launch_bounds__(1024) void dec_sample_kernel(float *logits, int V, const DecState *__restrict__ st,
-                                                          const double *__restrict__ unif, int ctx, int32_t *tok,
-                                                          int32_t *out) {
-  __shared__ float redf[16];
-  __shared__ double redd[16];
-  __shared__ double wsum[16];
-  const int b = blockIdx.x;
-  const float temp = st->temp, top_p = st->top_p;
-  const int step = gen_step(st);
-  float *lg = logits + (long)b * V;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  // p_i = exp(x_i - max) / sum, x_i = logit_i / temp  (generate.py:201-202, softmax 87-90)
-  float mx = -INFINITY;
-  for (int i = tid; i < V; i += nt) mx = fmaxf(mx, lg[i] / temp);
-  mx = block_max(mx, redf);
-  double zs = 0.0;
-  for (int i = tid; i < V; i += nt) zs += (double)expf(lg[i] / temp - mx);
-  const float Z = (float)block_sum_d(zs, redd);
-  for (int i = tid; i < V; i += nt) lg[i] = expf(lg[i] / temp - mx) / Z;
+// ------------------------------------------------------------------------- sampling ----
+//
+// p = softmax(logits / T) in fp32, an optional top-p mask, then the first index whose cumulative
+// mass exceeds u * total (np.random.choice: cdf.searchsorted(u, side='right')).  A sequence's
+// row of V logits is cut into SampArgs::G contiguous chunks, one block each, and the row passes
+// through a chain of kernels over them; what a kernel needs of the whole row (max, sum, masses)
+// every block of the next one reduces again from the G partials, in order.  As one block per
+// sequence (1024 threads, about 36 passes over the row, 31 of them the bisection for the top-p
+// threshold) a sample of 151,936 logits took 747 us at batch 1; the chain takes 34 us (seven launches of 4-6 us: latency).
+//
+// Masses are sums of fixed-point values, p * 2^62 as an integer (p <= 1; exact for p >= 2^-38,
+// smaller ones lose less than 2^-62 each): integer sums do not depend on the order of the atomics
+// that form them, so the same logits and uniform always give the same token.
+
+struct SampArgs {
+  float *logits;              // [B][V]: logits, then exp(x - max), then p
+  int V, G, chunk;            // chunk: columns per block (a multiple of 4); G * chunk >= V
+  const DecState *st;
+  const double *unif;         // [B][ctx]
+  int ctx;
+  int32_t *tok, *out;
+  float *pmax;                // [B][G]
+  double *psum;               // [B][G]
+  unsigned long long *hist;   // [B][3][SAMP_BINS] mass per bin of p's bit pattern
+  unsigned long long *mass;   // [B][G] kept mass per chunk
+  uint32_t *pre;              // [B][2] threshold bits found so far (levels 1, 2)
+  unsigned long long *above;  // [B][2] mass above that prefix
+  bool topp;
+};
+
+constexpr int SAMP_NT = 256, SAMP_BINS = 1024;  // 10 bits of the pattern per level
+constexpr int SAMP_G = 128;                     // chunks per row at most: half the CUs at batch 1
+constexpr double SAMP_ONE = 4611686018427387904.0;  // 2^62
+constexpr uint32_t SAMP_P1 = 0x3f800000u;       // the bits of p = 1, the largest
+
+__device__ __forceinline__ unsigned long long samp_mass(float p) {
+  return p > 0.f ? (unsigned long long)((double)p * SAMP_ONE) : 0ull;  // 0 for NaN
+}
+
+template <typename T>
+__device__ __forceinline__ T samp_wave_sum(T v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+// Sum over the block, the same in every thread, waves in order (red: SAMP_NT / 64 slots).
+template <typename T>
+__device__ __forceinline__ T samp_block_sum(T v, T *red) {
+  v = samp_wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  float thr = 0.f;  // keep p >= thr
-  if (top_p < 1.f) {
-    // thr = largest probability value v with mass(p >= v) >= top_p (generate.py:205-213):
-    // bisection on the float bit pattern (monotone for positive floats).
-    uint32_t lo = 0, hi = 0x3f800001u;  // mass(p >= bits(lo)) >= top_p holds at lo = 0
-    while (hi - lo > 1) {
-      const uint32_t mid = lo + (hi - lo) / 2;
-      const float v = __uint_as_float(mid);
-      double m = 0.0;
-      for (int i = tid; i < V; i += nt) m += lg[i] >= v ? (double)lg[i] : 0.0;
-      m = block_sum_d(m, redd);
-      if (m >= (double)top_p) lo = mid; else hi = mid;
-    }
-    thr = __uint_as_float(lo);
-  }
-  // cumulative mass in vocabulary order, then the first index with cdf > u * total.
-  // Thread i owns the contiguous chunk [i0, i1) and the mass interval [start[i], start[i+1]).
-  __shared__ double start[1025];
-  const int chunk = (V + nt - 1) / nt;
-  const int i0 = min(V, tid * chunk), i1 = min(V, i0 + chunk);
-  double local = 0.0;
-  for (int i = i0; i < i1; i++) local += lg[i] >= thr ? (double)lg[i] : 0.0;
-  double incl = local;
+  T s = red[0];
+#pragma unroll
+  for (int i = 1; i < SAMP_NT / 64; i++) s += red[i];
+  return s;
+}
+
+// Inclusive prefix sum over the block's threads; *total receives the block's sum.
+__device__ __forceinline__ unsigned long long samp_block_scan(unsigned long long v, unsigned long long *red,
+                                                              unsigned long long *total) {
   for (int o = 1; o < 64; o <<= 1) {
-    const double n = __shfl_up(incl, o, 64);
-    if ((tid & 63) >= o) incl += n;
+    const unsigned long long n = __shfl_up(v, o, 64);
+    if ((int)(threadIdx.x & 63) >= o) v += n;
   }
-  if ((tid & 63) == 63) wsum[tid >> 6] = incl;
+  if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  double before = 0.0, total = 0.0;
-  for (int w = 0; w < nt / 64; w++) {
-    if (w < (tid >> 6)) before += wsum[w];
-    total += wsum[w];
+  unsigned long long before = 0, t = 0;
+#pragma unroll
+  for (int i = 0; i < SAMP_NT / 64; i++) {
+    if (i < (int)(threadIdx.x >> 6)) before += red[i];
+    t += red[i];
   }
-  double prev = __shfl_up(incl, 1, 64);
-  if ((tid & 63) == 0) prev = 0.0;
-  start[tid] = before + prev;
-  if (tid == 0) start[nt] = total;
+  *total = t;
+  return before + v;
+}
+
+// 1. The chunk's max of x = logit / T, and this position's empty histograms.
+__global__ __launch_bounds__(SAMP_NT) void samp_max_kernel(SampArgs a) {
+  __shared__ float red[SAMP_NT / 64];
+  const int b = blockIdx.y, g = blockIdx.x, tid = threadIdx.x;
+  const float *lg = a.logits + (long)b * a.V;
+  const int i1 = min(a.V, (g + 1) * a.chunk);
+  float mx = -INFINITY;
+  const float temp = a.st->temp;
+  for (int i = g * a.chunk + tid * 4; i < i1; i += SAMP_NT * 4) {
+    const float4 v = *(const float4 *)(lg + i);
+    mx = fmaxf(fmaxf(fmaxf(mx, v.x / temp), v.y / temp), fmaxf(v.z / temp, v.w / temp));
+  }
+  if (a.topp)
+    for (int i = g * SAMP_NT + tid; i < 3 * SAMP_BINS; i += gridDim.x * SAMP_NT) a.hist[(long)b * 3 * SAMP_BINS + i] = 0;
+  mx = wave_max(mx);
+  if ((tid & 63) == 0) red[tid >> 6] = mx;
   __syncthreads();
-  const double u = unif[(long)b * ctx + step] * total;
-  const bool last = tid == nt - 1;
-  if ((start[tid] <= u && u < start[tid + 1]) || (last && u >= start[nt])) {
-    double c = start[tid];
-    int pick = -1;
-    for (int i = i0; i < i1; i++) {
-      const double p = lg[i] >= thr ? (double)lg[i] : 0.0;
-      if (p > 0.0) pick = i;
-      c += p;
-      if (p > 0.0 && c > u) break;
-    }
-    if (pick < 0) {  // empty chunk (rounding at a boundary): last kept index before it
-      pick = i0 - 1;
-      while (pick > 0 && !(lg[pick] >= thr && lg[pick] > 0.f)) pick--;
-      if (pick < 0) pick = 0;
-    }
-    tok[b] = pick;
-    out[(long)b * ctx + step] = pick;
+  if (tid == 0) {
+    for (int w = 1; w < SAMP_NT / 64; w++) mx = fmaxf(mx, red[w]);
+    a.pmax[b * a.G + g] = mx;
   }
+}
+
+// 2. exp(x - max) in place, and its fp64 sum over the chunk (generate.py:87-90).
+__global__ __launch_bounds__(SAMP_NT) void samp_exp_kernel(SampArgs a) {
+  __shared__ float redm[SAMP_NT / 64];
+  __shared__ double red[SAMP_NT / 64];
+  const int b = blockIdx.y, g = blockIdx.x, tid = threadIdx.x;
+  float *lg = a.logits + (long)b * a.V;
+  const int i1 = min(a.V, (g + 1) * a.chunk);
+  float mx = -INFINITY;
+  for (int i = tid; i < a.G; i += SAMP_NT) mx = fmaxf(mx, a.pmax[b * a.G + i]);
+  mx = wave_max(mx);
+  if ((tid & 63) == 0) redm[tid >> 6] = mx;
+  __syncthreads();
+  for (int w = 0; w < SAMP_NT / 64; w++) mx = fmaxf(mx, redm[w]);
+  const float temp = a.st->temp;
+  double z = 0.0;
+  for (int i = g * a.chunk + tid * 4; i < i1; i += SAMP_NT * 4) {
+    float4 v = *(const float4 *)(lg + i);
+    v.x = expf(v.x / temp - mx); v.y = expf(v.y / temp - mx);
+    v.z = expf(v.z / temp - mx); v.w = expf(v.w / temp - mx);
+    *(float4 *)(lg + i) = v;
+    z += (double)v.x; z += (double)v.y; z += (double)v.z; z += (double)v.w;
+  }
+  z = samp_block_sum(z, red);
+  if (tid == 0) a.psum[b * a.G + g] = z;
+}
+
+// The largest bin k whose suffix mass (base + bins k.. of `hist`) reaches top_p, and the suffix mass
+// above it; k = 0 when none does.  256 threads, 4 bins each; the same result in every thread.
+__device__ __forceinline__ void samp_select(const unsigned long long *hist, unsigned long long base, float top_p,
+                                            uint32_t &k, unsigned long long &above) {
+  __shared__ unsigned long long red[SAMP_NT / 64], s_above;
+  __shared__ uint32_t s_k;
+  const int tid = threadIdx.x;
+  unsigned long long h[4], own = 0;
+#pragma unroll
+  for (int e = 0; e < 4; e++) own += h[e] = hist[4 * tid + e];
+  if (tid == 0) s_k = 0;
+  unsigned long long total;
+  const unsigned long long incl = samp_block_scan(own, red, &total);
+  unsigned long long up = base + (total - incl);  // mass above this thread's bins
+  if (tid == 0) s_above = up + h[3] + h[2] + h[1];
+  __syncthreads();
+  // suffix masses fall with k: the one bin where the mass first reaches top_p from above
+#pragma unroll
+  for (int e = 3; e >= 0; e--) {
+    const unsigned long long at = up + h[e];
+    const bool top = tid == SAMP_NT - 1 && e == 3;
+    if ((double)at / SAMP_ONE >= (double)top_p && (top || !((double)up / SAMP_ONE >= (double)top_p))) {
+      s_k = 4 * tid + e;
+      s_above = up;
+    }
+    up = at;
+  }
+  __syncthreads();
+  k = s_k;
+  above = s_above;
+  __syncthreads();
+}
+
+// Bin of p at level LV (1: bits 20.., 2: bits 10..19, 3: bits 0..9), or -1 if p's higher bits are not
+// the prefix chosen so far.
+template <int LV>
+__device__ __forceinline__ int samp_bin(float p, uint32_t prefix) {
+  const uint32_t u = __float_as_uint(p);
+  if (LV == 1) return (int)(u >> 20);
+  if (LV == 2) return u >> 20 == prefix ? (int)((u >> 10) & 1023u) : -1;
+  return u >> 10 == prefix ? (int)(u & 1023u) : -1;
+}
+
+// The block's histogram in LDS, its non-empty bins added to the row's.
+template <int LV>
+__device__ __forceinline__ void samp_hist_add(unsigned long long *lds, float p, uint32_t prefix) {
+  if (!(p > 0.f)) return;
+  const int k = samp_bin<LV>(p, prefix);
+  if (k >= 0) atomicAdd(&lds[k], samp_mass(p));
+}
+__device__ __forceinline__ void samp_hist_out(const unsigned long long *lds, unsigned long long *out) {
+  __syncthreads();
+  for (int i = threadIdx.x; i < SAMP_BINS; i += SAMP_NT)
+    if (lds[i]) atomicAdd(out + i, lds[i]);
+}
+
+// 3. p = exp / Z in place; with top-p the first histogram level (8 bins per octave), without it the
+// chunk's mass.
+__global__ __launch_bounds__(SAMP_NT) void samp_prob_kernel(SampArgs a) {
+  __shared__ double red[SAMP_NT / 64];
+  __shared__ unsigned long long redm[SAMP_NT / 64];
+  __shared__ unsigned long long lds[SAMP_BINS];
+  const int b = blockIdx.y, g = blockIdx.x, tid = threadIdx.x;
+  float *lg = a.logits + (long)b * a.V;
+  const int i1 = min(a.V, (g + 1) * a.chunk);
+  double z = 0.0;
+  for (int i = tid; i < a.G; i += SAMP_NT) z += a.psum[b * a.G + i];
+  if (a.topp)
+    for (int i = tid; i < SAMP_BINS; i += SAMP_NT) lds[i] = 0;
+  const float Z = (float)samp_block_sum(z, red);
+  unsigned long long m = 0;
+  for (int i = g * a.chunk + tid * 4; i < i1; i += SAMP_NT * 4) {
+    float4 v = *(const float4 *)(lg + i);
+    v.x /= Z; v.y /= Z; v.z /= Z; v.w /= Z;
+    *(float4 *)(lg + i) = v;
+    if (a.topp) {
+      samp_hist_add<1>(lds, v.x, 0); samp_hist_add<1>(lds, v.y, 0);
+      samp_hist_add<1>(lds, v.z, 0); samp_hist_add<1>(lds, v.w, 0);
+    } else {
+      m += samp_mass(v.x) + samp_mass(v.y) + samp_mass(v.z) + samp_mass(v.w);
+    }
+  }
+  if (a.topp) {
+    samp_hist_out(lds, a.hist + (long)b * 3 * SAMP_BINS);
+  } else {
+    m = samp_block_sum(m, redm);
+    if (tid == 0) a.mass[b * a.G + g] = m;
+  }
+}
+
+// 4, 5. Histogram level LV (2, 3) among the values in the bin that level LV - 1 selects.
+template <int LV>
+__global__ __launch_bounds__(SAMP_NT) void samp_hist_kernel(SampArgs a) {
+  __shared__ unsigned long long lds[SAMP_BINS];
+  const int b = blockIdx.y, g = blockIdx.x, tid = threadIdx.x;
+  const float *lg = a.logits + (long)b * a.V;
+  const int i1 = min(a.V, (g + 1) * a.chunk);
+  for (int i = tid; i < SAMP_BINS; i += SAMP_NT) lds[i] = 0;
+  unsigned long long *hist = a.hist + (long)b * 3 * SAMP_BINS;
+  uint32_t k;
+  unsigned long long above;
+  samp_select(hist + (LV - 2) * SAMP_BINS, LV == 2 ? 0ull : a.above[b * 2], a.st->top_p, k, above);
+  const uint32_t prefix = LV == 2 ? k : (a.pre[b * 2] << 10) | k;
+  if (g == 0 && tid == 0) {
+    a.pre[b * 2 + LV - 2] = prefix;
+    a.above[b * 2 + LV - 2] = above;
+  }
+  for (int i = g * a.chunk + tid * 4; i < i1; i += SAMP_NT * 4) {
+    const float4 v = *(const float4 *)(lg + i);
+    samp_hist_add<LV>(lds, v.x, prefix); samp_hist_add<LV>(lds, v.y, prefix);
+    samp_hist_add<LV>(lds, v.z, prefix); samp_hist_add<LV>(lds, v.w, prefix);
+  }
+  samp_hist_out(lds, hist + (LV - 1) * SAMP_BINS);
+}
+
+// The top-p threshold: the largest probability v with mass(p >= v) >= top_p (generate.py:205-213), 0
+// when even the whole row's mass stays below it.
+__device__ __forceinline__ float samp_threshold(const SampArgs &a, int b) {
+  uint32_t k;
+  unsigned long long above;
+  samp_select(a.hist + ((long)b * 3 + 2) * SAMP_BINS, a.above[b * 2 + 1], a.st->top_p, k, above);
+  return __uint_as_float(min((a.pre[b * 2 + 1] << 10) | k, SAMP_P1));
+}
+
+// 6 (top-p). The chunk's mass of p >= threshold.
+__global__ __launch_bounds__(SAMP_NT) void samp_mass_kernel(SampArgs a) {
+  __shared__ unsigned long long red[SAMP_NT / 64];
+  const int b = blockIdx.y, g = blockIdx.x, tid = threadIdx.x;
+  const float *lg = a.logits + (long)b * a.V;
+  const int i1 = min(a.V, (g + 1) * a.chunk);
+  const float thr = samp_threshold(a, b);
+  unsigned long long m = 0;
+  for (int i = g * a.chunk + tid * 4; i < i1; i += SAMP_NT * 4) {
+    const float4 v = *(const float4 *)(lg + i);
+    m += (v.x >= thr ? samp_mass(v.x) : 0) + (v.y >= thr ? samp_mass(v.y) : 0) + (v.z >= thr ? samp_mass(v.z) : 0) +
+         (v.w >= thr ? samp_mass(v.w) : 0);
+  }
+  m = samp_block_sum(m, red);
+  if (tid == 0) a.mass[b * a.G + g] = m;
+}
+
+// 7. One block per sequence: the chunk whose cumulative mass passes u * total, then the index in it.
+// Token 0 when nothing is kept (no finite probability).
+__global__ __launch_bounds__(SAMP_NT) void samp_pick_kernel(SampArgs a) {
+  __shared__ unsigned long long red[SAMP_NT / 64], s_before;
+  __shared__ int s_chunk, s_pick;
+  const int b = blockIdx.x, tid = threadIdx.x;
+  const float *lg = a.logits + (long)b * a.V;
+  const float thr = a.topp ? samp_threshold(a, b) : 0.f;
+  const int step = gen_step(a.st);
+  static_assert(SAMP_G <= SAMP_NT, "one chunk mass per thread");
+  const unsigned long long own = tid < a.G ? a.mass[b * a.G + tid] : 0ull;
+  unsigned long long total;
+  const unsigned long long incl = samp_block_scan(own, red, &total);
+  if (tid == 0) {
+    s_chunk = -1;
+    s_pick = -1;
+  }
+  __syncthreads();
+  const double u = a.unif[(long)b * a.ctx + step] * (double)total;
+  // the first chunk that passes u; where rounding lets none pass, the last one that holds mass
+  if (own && (double)incl > u && !((double)(incl - own) > u)) {
+    s_chunk = tid;
+    s_before = incl - own;
+  }
+  __syncthreads();
+  const bool none = s_chunk < 0;
+  if (none && own && incl == total) {
+    s_chunk = tid;
+    s_before = incl - own;
+  }
+  __syncthreads();
+  if (s_chunk >= 0) {
+    const int c0 = s_chunk * a.chunk, c1 = min(a.V, c0 + a.chunk);
+    const int per = (a.chunk + SAMP_NT - 1) / SAMP_NT;
+    const int i0 = min(c1, c0 + tid * per), i1 = min(c1, i0 + per);
+    unsigned long long m = 0, tot;
+    for (int i = i0; i < i1; i++) m += lg[i] >= thr ? samp_mass(lg[i]) : 0ull;
+    unsigned long long c = s_before + samp_block_scan(m, red, &tot) - m;
+    if (m && (none ? c + m == s_before + tot : (double)(c + m) > u && !((double)c > u))) {
+      int pick = -1;
+      for (int i = i0; i < i1; i++) {
+        const unsigned long long q = lg[i] >= thr ? samp_mass(lg[i]) : 0ull;
+        if (!q) continue;
+        pick = i;
+        c += q;
+        if (!none && (double)c > u) break;
+      }
+      s_pick = pick;
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    const int pick = s_pick < 0 ? 0 : s_pick;
+    a.tok[b] = pick;
+    a.out[(long)b * a.ctx + step] = pick;
+  }
+}
+
+int launch_sample(const SampArgs &a, int B, hipStream_t s) {
+  const dim3 grid(a.G, B), block(SAMP_NT);
+  hipLaunchKernelGGL(samp_max_kernel, grid, block, 0, s, a);
+  hipLaunchKernelGGL(samp_exp_kernel, grid, block, 0, s, a);
+  hipLaunchKernelGGL(samp_prob_kernel, grid, block, 0, s, a);
+  if (a.topp) {
+    hipLaunchKernelGGL(samp_hist_kernel<2>, grid, block, 0, s, a);
+    hipLaunchKernelGGL(samp_hist_kernel<3>, grid, block, 0, s, a);
+    hipLaunchKernelGGL(samp_mass_kernel, grid, block, 0, s, a);
+  }
+  hipLaunchKernelGGL(samp_pick_kernel, dim3(B), block, 0, s, a);
+  return ne_hip_status(hipGetLastError(), "decode sampling");
 }
 
 __global__ void dec_advance_kernel(DecState *st) {
@@ -1123,7 +1365,8 @@ int launch_attn(ne_ctx *c, int B, const LayerOff &o, float *kc, float *vc, const
 // Enqueue the kernels of one position for B sequences.  gen: also the final norm, LM head
 // and token choice.  Position-independent (everything position-dependent is read from
 // d->st), so it can be captured once and replayed.
-int enqueue_position(ne_ctx *c, int B, bool gen, bool greedy) {
+int enqueue_position(ne_ctx *c, int B, bool gen, int mode) {
+  const bool greedy = mode == PICK_GREEDY;
   Dec *d = (Dec *)c->dec;
   const int D = c->D, H = c->H, Q = c->Q, NKV = c->NKV, HD = c->HD, QKV = c->QKV, V = c->V;
   const float eps = c->c.norm_eps, alpha = c->c.res_alpha;
@@ -1198,17 +1441,18 @@ int enqueue_position(ne_ctx *c, int B, bool gen, bool greedy) {
       }
     }
     if (!greedy)
-      hipLaunchKernelGGL(dec_sample_kernel, dim3(B), dim3(1024), 0, c->st, d->logits, V, d->st, d->unif, d->ctx,
-                         d->tok, d->out);
+      NE_CHECK(launch_sample({d->logits, V, d->sg, d->schunk, d->st, d->unif, d->ctx, d->tok, d->out, d->spmax, d->spsum,
+                              d->shist, d->smass, d->spre, d->sabove, mode == PICK_TOPP},
+                             B, c->st));
   }
   hipLaunchKernelGGL(dec_advance_kernel, dim3(1), dim3(64), 0, c->st, d->st);
   return ne_hip_status(hipGetLastError(), "decode position");
 }
 
-int capture(ne_ctx *c, int B, bool gen, bool greedy, hipGraphExec_t *exec) {
+int capture(ne_ctx *c, int B, bool gen, int mode, hipGraphExec_t *exec) {
   hipGraph_t graph = nullptr;
   NE_HIP(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
-  const int rc = enqueue_position(c, B, gen, greedy);
+  const int rc = enqueue_position(c, B, gen, mode);
   const hipError_t ec = hipStreamEndCapture(c->st, &graph);
   if (rc) {
     if (graph) (void)hipGraphDestroy(graph);
@@ -1248,6 +1492,11 @@ int decode_alloc(ne_ctx *c) {
   const size_t o_ws = take((size_t)d->ws_elems * 4), o_gate = take(Bp * H * 4);
   const size_t o_amv = take(Bp * (size_t)d->lm_nblk * 4), o_ami = take(Bp * (size_t)d->lm_nblk * 4);
   const size_t o_tok = take(Bp * 4), o_out = take(Bp * ctx * 4), o_pr = take(Bp * ctx * 4), o_u = take(Bp * ctx * 8);
+  // row chunks of at least 1024 columns, a multiple of 4 (16-byte accesses)
+  d->sg = std::max(1, std::min(SAMP_G, c->V / 1024));
+  d->schunk = ((c->V + d->sg - 1) / d->sg + 3) / 4 * 4;
+  const size_t o_pm = take(Bp * d->sg * 4), o_ps = take(Bp * d->sg * 8), o_ms = take(Bp * d->sg * 8);
+  const size_t o_hi = take(Bp * 3 * SAMP_BINS * 8), o_ab = take(Bp * 2 * 8), o_pf = take(Bp * 2 * 4);
   const size_t o_cos = take(ctx * HD / 2 * 4), o_sin = take(ctx * HD / 2 * 4), o_st = take(sizeof(DecState));
   NE_HIP(hipMalloc(&d->arena, off));
   char *base = (char *)d->arena;
@@ -1260,6 +1509,9 @@ int decode_alloc(ne_ctx *c) {
   d->amv = (float *)(base + o_amv); d->ami = (int32_t *)(base + o_ami);
   d->tok = (int32_t *)(base + o_tok); d->out = (int32_t *)(base + o_out); d->prompt = (int32_t *)(base + o_pr);
   d->unif = (double *)(base + o_u);
+  d->spmax = (float *)(base + o_pm); d->spsum = (double *)(base + o_ps);
+  d->smass = (unsigned long long *)(base + o_ms); d->shist = (unsigned long long *)(base + o_hi);
+  d->sabove = (unsigned long long *)(base + o_ab); d->spre = (uint32_t *)(base + o_pf);
   d->cosb = (float *)(base + o_cos); d->sinb = (float *)(base + o_sin);
   d->st = (DecState *)(base + o_st);
   NE_HIP(hipMemset(d->arena, 0, off));
@@ -1290,7 +1542,7 @@ void decode_free(ne_ctx *c) {
 }
 
 namespace {
-int replay(ne_ctx *c, int B, int P, int n_new, bool greedy);
+int replay(ne_ctx *c, int B, int P, int n_new, int mode);
 }
 
 int decode_run(ne_ctx *c, const int32_t *prompt, int B, int P, int n_new, float temp, float top_p,
@@ -1301,6 +1553,7 @@ int decode_run(ne_ctx *c, const int32_t *prompt, int B, int P, int n_new, float 
     return ne_fail(NE_ERR_ARG, "decode: B=%d P=%d n_new=%d exceed decode_batch=%d / decode_ctx=%d", B, P, n_new,
                    c->c.decode_batch, d->ctx);
   const bool greedy = temp < 1e-6f;
+  const int mode = greedy ? PICK_GREEDY : top_p < 1.f ? PICK_TOPP : PICK_SAMPLE;
   if (!greedy && !uniforms) return ne_fail(NE_ERR_ARG, "decode: sampling needs uniforms");
   for (long i = 0; i < (long)B * P; i++)
     if (prompt[i] < 0 || prompt[i] >= c->V) return ne_fail(NE_ERR_ARG, "decode: prompt id out of range");
@@ -1324,9 +1577,9 @@ int decode_run(ne_ctx *c, const int32_t *prompt, int B, int P, int n_new, float 
   NE_HIP(hipStreamSynchronize(c->st));  // host staging vectors are released at return
 
   if (!c->use_graphs) {  // eager launches (tracers that do not follow graph launches)
-    for (int pos = 0; pos < P + n_new - 1; pos++) NE_CHECK(enqueue_position(c, B, pos >= P - 1, greedy));
+    for (int pos = 0; pos < P + n_new - 1; pos++) NE_CHECK(enqueue_position(c, B, pos >= P - 1, mode));
   } else {
-    NE_CHECK(replay(c, B, P, n_new, greedy));
+    NE_CHECK(replay(c, B, P, n_new, mode));
   }
   std::vector<int32_t> o((size_t)d->Bp * d->ctx);
   NE_HIP(hipMemcpyAsync(o.data(), d->out, o.size() * 4, hipMemcpyDeviceToHost, c->st));
@@ -1339,15 +1592,15 @@ int decode_run(ne_ctx *c, const int32_t *prompt, int B, int P, int n_new, float 
 namespace {
 
 // Replay the captured position graphs (captured on first use per batch size and mode).
-int replay(ne_ctx *c, int B, int P, int n_new, bool greedy) {
+int replay(ne_ctx *c, int B, int P, int n_new, int mode) {
   Dec *d = (Dec *)c->dec;
   Dec::Graph *gr = nullptr;
   for (auto &g : d->graphs)
-    if (g.B == B && g.greedy == greedy) gr = &g;
+    if (g.B == B && g.mode == mode) gr = &g;
   if (!gr) {
-    Dec::Graph g = {B, greedy, nullptr, nullptr};
-    int rc = capture(c, B, false, greedy, &g.pre);
-    if (!rc) rc = capture(c, B, true, greedy, &g.gen);
+    Dec::Graph g = {B, mode, nullptr, nullptr};
+    int rc = capture(c, B, false, mode, &g.pre);
+    if (!rc) rc = capture(c, B, true, mode, &g.gen);
     if (rc) {
       if (g.pre) hipGraphExecDestroy(g.pre);
       return rc;

@@ -78,3 +78,31 @@ def test_qk_prep_bwd_edges(fmt, T, S, NH, NKV, HD, pad, qk):
     assert not got[:, Q + KV:].any()  # the v columns and the padding are not this call's
     if qk:
         assert rel_l2(host(dgq), 1 + 2 * dgqr) < 1e-4 and rel_l2(host(dgk), 1 + 2 * dgkr) < 1e-4
+
+
+# Sampling runs a row of logits in chunks of at least 1024 columns: one chunk, two, a last chunk shorter
+# than the others; peaked (gain 8) and flat (gain 1) distributions, with and without the top-p mask.
+# A pick may differ from the oracle's only where its uniform lies within 1e-5 of the boundary between
+# the two in cumulative probability (the fp32 logits and their softmax, 32k terms of rounding 6e-8).
+@pytest.mark.parametrize("V,B,gain,top_p", [(512, 1, 8.0, 0.9), (1024, 3, 1.0, 1.0), (2112, 5, 8.0, 0.95),
+                                            (2112, 2, 1.0, 0.5), (32064, 1, 8.0, 0.9), (32064, 6, 1.0, 1.0)])
+def test_decode_sampling_chunks(V, B, gain, top_p):
+    cfg = om.tiny(vocab=V)
+    P = {k: om.round_bf16(v) for k, v in om.init_params(cfg, seed=V).items()}
+    P["rms_final"] = np.full_like(P["rms_final"], gain)
+    n, temp = 12, 0.8
+    m = ne.Model.from_oracle(cfg, decode_batch=B, decode_ctx=4 + n, dtype=ne.NE_BF16)
+    m.set_params(P)
+    rng = np.random.default_rng(V + B)
+    prompt, u = rng.integers(0, V, (B, 4)).astype(np.int32), rng.random((B, n))
+    got = m.decode(prompt, n, temp, top_p, u)
+    np.testing.assert_array_equal(m.decode(prompt, n, temp, top_p, u), got)
+    picks, dist = om.decode(cfg, P, prompt, n, temperature=temp, top_p=top_p, uniforms=u, forced=got)
+    assert np.abs(dist).max() < 1e-5, (np.argwhere(picks != got), np.abs(dist).max())
+    # the first uniform picks the first kept token, the last one the last; no finite logit: token 0
+    lo = m.decode(prompt, 1, temp, 1.0, np.zeros((B, 1)))
+    hi = m.decode(prompt, 1, temp, 1.0, np.full((B, 1), 1 - 2.0 ** -53))
+    assert (lo == 0).all() and (hi > V - 64).all()
+    m.set("rms_final", np.full(cfg.dim, np.nan, np.float32))
+    assert (m.decode(prompt, 2, temp, top_p, u[:, :2]) == 0).all()
+    m.close()
