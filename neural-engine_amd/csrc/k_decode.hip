@@ -7,8 +7,9 @@
 // the KV cache and all accumulation are fp32.
 //
 // Every kernel reads the position from device memory (DecState), so the launch sequence of
-// one position does not depend on it: it is captured once as a HIP graph (one for prompt
-// positions, one for generated positions) and replayed per position.
+// one generated position does not depend on it: it is captured once as a HIP graph and replayed
+// per position.  The prompt's positions before the last run in chunks of up to 256 rows (sequence x
+// position) through the batch 5..32 GEMVs (enqueue_prompt).
 //
 // GEMVs are HBM-bound (each weight byte is read once per position whatever the batch):
 //  * batch <= 4: VALU kernel.  The block stages its input rows in LDS (fusing the RMSNorm or
@@ -35,17 +36,20 @@ struct DecState {
 enum { PICK_GREEDY = 0, PICK_SAMPLE = 1, PICK_TOPP = 2 };
 
 constexpr int VB = 4;            // largest batch of the VALU GEMV path
+constexpr int PROMPT_ROWS = 256; // most rows of a prompt chunk
 constexpr int BIG_ARGMAX = 256;  // argmax partials per sequence on the MFMA path
 
 struct Dec {
   int Bmax;               // decode_batch
   int Bp;                 // MFMA path: batch padded to 16 or 32
+  int Rp;                 // rows (sequence x position) of a prompt chunk: >= Bp, a multiple of 16
   int ctx;                // max positions
   float *kc, *vc;         // [L][Bmax][NKV] of V [ctx][HD] and K [ctx][HD] (batch <= 4: [HD/4][ctx] float4 pieces)
-  float *x, *xn, *qkv, *att, *logits;  // [Bp, *]
+  float *x, *xn, *att;    // [Rp, *]
+  float *qkv, *logits;    // [Bp, *]
   float *ws;              // MFMA split-K partials
   long ws_elems;
-  float *gate;            // [Bp, H] SwiGLU gate (batch 5..32)
+  float *gate;            // [Rp, H] SwiGLU gate (MFMA path)
   float *amv;             // argmax partials [Bmax][nblk]
   int32_t *ami;
   int lm_nblk;
@@ -61,7 +65,7 @@ struct Dec {
   float *cosb, *sinb;     // [ctx, HD/2]
   DecState *st;
   void *arena;
-  struct Graph { int B, mode; hipGraphExec_t pre, gen; };  // mode: PICK_*
+  struct Graph { int B, mode; hipGraphExec_t gen; };  // mode: PICK_*
   std::vector<Graph> graphs;
 };
 
@@ -246,6 +250,7 @@ __device__ __forceinline__ f32x4 mfma_f32(float a, float b, const f32x4 &c) {
 // K range of split blockIdx.y, for NT tiles of 16 sequences; the 4 waves split that range.
 // With a workspace ws, split z's products go to slice z of ws [ksplit][Bp, N] (one split's
 // slice is laid out as the output rows); without (one split), out = alpha * products + resid.
+// blockIdx.z takes the rows NT * 16 * z .. of x (a prompt chunk has more than NT * 16).
 // GATE (one split; W = [W1; W3], gate_n rows each): the block's rows are j0..j0+7 of W1 and
 // the same of W3 (j0 = 8 * blockIdx.x), and it writes out[b, j] = silu(h1) * h3
 // (generate.py:190).  WV waves per block split the K range; each loads up to 8 weight chunks
@@ -254,7 +259,7 @@ template <typename HT, int NT, bool GATE, int WV = 4>
 __global__ __launch_bounds__(WV * 64) void gemv_mfma_kernel(const h16_t *__restrict__ W, long ldw,
                                                         const float *__restrict__ x, long ldx, int K, int ksplit,
                                                         float *out, long ldo, const float *resid, float alpha,
-                                                        float *ws, int N, int B, long gate_n) {
+                                                        float *ws, int N, int B, int Bp, long gate_n) {
   __shared__ f32x4 red[WV][NT][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = lane >> 4, r = lane & 15;
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(WV * 64) void gemv_mfma_kernel(const h16_t *__restr
       if (k0 < kend) {
 #pragma unroll
         for (int t = 0; t < NT; t++) {
-          const float *xr = x + (long)(t * 16 + r) * ldx + k0 + g * 8;
+          const float *xr = x + (long)((blockIdx.z * NT + t) * 16 + r) * ldx + k0 + g * 8;
           const float4 a0 = *(const float4 *)xr, a1 = *(const float4 *)(xr + 4);
           const float xv[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
 #pragma unroll
@@ -295,8 +300,8 @@ __global__ __launch_bounds__(WV * 64) void gemv_mfma_kernel(const h16_t *__restr
       f32x4 s = red[0][t][lane];
 #pragma unroll
       for (int v = 1; v < WV; v++) s += red[v][t][lane];
-      // s[i] = sum for sequence t*16 + r, weight row blockIdx.x*16 + 4g + i
-      const int b = t * 16 + r;
+      // s[i] = sum for sequence b, weight row blockIdx.x*16 + 4g + i
+      const int b = (blockIdx.z * NT + t) * 16 + r;
       const long n = (long)blockIdx.x * 16 + g * 4;
       if (GATE) {
         // lanes g = 0, 1 hold h1 of gate outputs j0 + 4g + i; lanes g + 2 hold their h3
@@ -311,7 +316,7 @@ __global__ __launch_bounds__(WV * 64) void gemv_mfma_kernel(const h16_t *__restr
           *(float4 *)(out + b * ldo + (long)blockIdx.x * 8 + g * 4) = o;
         }
       } else if (ws) {
-        *(f32x4 *)(ws + ((long)blockIdx.y * NT * 16 + b) * N + n) = s;
+        *(f32x4 *)(ws + ((long)blockIdx.y * Bp + b) * N + n) = s;
       } else if (b < B) {
         float4 o = make_float4(alpha * s[0], alpha * s[1], alpha * s[2], alpha * s[3]);
         if (resid) {
@@ -354,6 +359,7 @@ enum { BF3_WS = 0, BF3_GATE = 1, BF3_PLAIN = 2 };
 //             j0 + 16 rt.., the rest the same rows of W3; writes out[b, j] = silu(h1) * h3
 //             (generate.py:190) for b < B;
 //  BF3_PLAIN: one split, out[b, n] = sums for b < B (the LM head's logits).
+// blockIdx.z takes the x rows 16 * NTW * z .. (a prompt chunk has more than 16 * NTW).
 template <int NTW, int RT, int KS, int MODE>
 __global__ __launch_bounds__(NTW * 256) void gemv_bf3_kernel(const h16_t *__restrict__ W, long ldw,
                                                              const float *__restrict__ x, long ldx,
@@ -381,7 +387,7 @@ __global__ __launch_bounds__(NTW * 256) void gemv_bf3_kernel(const h16_t *__rest
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) wf[rt][ks] = __builtin_nontemporal_load((const u16x8 *)(wr + ks * 32));
   }
-  const int b = t * 16 + r16;
+  const int b = (blockIdx.z * NTW + t) * 16 + r16;
   u16x8 xh[KS], xm[KS], xl[KS];
   {
     const float *xr = x + (long)b * ldx + kb;
@@ -543,13 +549,17 @@ __global__ void dec_token_kernel(const int32_t *__restrict__ prompt, int ctx, co
 // KCOL (batch <= 4, one block per KV head): the K cache holds float4 d4 of position t at
 // K4[d4 * ctx + t], so that the score loop's lanes (one position each) read consecutive 16-byte
 // pieces; else row-major like V ([ctx][HD]), which measured faster at batch 32.
-template <int HD, int RATIO, bool KCOL>
+// PRE: row blockIdx.x of a prompt chunk (sequence row / nc, position p0 + row % nc), whose keys
+// and values pre_append_kernel has put into the cache; otherwise row = sequence, the position is
+// the state's, and its key and value are appended here.
+template <int HD, int RATIO, bool KCOL, bool PRE>
 __global__ __launch_bounds__(256) void dec_attn_kernel(const float *__restrict__ qkv, int QKV,
                                                        const float *__restrict__ gq, const float *__restrict__ gk,
                                                        const float *__restrict__ cosb, const float *__restrict__ sinb,
                                                        float *kc, float *vc, float *att, int NH, int NKV, int ctx,
                                                        const DecState *__restrict__ st, float eps, double scale,
-                                                       const float *__restrict__ qws, int qnz, int Bp) {
+                                                       const float *__restrict__ qws, int qnz, int Bp, int p0,
+                                                       int nc) {
   extern __shared__ float sc[];  // [RATIO][ctx]
   constexpr int C4 = HD / 4, NG = 256 / C4, HALF = HD / 2;
   __shared__ float4 qs[RATIO][C4];
@@ -559,21 +569,22 @@ __global__ __launch_bounds__(256) void dec_attn_kernel(const float *__restrict__
   // block y: query heads qh0 .. qh0 + RATIO - 1 of KV head kvh (RATIO may be a part of the
   // model's NH / NKV query heads per KV head: the blocks of one KV head then append the same
   // K and V values)
-  const int b = blockIdx.x, qh0 = blockIdx.y * RATIO, kvh = qh0 / (NH / NKV), tid = threadIdx.x;
-  const int pos = st->pos, npos = pos + 1;
+  const int ri = blockIdx.x, b = PRE ? ri / nc : ri;
+  const int qh0 = blockIdx.y * RATIO, kvh = qh0 / (NH / NKV), tid = threadIdx.x;
+  const int pos = PRE ? p0 + ri % nc : st->pos, npos = pos + 1;
   float *K = kc + ((long)b * NKV + kvh) * ctx * HD;
   float *V = vc + ((long)b * NKV + kvh) * ctx * HD;
-  const float *row = qkv + (long)b * QKV;
+  const float *row = qkv + (long)ri * QKV;
   // element col of this sequence's q|k|v row: the row itself, or (qnz > 1) the ordered sum of
   // the QKV GEMV's split-K partial slices [qnz][Bp, QKV]
   auto qval = [&](int col) -> float {
     if (qnz <= 1) return row[col];
     float s = 0.f;
-    for (int z = 0; z < qnz; z++) s += qws[((long)z * Bp + b) * QKV + col];
+    for (int z = 0; z < qnz; z++) s += qws[((long)z * Bp + ri) * QKV + col];
     return s;
   };
   // slots 0..RATIO-1: q heads qh0 + slot; RATIO: k head kvh; RATIO+1: v head kvh
-  for (int i = tid; i < (RATIO + 2) * HALF; i += 256) {
+  for (int i = tid; i < (PRE ? RATIO : RATIO + 2) * HALF; i += 256) {
     const int slot = i / HALF, p = i % HALF;
     float *q2 = (float *)qs, *v2 = (float *)vn;
     if (slot == RATIO + 1) {
@@ -670,7 +681,7 @@ __global__ __launch_bounds__(256) void dec_attn_kernel(const float *__restrict__
 #pragma unroll
     for (int u = 0; u < 4; u++) {
       const int tu = t + u * NG;
-      v[u] = tu == pos ? vn[c] : *(const float4 *)(V + (long)tu * HD + c * 4);
+      v[u] = !PRE && tu == pos ? vn[c] : *(const float4 *)(V + (long)tu * HD + c * 4);
     }
 #pragma unroll
     for (int u = 0; u < 4; u++)
@@ -681,7 +692,7 @@ __global__ __launch_bounds__(256) void dec_attn_kernel(const float *__restrict__
       }
   }
   for (; t < npos; t += NG) {
-    const float4 v = t == pos ? vn[c] : *(const float4 *)(V + (long)t * HD + c * 4);
+    const float4 v = !PRE && t == pos ? vn[c] : *(const float4 *)(V + (long)t * HD + c * 4);
 #pragma unroll
     for (int r = 0; r < RATIO; r++) {
       const float p = sc[r * ctx + t];
@@ -700,8 +711,66 @@ __global__ __launch_bounds__(256) void dec_attn_kernel(const float *__restrict__
       o.x += p.x; o.y += p.y; o.z += p.z; o.w += p.w;
     }
     o.x *= inv; o.y *= inv; o.z *= inv; o.w *= inv;
-    *(float4 *)(att + (long)b * NH * HD + (long)(qh0 + r) * HD + c * 4) = o;
+    *(float4 *)(att + (long)ri * NH * HD + (long)(qh0 + r) * HD + c * 4) = o;
   }
+}
+
+// Tokens and embedding rows of a prompt chunk (row i: sequence i / nc, position p0 + i % nc),
+// and their RMSNorm with the first gain.  One block per row.
+template <typename HT>
+__global__ __launch_bounds__(256) void pre_token_kernel(const int32_t *__restrict__ prompt, int ctx, int p0, int nc,
+                                                        const h16_t *__restrict__ E, float *x, int D,
+                                                        const float *__restrict__ gn, float *xn, float eps) {
+  __shared__ float red[4];
+  const long i = blockIdx.x;
+  const int t = prompt[(i / nc) * ctx + p0 + i % nc];
+  float ss = 0.f;
+  for (int k = threadIdx.x; k < D; k += 256) {
+    const float v = HT::f(E[(long)t * D + k]);
+    x[i * D + k] = v;
+    ss += v * v;
+  }
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  const float rms = sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)D + eps);
+  for (int k = threadIdx.x; k < D; k += 256) xn[i * D + k] = x[i * D + k] / rms * gn[k];
+}
+
+// Keys (QK-norm, RoPE) and values of a prompt chunk into the cache, from the qnz split-K slices
+// [Rp, QKV] of the QKV rows.  Block (row, KV head): HD / 2 threads for the key's pairs, as many for
+// the value's.
+template <int HD, bool KCOL>
+__global__ __launch_bounds__(HD) void pre_append_kernel(const float *__restrict__ qws, int qnz, int Rp, int QKV,
+                                                        const float *__restrict__ gk, const float *__restrict__ cosb,
+                                                        const float *__restrict__ sinb, float *kc, float *vc, int NH,
+                                                        int NKV, int ctx, int p0, int nc, float eps) {
+  constexpr int HALF = HD / 2;
+  const int ri = blockIdx.x, kvh = blockIdx.y, b = ri / nc, pos = p0 + ri % nc;
+  const bool isv = threadIdx.x >= HALF;
+  const int p = threadIdx.x % HALF, col = (NH + (isv ? NKV : 0) + kvh) * HD + 2 * p;
+  const long cache = ((long)b * NKV + kvh) * ctx * HD;
+  float x0 = 0.f, x1 = 0.f;
+  for (int z = 0; z < qnz; z++) {
+    const float2 v = *(const float2 *)(qws + ((long)z * Rp + ri) * QKV + col);
+    x0 += v.x;
+    x1 += v.y;
+  }
+  float ss = x0 * x0 + x1 * x1;
+  ss = HALF == 64 ? wave_sum(ss) : half_wave_sum(ss);
+  if (isv) {
+    *(float2 *)(vc + cache + (long)pos * HD + 2 * p) = make_float2(x0, x1);
+    return;
+  }
+  if (gk) {
+    const float rms = sqrtf(ss / (float)HD + eps);
+    x0 = x0 / rms * gk[2 * p];
+    x1 = x1 / rms * gk[2 * p + 1];
+  }
+  const float c = cosb[pos * HALF + p], s = sinb[pos * HALF + p];
+  const float2 y = make_float2(x0 * c - x1 * s, x0 * s + x1 * c);
+  if (KCOL) *(float2 *)(kc + cache + ((long)(p >> 1) * ctx + pos) * 4 + 2 * (p & 1)) = y;
+  else *(float2 *)(kc + cache + (long)pos * HD + 2 * p) = y;
 }
 
 __device__ __forceinline__ int gen_step(const DecState *st) { return st->pos - (st->P - 1); }
@@ -1179,7 +1248,11 @@ int gemv_small(ne_ctx *c, int B, int pro, bool amx, const h16_t *W, int N, int K
   }());
 }
 
-// Batch 5..32: the products of W [N, K] with x rows [Bp, K] (row stride ldx).  wsp
+// Rows of the MFMA GEMVs' x and outputs: 16, or a multiple of 32 of them (decode: d->Bp).
+inline int pad_rows(int rows) { return rows <= 16 ? 16 : (rows + 31) / 32 * 32; }
+
+// Batch 5..32 (or the B rows of a prompt chunk, padded to Bp): the products of W [N, K] with x
+// rows [Bp, K] (row stride ldx).  wsp
 // (nullable): a workspace of cap floats for the split-K partials.
 //  * nz_out != null: the partials stay in wsp for the consumer (*nz_out slices of [Bp, N]);
 //  * else, with wsp: out = alpha * (their ordered sum) + resid, one block per sequence, and
@@ -1187,27 +1260,26 @@ int gemv_small(ne_ctx *c, int B, int pro, bool amx, const h16_t *W, int N, int K
 //  * without wsp: one split, out = alpha * products (+ resid) directly;
 //  * gate: W = [W1; W3] (2N rows), out [Bp, N] = silu(W1.x) * (W3.x), one split.
 // Requires N % 16 (gate: N % 8), K % 128.
-int gemv_big(ne_ctx *c, int B, const h16_t *W, int N, int K, const float *x, long ldx, float *wsp, long cap,
+int gemv_big(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float *x, long ldx, float *wsp, long cap,
              float *out, long ldo, const float *resid, float alpha, int *nz_out, const float *gn = nullptr,
              float *xn = nullptr, bool gate = false) {
-  Dec *d = (Dec *)c->dec;
   if ((gate ? N % 8 : N % 16) || K % 128)
     return ne_fail(NE_ERR_ARG, "decode gemv: N=%d K=%d (need N%%16 (gate: %%8), K%%128)", N, K);
   if (gate && wsp) return ne_fail(NE_ERR_ARG, "decode gemv: the gate form has one split");
   int ks = 1;
   if (wsp)
-    while ((N / 16) * ks < 512 && K % (128 * ks * 2) == 0 && (long)ks * 2 * d->Bp * N <= cap) ks *= 2;
-  if (wsp && (long)ks * d->Bp * N > cap) return ne_fail(NE_ERR_ARG, "decode gemv: workspace too small");
-  const dim3 grid(gate ? N / 8 : N / 16, ks);
+    while ((N / 16) * ks < 512 && K % (128 * ks * 2) == 0 && (long)ks * 2 * Bp * N <= cap) ks *= 2;
+  if (wsp && (long)ks * Bp * N > cap) return ne_fail(NE_ERR_ARG, "decode gemv: workspace too small");
+  const dim3 grid(gate ? N / 8 : N / 16, ks, Bp <= 16 ? 1 : Bp / 32);
   // the gate form has one split: 8 waves per block shorten each wave's K range instead
   // (K % 256 then; else 4 waves)
   const bool wide = gate && K % 256 == 0;
   NE_CHECK(DISPATCH_H16(c->dt, [&] {
     auto go = [&](auto kernel, int threads) {
       hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, c->st, W, (long)K, x, ldx, K, ks, out, ldo, resid, alpha,
-                         wsp, N, B, (long)N);
+                         wsp, N, B, Bp, (long)N);
     };
-    if (d->Bp == 16) {
+    if (Bp == 16) {
       if (wide) go(gemv_mfma_kernel<HT, 1, true, 8>, 512);
       else if (gate) go(gemv_mfma_kernel<HT, 1, true>, 256);
       else go(gemv_mfma_kernel<HT, 1, false>, 256);
@@ -1224,7 +1296,7 @@ int gemv_big(ne_ctx *c, int B, const h16_t *W, int N, int K, const float *x, lon
   }
   if (wsp) {
     auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(B), dim3(256), 0, c->st, wsp, ks, d->Bp, N, out, ldo, resid, alpha, gn, xn,
+      hipLaunchKernelGGL(kernel, dim3(B), dim3(256), 0, c->st, wsp, ks, Bp, N, out, ldo, resid, alpha, gn, xn,
                          c->c.norm_eps);
     };
     if (N > 1024) go(gemv_reduce_rows_kernel<0>);
@@ -1242,7 +1314,7 @@ int gemv_big(ne_ctx *c, int B, const h16_t *W, int N, int K, const float *x, lon
 // 1 after launching; 0: not applicable, nothing launched).  mode BF3_WS: the split-K partials
 // go to d->ws and *nz receives the split count; BF3_GATE: W = [W1; W3] (N rows each), gate
 // [Bp, N] -> out; BF3_PLAIN: out [Bp, ldo] = products.
-int gemv_bf3(ne_ctx *c, int B, const h16_t *W, int N, int K, const float *x, long ldx, int mode, float *out,
+int gemv_bf3(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float *x, long ldx, int mode, float *out,
              long ldo, int *nz) {
   Dec *d = (Dec *)c->dec;
   if (c->dt != NE_BF16 || K % 128) return 0;
@@ -1256,7 +1328,7 @@ int gemv_bf3(ne_ctx *c, int B, const h16_t *W, int N, int K, const float *x, lon
     if (!ks) return 0;
     ksplit = K / (128 * ks);
     rt = (N % 64 == 0 && (N / 64) * ksplit >= 192) ? 4 : 2;
-    if (N % (16 * rt) || (long)ksplit * d->Bp * N > d->ws_elems) return 0;
+    if (N % (16 * rt) || (long)ksplit * Bp * N > d->ws_elems) return 0;
   } else {
     ks = K / 128;
     if (ks != 1 && ks != 6 && ks != 8) return 0;
@@ -1265,13 +1337,13 @@ int gemv_bf3(ne_ctx *c, int B, const h16_t *W, int N, int K, const float *x, lon
     // position against 32)
     if (mode == BF3_PLAIN && N % 128 == 0) rt = 8;
   }
-  const int ntw = d->Bp / 16;
-  const dim3 grid(mode == BF3_GATE ? N / 16 : N / (16 * rt), ksplit);
+  const int ntw = Bp == 16 ? 1 : 2;
+  const dim3 grid(mode == BF3_GATE ? N / 16 : N / (16 * rt), ksplit, Bp / (16 * ntw));
   float *dst = mode == BF3_WS ? d->ws : out;
   const long ldd = mode == BF3_WS ? N : ldo;
   bool done = false;
   auto go = [&](auto kernel, int nt) {
-    hipLaunchKernelGGL(kernel, grid, dim3(nt * 256), 0, c->st, W, (long)K, x, ldx, dst, ldd, N, B, d->Bp, (long)N);
+    hipLaunchKernelGGL(kernel, grid, dim3(nt * 256), 0, c->st, W, (long)K, x, ldx, dst, ldd, N, B, Bp, (long)N);
     done = true;
   };
 #define NE_BF3(NTW_)                                                                                 \
@@ -1309,14 +1381,14 @@ int gemv_bf3(ne_ctx *c, int B, const h16_t *W, int N, int K, const float *x, lon
 
 // Wo / W2 on gemv_bf3_kernel with the split-K sum, residual and RMSNorm of gemv_big's
 // workspace form (gemv_reduce_rows_kernel); returns 0 when not applicable.
-int gemv_bf3_resid(ne_ctx *c, int B, const h16_t *W, int N, int K, const float *x, long ldx, float *out, long ldo,
+int gemv_bf3_resid(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float *x, long ldx, float *out, long ldo,
                    const float *resid, float alpha, const float *gn, float *xn) {
   Dec *d = (Dec *)c->dec;
   int ks = 0;
-  const int rc = gemv_bf3(c, B, W, N, K, x, ldx, BF3_WS, nullptr, 0, &ks);
+  const int rc = gemv_bf3(c, B, Bp, W, N, K, x, ldx, BF3_WS, nullptr, 0, &ks);
   if (rc <= 0) return rc;
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(B), dim3(256), 0, c->st, d->ws, ks, d->Bp, N, out, ldo, resid, alpha, gn, xn,
+    hipLaunchKernelGGL(kernel, dim3(B), dim3(256), 0, c->st, d->ws, ks, Bp, N, out, ldo, resid, alpha, gn, xn,
                        c->c.norm_eps);
   };
   if (N > 1024) go(gemv_reduce_rows_kernel<0>);
@@ -1329,37 +1401,127 @@ int gemv_bf3_resid(ne_ctx *c, int B, const h16_t *W, int N, int K, const float *
   return 1;
 }
 
-// qkv: the q|k|v rows [Bp, QKV], or (qnz > 1) qnz split-K partial slices of them.
-int launch_attn(ne_ctx *c, int B, const LayerOff &o, float *kc, float *vc, const float *qkv, int qnz, bool kcol) {
+// qkv: the q|k|v rows [Bp, QKV], or (qnz > 1) qnz split-K partial slices of them.  nc > 0: the
+// rows of a prompt chunk of nc positions from p0 on (PRE of dec_attn_kernel).
+template <int HD, int R, bool KCOL>
+void attn_go(ne_ctx *c, dim3 grid, size_t sh, const float *gq, const float *gk, float *kc, float *vc, const float *qkv,
+             int qnz, int Bp, int p0, int nc) {
+  Dec *d = (Dec *)c->dec;
+  const double scale = 1.0 / sqrt((double)c->HD);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), sh, c->st, qkv, c->QKV, gq, gk, d->cosb, d->sinb, kc, vc, d->att, c->NH,
+                       c->NKV, d->ctx, d->st, c->c.norm_eps, scale, qkv, qnz, Bp, p0, nc);
+  };
+  if (nc > 0) go(dec_attn_kernel<HD, R, KCOL, true>);
+  else go(dec_attn_kernel<HD, R, KCOL, false>);
+}
+
+template <int HD, int R>
+void attn_kcol(ne_ctx *c, bool kcol, dim3 grid, size_t sh, const float *gq, const float *gk, float *kc, float *vc,
+               const float *qkv, int qnz, int Bp, int p0, int nc) {
+  if (kcol) attn_go<HD, R, true>(c, grid, sh, gq, gk, kc, vc, qkv, qnz, Bp, p0, nc);
+  else attn_go<HD, R, false>(c, grid, sh, gq, gk, kc, vc, qkv, qnz, Bp, p0, nc);
+}
+
+int launch_attn(ne_ctx *c, int rows, int Bp, const LayerOff &o, float *kc, float *vc, const float *qkv, int qnz,
+                bool kcol, int p0 = 0, int nc = 0) {
   Dec *d = (Dec *)c->dec;
   const int ratio = c->NH / c->NKV;
   // query heads per block: at batch <= 4 one (the blocks of a KV head share its K/V reads
-  // through L2, and twice the blocks run), else all of the KV head's
-  const int qpb = kcol ? 1 : ratio;
+  // through L2, and twice the blocks run), else all of the KV head's.  A prompt chunk has blocks
+  // enough: all, unless their scores would not fit the LDS that batch <= 4 gets by with.
+  const bool fits = (size_t)ratio * d->ctx * sizeof(float) <= 32768;
+  const int qpb = kcol && !(nc && fits) ? 1 : ratio;
   const size_t sh = (size_t)qpb * d->ctx * sizeof(float);
-  const double scale = 1.0 / sqrt((double)c->HD);
   const float *gq = c->c.qk_norm ? c->P + o.gq : nullptr, *gk = c->c.qk_norm ? c->P + o.gk : nullptr;
-  const dim3 grid(B, c->NH / qpb);
-#define NE_DEC_ATTN(HDV, R)                                                                                     \
-  if (kcol)                                                                                                     \
-    hipLaunchKernelGGL((dec_attn_kernel<HDV, R, true>), grid, dim3(256), sh, c->st, qkv, c->QKV, gq, gk,        \
-                       d->cosb, d->sinb, kc, vc, d->att, c->NH, c->NKV, d->ctx, d->st, c->c.norm_eps, scale,   \
-                       qkv, qnz, d->Bp);                                                                        \
-  else                                                                                                          \
-    hipLaunchKernelGGL((dec_attn_kernel<HDV, R, false>), grid, dim3(256), sh, c->st, qkv, c->QKV, gq, gk,       \
-                       d->cosb, d->sinb, kc, vc, d->att, c->NH, c->NKV, d->ctx, d->st, c->c.norm_eps, scale,   \
-                       qkv, qnz, d->Bp)
+  const dim3 grid(rows, c->NH / qpb);
   if (c->HD == 128) {
-    if (qpb == 1) NE_DEC_ATTN(128, 1);
-    else if (qpb == 2) NE_DEC_ATTN(128, 2);
-    else NE_DEC_ATTN(128, 4);
+    if (qpb == 1) attn_kcol<128, 1>(c, kcol, grid, sh, gq, gk, kc, vc, qkv, qnz, Bp, p0, nc);
+    else if (qpb == 2) attn_kcol<128, 2>(c, kcol, grid, sh, gq, gk, kc, vc, qkv, qnz, Bp, p0, nc);
+    else attn_kcol<128, 4>(c, kcol, grid, sh, gq, gk, kc, vc, qkv, qnz, Bp, p0, nc);
   } else {
-    if (qpb == 1) NE_DEC_ATTN(64, 1);
-    else if (qpb == 2) NE_DEC_ATTN(64, 2);
-    else NE_DEC_ATTN(64, 4);
+    if (qpb == 1) attn_kcol<64, 1>(c, kcol, grid, sh, gq, gk, kc, vc, qkv, qnz, Bp, p0, nc);
+    else if (qpb == 2) attn_kcol<64, 2>(c, kcol, grid, sh, gq, gk, kc, vc, qkv, qnz, Bp, p0, nc);
+    else attn_kcol<64, 4>(c, kcol, grid, sh, gq, gk, kc, vc, qkv, qnz, Bp, p0, nc);
   }
-#undef NE_DEC_ATTN
   return ne_hip_status(hipGetLastError(), "decode attention");
+}
+
+// One layer from its Wo on, on the MFMA GEMVs: x += alpha Wo.att, the FFN, and xn = RMSNorm(x)
+// with the next gain.  rows of x, padded to Bp.
+int big_layer_tail(ne_ctx *c, int rows, int Bp, const LayerOff &o, const float *g_next) {
+  Dec *d = (Dec *)c->dec;
+  const int D = c->D, H = c->H, Q = c->Q;
+  const float alpha = c->c.res_alpha;
+  const long cap = d->ws_elems;
+  const h16_t *Pb = c->Pb;
+  const float *g_ffn = c->P + o.g_ffn;
+  int rc = gemv_bf3_resid(c, rows, Bp, Pb + o.wo, D, Q, d->att, Q, d->x, D, d->x, alpha, g_ffn, d->xn);
+  if (rc < 0) return rc;
+  if (!rc)
+    NE_CHECK(gemv_big(c, rows, Bp, Pb + o.wo, D, Q, d->att, Q, d->ws, cap, d->x, D, d->x, alpha, nullptr, g_ffn, d->xn));
+  rc = gemv_bf3(c, rows, Bp, Pb + o.w13, H, D, d->xn, D, BF3_GATE, d->gate, H, nullptr);
+  if (rc < 0) return rc;
+  if (!rc)
+    NE_CHECK(gemv_big(c, rows, Bp, Pb + o.w13, H, D, d->xn, D, nullptr, 0, d->gate, H, nullptr, 1.f, nullptr, nullptr,
+                      nullptr, true));
+  rc = gemv_bf3_resid(c, rows, Bp, Pb + o.w2, D, H, d->gate, H, d->x, D, d->x, alpha, g_next, d->xn);
+  if (rc < 0) return rc;
+  if (!rc)
+    NE_CHECK(gemv_big(c, rows, Bp, Pb + o.w2, D, H, d->gate, H, d->ws, cap, d->x, D, d->x, alpha, nullptr, g_next, d->xn));
+  return 0;
+}
+
+// The QKV products of the rows of xn into d->ws; *qnz receives their split-K slice count.
+int big_qkv(ne_ctx *c, int rows, int Bp, const LayerOff &o, int *qnz) {
+  Dec *d = (Dec *)c->dec;
+  const int rc = gemv_bf3(c, rows, Bp, c->Pb + o.wqkv, c->QKV, c->D, d->xn, c->D, BF3_WS, nullptr, 0, qnz);
+  if (rc < 0) return rc;
+  if (!rc)
+    NE_CHECK(gemv_big(c, rows, Bp, c->Pb + o.wqkv, c->QKV, c->D, d->xn, c->D, d->ws, d->ws_elems, nullptr, 0, nullptr,
+                      1.f, qnz));
+  return 0;
+}
+
+// Prompt positions 0 .. n_pos - 1 of B sequences into the KV cache, in chunks of up to d->Rp rows
+// (row = sequence x position): the weights are read once per 32 rows and the chain of a position's
+// launches is paid once per chunk.  Position by position that chain bounded the prompt (about
+// 0.63 ms a position at batch 1, 1.43 ms at batch 32, Qwen3-0.6B): a 32-token prompt and 64 new
+// tokens took 60.6 ms at batch 1 (fp16, sampled), 136.1 at batch 32 (bf16, greedy), now 44.8 and 115.6.
+// The last layer's outputs are not needed: it ends with its keys and values.
+int enqueue_prompt(ne_ctx *c, int B, int n_pos) {
+  Dec *d = (Dec *)c->dec;
+  const bool kcol = B <= VB;
+  const float eps = c->c.norm_eps;
+  const int per = d->Rp / B;  // positions per chunk
+  for (int p0 = 0; p0 < n_pos; p0 += per) {
+    const int nc = std::min(per, n_pos - p0), rows = B * nc, Bp = pad_rows(rows);
+    auto token = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, c->st, d->prompt, d->ctx, p0, nc, c->Pb + c->off_E, d->x,
+                         c->D, c->P + c->lo[0].g_att, d->xn, eps);
+    };
+    if (c->dt == NE_FP16) token(pre_token_kernel<H16F>);
+    else token(pre_token_kernel<H16B>);
+    NE_HIP(hipGetLastError());
+    for (int l = 0; l < c->L; l++) {
+      const LayerOff &o = c->lo[l];
+      const size_t kvl = (size_t)l * d->Bmax * c->NKV * d->ctx * c->HD;
+      int qnz = 0;
+      NE_CHECK(big_qkv(c, rows, Bp, o, &qnz));
+      auto append = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(rows, c->NKV), dim3(c->HD), 0, c->st, d->ws, qnz, Bp, c->QKV,
+                           c->c.qk_norm ? c->P + o.gk : nullptr, d->cosb, d->sinb, d->kc + kvl, d->vc + kvl, c->NH,
+                           c->NKV, d->ctx, p0, nc, eps);
+      };
+      if (c->HD == 128) kcol ? append(pre_append_kernel<128, true>) : append(pre_append_kernel<128, false>);
+      else kcol ? append(pre_append_kernel<64, true>) : append(pre_append_kernel<64, false>);
+      NE_HIP(hipGetLastError());
+      if (l + 1 == c->L) break;
+      NE_CHECK(launch_attn(c, rows, Bp, o, d->kc + kvl, d->vc + kvl, d->ws, qnz, kcol, p0, nc));
+      NE_CHECK(big_layer_tail(c, rows, Bp, o, c->P + c->lo[l + 1].g_att));
+    }
+  }
+  return 0;
 }
 
 // Enqueue the kernels of one position for B sequences.  gen: also the final norm, LM head
@@ -1376,7 +1538,6 @@ int enqueue_position(ne_ctx *c, int B, bool gen, int mode) {
   // batch 5..32: the kernels that write x (the token lookup, the Wo / W2 split-K reductions)
   // also write its RMSNorm with the next gain into xn; the QKV GEMV's partials are summed by
   // the attention kernel
-  const long cap = d->ws_elems;
   const float *g0 = small ? nullptr : Pf + c->lo[0].g_att;
   if (c->dt == NE_FP16)
     hipLaunchKernelGGL(dec_token_kernel<H16F>, dim3(B), dim3(256), 0, c->st, d->prompt, d->ctx, d->st, d->tok,
@@ -1390,36 +1551,17 @@ int enqueue_position(ne_ctx *c, int B, bool gen, int mode) {
     const size_t kvl = (size_t)l * d->Bmax * NKV * d->ctx * HD;
     if (small) {
       NE_CHECK(gemv_small(c, B, PRO_RMSNORM, false, Pb + o.wqkv, QKV, D, d->x, D, Pf + o.g_att, d->qkv, QKV, nullptr, 1.f));
-      NE_CHECK(launch_attn(c, B, o, d->kc + kvl, d->vc + kvl, d->qkv, 1, true));
-    } else {
-      int qnz = 0;
-      int rc = gemv_bf3(c, B, Pb + o.wqkv, QKV, D, d->xn, D, BF3_WS, nullptr, 0, &qnz);
-      if (rc < 0) return rc;
-      if (!rc) NE_CHECK(gemv_big(c, B, Pb + o.wqkv, QKV, D, d->xn, D, d->ws, cap, nullptr, 0, nullptr, 1.f, &qnz));
-      NE_CHECK(launch_attn(c, B, o, d->kc + kvl, d->vc + kvl, d->ws, qnz, false));
-    }
-    if (small) {
+      NE_CHECK(launch_attn(c, B, d->Bp, o, d->kc + kvl, d->vc + kvl, d->qkv, 1, true));
       NE_CHECK(gemv_small(c, B, PRO_NONE, false, Pb + o.wo, D, Q, d->att, Q, nullptr, d->x, D, d->x, alpha));
       // W1|W3 with the SwiGLU gate in its epilogue (gate -> xn), then W2 + residual
       NE_CHECK(gemv_small(c, B, PRO_RMSNORM, false, Pb + o.w13, H, D, d->x, D, Pf + o.g_ffn, d->xn, H, nullptr, 1.f,
                           true));
       NE_CHECK(gemv_small(c, B, PRO_NONE, false, Pb + o.w2, D, H, d->xn, H, nullptr, d->x, D, d->x, alpha));
     } else {
-      const float *g_next = l + 1 < c->L ? Pf + c->lo[l + 1].g_att : Pf + c->off_gfinal;
-      int rc = gemv_bf3_resid(c, B, Pb + o.wo, D, Q, d->att, Q, d->x, D, d->x, alpha, Pf + o.g_ffn, d->xn);
-      if (rc < 0) return rc;
-      if (!rc)
-        NE_CHECK(gemv_big(c, B, Pb + o.wo, D, Q, d->att, Q, d->ws, cap, d->x, D, d->x, alpha, nullptr, Pf + o.g_ffn,
-                          d->xn));
-      rc = gemv_bf3(c, B, Pb + o.w13, H, D, d->xn, D, BF3_GATE, d->gate, H, nullptr);
-      if (rc < 0) return rc;
-      if (!rc)
-        NE_CHECK(gemv_big(c, B, Pb + o.w13, H, D, d->xn, D, nullptr, 0, d->gate, H, nullptr, 1.f, nullptr, nullptr,
-                          nullptr, true));
-      rc = gemv_bf3_resid(c, B, Pb + o.w2, D, H, d->gate, H, d->x, D, d->x, alpha, g_next, d->xn);
-      if (rc < 0) return rc;
-      if (!rc)
-        NE_CHECK(gemv_big(c, B, Pb + o.w2, D, H, d->gate, H, d->ws, cap, d->x, D, d->x, alpha, nullptr, g_next, d->xn));
+      int qnz = 0;
+      NE_CHECK(big_qkv(c, B, d->Bp, o, &qnz));
+      NE_CHECK(launch_attn(c, B, d->Bp, o, d->kc + kvl, d->vc + kvl, d->ws, qnz, false));
+      NE_CHECK(big_layer_tail(c, B, d->Bp, o, l + 1 < c->L ? Pf + c->lo[l + 1].g_att : Pf + c->off_gfinal));
     }
   }
   if (gen) {
@@ -1430,9 +1572,9 @@ int enqueue_position(ne_ctx *c, int B, bool gen, int mode) {
         hipLaunchKernelGGL(dec_argmax_kernel, dim3(B), dim3(1024), 0, c->st, d->amv, d->ami, V / (4 * pick_rpw(V)),
                            d->st, d->ctx, d->tok, d->out);
     } else {
-      const int rc = gemv_bf3(c, B, Pb + c->off_E, V, D, d->xn, D, BF3_PLAIN, d->logits, V, nullptr);
+      const int rc = gemv_bf3(c, B, d->Bp, Pb + c->off_E, V, D, d->xn, D, BF3_PLAIN, d->logits, V, nullptr);
       if (rc < 0) return rc;
-      if (!rc) NE_CHECK(gemv_big(c, B, Pb + c->off_E, V, D, d->xn, D, nullptr, 0, d->logits, V, nullptr, 1.f, nullptr));
+      if (!rc) NE_CHECK(gemv_big(c, B, d->Bp, Pb + c->off_E, V, D, d->xn, D, nullptr, 0, d->logits, V, nullptr, 1.f, nullptr));
       if (greedy) {
         hipLaunchKernelGGL(dec_argmax_part_kernel, dim3(BIG_ARGMAX, B), dim3(256), 0, c->st, d->logits, V, BIG_ARGMAX,
                            d->amv, d->ami);
@@ -1449,10 +1591,10 @@ int enqueue_position(ne_ctx *c, int B, bool gen, int mode) {
   return ne_hip_status(hipGetLastError(), "decode position");
 }
 
-int capture(ne_ctx *c, int B, bool gen, int mode, hipGraphExec_t *exec) {
+int capture(ne_ctx *c, int B, int mode, hipGraphExec_t *exec) {
   hipGraph_t graph = nullptr;
   NE_HIP(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
-  const int rc = enqueue_position(c, B, gen, mode);
+  const int rc = enqueue_position(c, B, true, mode);
   const hipError_t ec = hipStreamEndCapture(c->st, &graph);
   if (rc) {
     if (graph) (void)hipGraphDestroy(graph);
@@ -1478,18 +1620,19 @@ int decode_alloc(ne_ctx *c) {
   d->Bmax = c->c.decode_batch;
   d->Bp = d->Bmax <= 16 ? 16 : 32;
   d->ctx = c->c.decode_ctx;
-  const size_t Bp = d->Bp, Bm = d->Bmax, ctx = d->ctx, L = c->L, D = c->D, H = c->H, Q = c->Q, NKV = c->NKV,
+  d->Rp = std::max(d->Bp, pad_rows((int)std::min<long>(PROMPT_ROWS, (long)d->Bmax * (d->ctx - 1))));
+  const size_t Rp = d->Rp, Bp = d->Bp, Bm = d->Bmax, ctx = d->ctx, L = c->L, D = c->D, H = c->H, Q = c->Q, NKV = c->NKV,
                HD = c->HD, V = c->V;
   const size_t kv = L * Bm * NKV * ctx * HD;
   d->lm_nblk = std::max<int>(c->V / (4 * pick_rpw(c->V)), BIG_ARGMAX);
-  d->ws_elems = (long)8 * Bp * std::max<size_t>(2 * H, Q + 2 * NKV * HD);
+  d->ws_elems = (long)8 * Rp * std::max<size_t>(2 * H, Q + 2 * NKV * HD);
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off += (bytes + 255) & ~(size_t)255; return o; };
-  const size_t o_kc = take(kv * 4), o_vc = take(kv * 4), o_x = take(Bp * D * 4);
-  const size_t o_xn = take(Bp * std::max(D, H) * 4);
-  const size_t o_qkv = take(Bp * (Q + 2 * NKV * HD) * 4), o_att = take(Bp * Q * 4);
+  const size_t o_kc = take(kv * 4), o_vc = take(kv * 4), o_x = take(Rp * D * 4);
+  const size_t o_xn = take(Rp * std::max(D, H) * 4);
+  const size_t o_qkv = take(Bp * (Q + 2 * NKV * HD) * 4), o_att = take(Rp * Q * 4);
   const size_t o_lg = take(Bp * V * 4);
-  const size_t o_ws = take((size_t)d->ws_elems * 4), o_gate = take(Bp * H * 4);
+  const size_t o_ws = take((size_t)d->ws_elems * 4), o_gate = take(Rp * H * 4);
   const size_t o_amv = take(Bp * (size_t)d->lm_nblk * 4), o_ami = take(Bp * (size_t)d->lm_nblk * 4);
   const size_t o_tok = take(Bp * 4), o_out = take(Bp * ctx * 4), o_pr = take(Bp * ctx * 4), o_u = take(Bp * ctx * 8);
   // row chunks of at least 1024 columns, a multiple of 4 (16-byte accesses)
@@ -1533,7 +1676,6 @@ void decode_free(ne_ctx *c) {
   Dec *d = (Dec *)c->dec;
   if (!d) return;
   for (auto &g : d->graphs) {
-    if (g.pre) hipGraphExecDestroy(g.pre);
     if (g.gen) hipGraphExecDestroy(g.gen);
   }
   if (d->arena) hipFree(d->arena);
@@ -1542,7 +1684,7 @@ void decode_free(ne_ctx *c) {
 }
 
 namespace {
-int replay(ne_ctx *c, int B, int P, int n_new, int mode);
+int replay(ne_ctx *c, int B, int n_new, int mode);
 }
 
 int decode_run(ne_ctx *c, const int32_t *prompt, int B, int P, int n_new, float temp, float top_p,
@@ -1572,14 +1714,19 @@ int decode_run(ne_ctx *c, const int32_t *prompt, int B, int P, int n_new, float 
       for (int j = 0; j < n_new; j++) u[(size_t)b * d->ctx + j] = uniforms[(size_t)b * n_new + j];
     NE_HIP(hipMemcpyAsync(d->unif, u.data(), u.size() * 8, hipMemcpyHostToDevice, c->st));
   }
-  const DecState s0 = {0, P, temp, top_p};
+  // Prompt positions before the last: in chunks, except the one or two of a small batch (a chunk
+  // takes about as long as two positions of the VALU GEMVs).
+  const bool by_chunk = P - 1 > (B <= VB ? 2 : 1);
+  const DecState s0 = {by_chunk ? P - 1 : 0, P, temp, top_p};
   NE_HIP(hipMemcpyAsync(d->st, &s0, sizeof s0, hipMemcpyHostToDevice, c->st));
   NE_HIP(hipStreamSynchronize(c->st));  // host staging vectors are released at return
 
+  if (by_chunk) NE_CHECK(enqueue_prompt(c, B, P - 1));
+  else for (int pos = 0; pos < P - 1; pos++) NE_CHECK(enqueue_position(c, B, false, mode));
   if (!c->use_graphs) {  // eager launches (tracers that do not follow graph launches)
-    for (int pos = 0; pos < P + n_new - 1; pos++) NE_CHECK(enqueue_position(c, B, pos >= P - 1, mode));
+    for (int j = 0; j < n_new; j++) NE_CHECK(enqueue_position(c, B, true, mode));
   } else {
-    NE_CHECK(replay(c, B, P, n_new, mode));
+    NE_CHECK(replay(c, B, n_new, mode));
   }
   std::vector<int32_t> o((size_t)d->Bp * d->ctx);
   NE_HIP(hipMemcpyAsync(o.data(), d->out, o.size() * 4, hipMemcpyDeviceToHost, c->st));
@@ -1591,24 +1738,18 @@ int decode_run(ne_ctx *c, const int32_t *prompt, int B, int P, int n_new, float 
 
 namespace {
 
-// Replay the captured position graphs (captured on first use per batch size and mode).
-int replay(ne_ctx *c, int B, int P, int n_new, int mode) {
+// Replay the captured graph of a generated position (captured on first use per batch size and mode).
+int replay(ne_ctx *c, int B, int n_new, int mode) {
   Dec *d = (Dec *)c->dec;
   Dec::Graph *gr = nullptr;
   for (auto &g : d->graphs)
     if (g.B == B && g.mode == mode) gr = &g;
   if (!gr) {
-    Dec::Graph g = {B, mode, nullptr, nullptr};
-    int rc = capture(c, B, false, mode, &g.pre);
-    if (!rc) rc = capture(c, B, true, mode, &g.gen);
-    if (rc) {
-      if (g.pre) hipGraphExecDestroy(g.pre);
-      return rc;
-    }
+    Dec::Graph g = {B, mode, nullptr};
+    NE_CHECK(capture(c, B, mode, &g.gen));
     d->graphs.push_back(g);
     gr = &d->graphs.back();
   }
-  for (int pos = 0; pos < P - 1; pos++) NE_HIP(hipGraphLaunch(gr->pre, c->st));
   for (int j = 0; j < n_new; j++) NE_HIP(hipGraphLaunch(gr->gen, c->st));
   return 0;
 }

@@ -106,3 +106,30 @@ def test_decode_sampling_chunks(V, B, gain, top_p):
     m.set("rms_final", np.full(cfg.dim, np.nan, np.float32))
     assert (m.decode(prompt, 2, temp, top_p, u[:, :2]) == 0).all()
     m.close()
+
+
+# The prompt before its last position runs in chunks of up to 256 rows (sequence x position): rows below 16
+# and 32 and at several 32s, chunk borders, the last chunk with one position, batches of both K-cache
+# layouts, and the one or two positions that a small batch takes one at a time.  Picks as in
+# test_decode_sampling_chunks.
+@pytest.mark.parametrize("B,P,fmt,kw", [(1, 2, "bf16", {}), (1, 4, "fp16", {}), (2, 40, "bf16", dict(qk_norm=True)),
+                                        (3, 87, "fp16", dict(head_dim=128, qk_norm=True)), (4, 66, "bf16", {}),
+                                        (5, 53, "bf16", dict(head_dim=128, n_heads=2, qk_norm=True)),
+                                        (5, 2, "fp16", {}), (17, 17, "fp16", dict(n_heads=8)),
+                                        (32, 18, "bf16", dict(dim=256, hidden=384))])
+def test_decode_prompt_chunks(B, P, fmt, kw):
+    cfg = om.tiny(**kw)
+    dt, _, rnd, _ = FMT[fmt]
+    W = {k: rnd(v) for k, v in om.init_params(cfg, seed=P).items()}
+    W["rms_final"] = np.full_like(W["rms_final"], 8.0)
+    n = 6
+    m = ne.Model.from_oracle(cfg, decode_batch=B, decode_ctx=P + n, dtype=dt)
+    m.set_params(W)
+    rng = np.random.default_rng(P + B)
+    prompt, u = rng.integers(0, cfg.vocab, (B, P)).astype(np.int32), rng.random((B, n))
+    got = m.decode(prompt, n, 0.8, 1.0, u)
+    m.use_graphs(False)
+    np.testing.assert_array_equal(m.decode(prompt, n, 0.8, 1.0, u), got)
+    picks, dist = om.decode(cfg, W, prompt, n, temperature=0.8, top_p=1.0, uniforms=u, forced=got)
+    assert np.abs(dist).max() < 1e-5, (np.argwhere(picks != got), np.abs(dist).max())
+    m.close()
