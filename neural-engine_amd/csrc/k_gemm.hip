@@ -45,7 +45,8 @@ __device__ __forceinline__ u16x4 tr4(const h16_t *tile, int row0, int col0) {
 //    16-lane group reads on distinct banks.
 template <int NT, int R, int BK, bool KC>
 struct Stage {
-  static constexpr int PITCH = KC ? BK + 8 : R + 32;
+  // (rows of 32 elements need no pad: 4 of them are one 256-byte pass over the banks)
+  static constexpr int PITCH = KC ? BK + 8 : R == 32 ? 32 : R + 32;
   static constexpr int ELEMS = KC ? R * PITCH : BK * PITCH;
   static constexpr int NCH = R * BK / 8;  // 16-byte chunks
   static constexpr int PER = (NCH + NT - 1) / NT;
@@ -228,7 +229,11 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
-  const int n0 = nt * BN, m0 = mt * BM;
+  // The last tile of an M (N) that is not a multiple of BM (BN) is moved back to end with the
+  // matrix: the K loop needs no bounds, and the epilogue skips the 32-wide fragments that the tile
+  // before it writes (M and N are multiples of 64).
+  const int n0 = min(nt * BN, g.N - BN), m0 = min(mt * BM, g.M - BM);
+  const int m_own = mt * BM, n_own = nt * BN;
   const h16_t *A = (const h16_t *)g.A;
   const h16_t *B = (const h16_t *)g.B;
   // K steps of this split: [kt0, kt1)
@@ -434,6 +439,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const
     for (int i = 0; i < FM; i++)
 #pragma unroll
       for (int j = 0; j < FN; j++) {
+        if (m0 + wm * TM + i * 32 < m_own || n0 + wn * TN + j * 32 < n_own) continue;
         const int col = n0 + wn * TN + j * 32 + (lane & 31);
 #pragma unroll
         for (int e = 0; e < 16; e++) {
@@ -477,6 +483,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const
         const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
         const long grow = m0 + (row / 32) * TM + i * 32 + row % 32;
         const int gcol = n0 + c8 * 8;
+        if (grow < m_own || gcol < n_own) continue;
         if constexpr (EPI == EPI_SWIGLU_BWD) {
           const h16_t *hb = (const h16_t *)g.R;
           h16_t *db = (h16_t *)g.C;
@@ -528,6 +535,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const
   for (int i = 0; i < FM; i++) {
 #pragma unroll
     for (int j = 0; j < FN; j++) {
+      if (m0 + wm * TM + i * 32 < m_own || n0 + wn * TN + j * 32 < n_own) continue;
       const int col = n0 + wn * TN + j * 32 + (lane & 31);
 #pragma unroll
       for (int e = 0; e < 16; e++) {
@@ -614,6 +622,112 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_group_kernel(GemmGroup gg) 
   gemm_body<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KM_TAIL>(g, mt, nt, 0);
 }
 
+// Small outputs without a split-K workspace (the kernel-level entry point on a short step): a
+// BM x BN tile (32 or 64 wide) per block, its K range divided over the block's NW waves.  What
+// bounds these launches is the chain of load latencies of one tile's K loop on the few CUs that
+// get a tile, so a wave keeps DEPTH 64-wide K steps in flight in registers, stages each into LDS of
+// its own (coalesced 16-byte loads, no barrier: a wave's LDS operations run in order) and
+// accumulates the whole tile; the waves' sums meet in LDS in wave order (deterministic), and the
+// epilogue's lanes run along the rows.  256 x
+// 768 x 2048, fp16: 9.5 us on 64x64 tiles (48 work-groups, 16 K steps of 128), 5.6 us on 192
+// blocks of 32x32 with 8 waves.
+template <typename HT, int BM, int BN, int NW, int DEPTH, bool AKC, bool BKC, int EPI>
+__global__ __launch_bounds__(NW * 64) void gemm_kwave_kernel(GemmArgs g) {
+  constexpr int BK = 64, FM = BM / 32, FN = BN / 32, RP = BN + 8;
+  typedef Stage<64, BM, BK, AKC> SA;
+  typedef Stage<64, BN, BK, BKC> SB;
+  constexpr int PER_WAVE = SA::ELEMS + SB::ELEMS;
+  static_assert(BM * RP * 4 <= PER_WAVE * 2, "a wave's partial tile fits its staging area");
+  __shared__ __attribute__((aligned(16))) h16_t lds[NW * PER_WAVE];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int u = xcd_stretch(blockIdx.x, gridDim.x);
+  int mt, nt;
+  grouped_tile(u, g.M / BM, g.N / BN, mt, nt);
+  const int m0 = mt * BM, n0 = nt * BN;
+  const h16_t *A = (const h16_t *)g.A;
+  const h16_t *B = (const h16_t *)g.B;
+  const int nkt = g.K / BK;
+  const int kt0 = (int)((long)nkt * wave / NW), n = (int)((long)nkt * (wave + 1) / NW) - kt0;
+
+  f32x16 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; i++)
+#pragma unroll
+    for (int j = 0; j < FN; j++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
+  h16_t *As = lds + wave * PER_WAVE, *Bs = As + SA::ELEMS;
+  if (n > 0) {  // K steps of this wave: [kt0, kt0 + n); none when K has fewer steps than NW
+    SA sa[DEPTH];
+    SB sb[DEPTH];
+    auto load = [&](int d, int j) {  // past the end: the last step again (valid memory, unused)
+      const int kt = kt0 + min(j, n - 1);
+      sa[d].load(A, g.lda, m0, kt * BK, lane);
+      sb[d].load(B, g.ldb, n0, kt * BK, lane);
+    };
+    auto store = [&](int d) {
+      sa[d].store(As, lane);
+      sb[d].store(Bs, lane);
+      __builtin_amdgcn_wave_barrier();
+    };
+    auto compute = [&]() {
+#pragma unroll
+      for (int kk = 0; kk < BK / 16; kk++) {
+        typename HT::v8 a[FM], b[FN];
+#pragma unroll
+        for (int i = 0; i < FM; i++) a[i] = HT::op(SA::frag(As, i * 32, kk, lane));
+#pragma unroll
+        for (int j = 0; j < FN; j++) b[j] = HT::op(SB::frag(Bs, j * 32, kk, lane));
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+          for (int j = 0; j < FN; j++) acc[i][j] = HT::mfma32(a[i], b[j], acc[i][j]);
+      }
+      __builtin_amdgcn_wave_barrier();
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) load(d, d);
+    int i = 0;
+    for (; i + DEPTH < n; i += DEPTH) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; d++) {
+        store(d);
+        load(d, i + DEPTH + d);
+        compute();
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++)
+      if (i + d < n) {
+        store(d);
+        compute();
+      }
+  }
+  float *red = (float *)As;  // this wave's sums over its own staging area, row pitch RP
+#pragma unroll
+  for (int i = 0; i < FM; i++)
+#pragma unroll
+    for (int j = 0; j < FN; j++)
+#pragma unroll
+      for (int e = 0; e < 16; e++)
+        red[(i * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)) * RP + j * 32 + (lane & 31)] = acc[i][j][e];
+  __syncthreads();
+  bool bad = false;
+  float sq = 0.f;
+#pragma unroll
+  for (int c = 0; c < BM * BN / (NW * 64); c++) {
+    const int el = threadIdx.x + c * NW * 64, row = el / BN, col = el % BN;
+    float s = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) s += ((const float *)(lds + w * PER_WAVE))[row * RP + col];
+    const float o = store_out<HT, EPI>(g, m0 + row, n0 + col, s * g.alpha, bad);
+    if constexpr (epi_sq<EPI>()) sq += o * o;
+  }
+  flag_overflow(g.ovf, bad);
+  if constexpr (epi_sq<EPI>())
+    if (g.sq) block_sumsq_store<NW>(sq, g.sq + (long)mt * (g.N / BN) + nt);
+}
+
 // Ordered sum of the split-K partials (split 0 first) followed by the epilogue; four
 // consecutive columns per thread.  The partials are read KS at a time (KS divides the split,
 // a power of two), all KS loads issued before the first add, so a thread waits on HBM once per
@@ -663,8 +777,11 @@ int reduce_blocks(int M, int N) { return (int)std::min<long>(((long)M * N / 4 + 
 
 template <typename HT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC, int EPI>
 int launch_t(GemmArgs g, hipStream_t s) {
+  if (g.M < BM || g.N < BN || ((g.sq || EPI == EPI_CE_FWD || EPI == EPI_CE_BWD || EPI == EPI_SWIGLU_FWD) &&
+                               (g.M % BM || g.N % BN)))
+    return ne_fail(NE_ERR_ARG, "gemm: a %dx%d tile does not fit %dx%d", BM, BN, g.M, g.N);
   g.n_tiles = g.part_ld > 0 ? g.part_ld : g.N / BN;
-  dim3 grid(g.N / BN, g.M / BM, g.split);
+  dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, g.split);
   if constexpr (EPI == EPI_CE_FWD || EPI == EPI_CE_BWD) {  // never split
     if ((g.K / BK) % 2 == 0)
       hipLaunchKernelGGL((gemm_kernel<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KM_EVEN>), grid, dim3(WM * WN * 64), 0, s, g);
@@ -688,21 +805,42 @@ int launch_t(GemmArgs g, hipStream_t s) {
 }
 
 // Block tiles: 256x256 (8 waves of 64x128), 256x128 (8 waves of 64x64), 128x128 (4 waves of
-// 64x64), 64x64 (4 waves of 32x32).  The 8-wave tiles take most of a CU's LDS (one work-group
-// per CU), the 4-wave tiles fit two.
-enum { TILE_256 = 0, TILE_256x128 = 1, TILE_128 = 2, TILE_64 = 3 };
+// 64x64), 64x64 (4 waves of 32x32).  The 256-row tiles take most of a CU's LDS (one work-group
+// per CU), the others fit two.  Without a split-K workspace also 128x128 and 128x64 on 8 waves
+// (32x64 and 32x32 each) and the K-divided tiles of gemm_kwave_kernel.
+enum { TILE_256 = 0, TILE_256x128 = 1, TILE_128 = 2, TILE_64 = 3, TILE_128W8 = 4, TILE_128x64 = 5, KWAVE_64 = 6,
+       KWAVE_64x32 = 7, KWAVE_32 = 8 };
 constexpr int tile_bm(int t) { return t == TILE_256 || t == TILE_256x128 ? 256 : t == TILE_128 ? 128 : 64; }
 constexpr int tile_bn(int t) { return t == TILE_256 ? 256 : t == TILE_64 ? 64 : 128; }
+
+template <typename HT, int BM, int BN, int NW, int DEPTH, bool AKC, bool BKC, int EPI>
+int launch_kwave(const GemmArgs &g, hipStream_t s) {
+  if (g.M % BM || g.N % BN) return ne_fail(NE_ERR_ARG, "gemm: a %dx%d tile does not fit %dx%d", BM, BN, g.M, g.N);
+  const int blocks = (g.M / BM) * (g.N / BN);
+  hipLaunchKernelGGL((gemm_kwave_kernel<HT, BM, BN, NW, DEPTH, AKC, BKC, EPI>), dim3(blocks), dim3(NW * 64), 0, s, g);
+  return ne_hip_status(hipGetLastError(), "gemm (K over waves)");
+}
 
 template <typename HT, bool AKC, bool BKC, int EPI>
 int launch_e(GemmArgs g, int tile, hipStream_t s) {
   if (tile == TILE_256) return launch_t<HT, 256, 256, 64, 4, 2, AKC, BKC, EPI>(g, s);
   if (tile == TILE_256x128) return launch_t<HT, 256, 128, 64, 4, 2, AKC, BKC, EPI>(g, s);
   if (tile == TILE_128) return launch_t<HT, 128, 128, 64, 2, 2, AKC, BKC, EPI>(g, s);
+  if constexpr (EPI != EPI_CE_FWD && EPI != EPI_CE_BWD && EPI != EPI_SWIGLU_FWD) {
+    if (tile == TILE_128W8) return launch_t<HT, 128, 128, 64, 4, 2, AKC, BKC, EPI>(g, s);
+    if (tile == TILE_128x64) return launch_t<HT, 128, 64, 64, 4, 2, AKC, BKC, EPI>(g, s);
+    if (tile == KWAVE_64) return launch_kwave<HT, 64, 64, 4, 2, AKC, BKC, EPI>(g, s);
+    if (tile == KWAVE_64x32) return launch_kwave<HT, 64, 32, 8, 2, AKC, BKC, EPI>(g, s);
+    if (tile == KWAVE_32) return launch_kwave<HT, 32, 32, 8, 2, AKC, BKC, EPI>(g, s);
+  }
   // The 64x64 tile serves the short-token GEMMs (a 256-token step), whose K loops are bound by
   // the latency of each step's loads: steps of 128 halve the loop's trips (the forward GEMMs of
-  // a 256-token Qwen3-0.6B step: 1.41 -> 1.25 ms, the backward's 2.86 -> 2.68 ms).
-  if (g.K % 128 == 0) return launch_t<HT, 64, 64, 128, 2, 2, AKC, BKC, EPI>(g, s);
+  // a 256-token Qwen3-0.6B step: 1.41 -> 1.25 ms, the backward's 2.86 -> 2.68 ms).  Their LDS (70
+  // KB, 98 KB with an M/N-contiguous operand) leaves room for two work-groups a CU, or one: a
+  // launch with more runs on steps of 64 (fp16, 3264 x 1024 x 4096 NN 96 -> 65 us, 4096 x 4096 x
+  // 1024 rows 3264 NT 80 -> 53 us).
+  const long blocks = (long)(g.M / 64) * (g.N / 64) * g.split;
+  if (g.K % 128 == 0 && blocks <= (AKC && BKC ? 512 : 256)) return launch_t<HT, 64, 64, 128, 2, 2, AKC, BKC, EPI>(g, s);
   return launch_t<HT, 64, 64, 64, 2, 2, AKC, BKC, EPI>(g, s);
 }
 
@@ -745,6 +883,40 @@ int gemm_tile(int M, int N, int K) {
   if (M % 256 == 0 && N % 128 == 0 && (t256x128 >= 200 || (t128 < 128 && K >= 8192))) return TILE_256x128;
   if (M % 128 == 0 && N % 128 == 0 && t128 >= 128) return TILE_128;
   return TILE_64;
+}
+
+// Block tile of a shape without a split-K workspace (the kernel-level entry points), from the
+// time of every tile at some 70 shapes of 64 to 4096 rows (fp16, MI355X; us, the tile that the
+// workspace form's rule gives -> this one's).  mn: an operand is M/N-contiguous.  Tile counts
+// round up: a ragged last tile overlaps the one before it.
+//  * The 256-row tiles while they leave at most a quarter of the CUs idle: 3264x4096x1024 79.6 ->
+//    36.9, 6144x1024x2048 (TN) 47.9 -> 38.1 (the SwiGLU backward's staged epilogue wants more than
+//    one work-group a CU: 2048x3072x1024, 192 tiles, 34.2 on this one, 30.9 on 128x128).
+//  * 128x128 on 8 waves (two work-groups of 4 waves a CU hide no more, and below 256 tiles a CU
+//    has one; above 256 the 4-wave form): 4096x1024x151936 (NN) 1760 -> 1626, 3264x1024x4096 (NN) 96.3 -> 42.3.
+//  * Fewer tiles than that: 128x64 while it is one a CU (2048x1024x6144 (NN) 54.8 -> 45.6,
+//    1024x2048x3264 (TN) 35.1 -> 28.4), else 64x64 if it is two (2496x832x3456 (NN) 40.2 -> 28.6).
+//  * One 64x64 tile a CU or less: the K range over a block's waves, in smaller tiles as they get
+//    fewer (kwave; 256x768x2048 9.5 -> 5.6, 256x1024x6144 (NN) 30.6 -> 16.4, 384x1024x4096 (NN)
+//    21.7 -> 13.7, 1024x1024x6144 (NN) 32.9 -> 26.6), except where the K loop is short (or, at 129
+//    and more tiles, both operands are K-contiguous: 1024x1024x2048 10.3, 12.0 with it), and
+//    except for 16-bit outputs of the forward layout: EPI_SWIGLU_FWD promises their bits, and it
+//    sums K in one chain.
+int gemm_tile_nows(int layout, int epi, int M, int N, int K) {
+  const bool mn = layout != GEMM_NT;
+  auto tiles = [&](int bm, int bn) { return M < bm || N < bn ? 0L : (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  const long t128 = tiles(128, 128), t128x64 = tiles(128, 64), t64 = tiles(64, 64);
+  if (tiles(256, 256) >= 192) return TILE_256;
+  if (tiles(256, 128) >= (epi == EPI_SWIGLU_BWD ? 256 : 192)) return TILE_256x128;
+  if (t128 >= 176) return t128 > 256 ? TILE_128 : TILE_128W8;
+  if (t64 > 256) {
+    if (t128x64 >= 128 && t128x64 <= 256) return TILE_128x64;
+    return t128 >= 128 && t64 > 512 ? TILE_128W8 : TILE_64;
+  }
+  if (!mn && epi == EPI_H16) return TILE_64;
+  if (t64 > 128) return mn && K >= 2048 ? KWAVE_64 : TILE_64;
+  if (t64 > 80) return K >= 1024 ? KWAVE_64x32 : TILE_64;
+  return K >= 512 || t64 <= 16 ? KWAVE_32 : TILE_64;
 }
 
 }  // namespace
@@ -896,6 +1068,13 @@ int gemm_launch(int dt, int layout, int epi, GemmArgs g, hipStream_t s, int *spl
     return ne_fail(NE_ERR_ARG, "gemm: the cross-entropy backward needs 16-byte aligned dlogits rows");
   if (epi == EPI_SWIGLU_FWD && (!g.C || !g.C2 || g.ldc < g.N || g.ldc2 < g.N / 2 || g.N % 128))
     return ne_fail(NE_ERR_ARG, "gemm: the SwiGLU forward needs h13 [M,N] and gate [M,N/2] outputs, N %% 128 == 0");
+  const bool whole = epi == EPI_CE_FWD || epi == EPI_CE_BWD || epi == EPI_SWIGLU_FWD;  // whole tiles only
+  if (!g.ws && !g.sq && !g.defer_reduce && !whole) {
+    g.split = 1;
+    if (split_out) *split_out = 1;
+    const int tile = gemm_tile_nows(layout, epi, g.M, g.N, g.K);
+    return DISPATCH_H16(dt, launch_dt<HT>(layout, epi, g, tile, s));
+  }
   // ragged shapes: the main part of whole 256-wide tiles, then the rest (see ragged_main)
   if (epi != EPI_SWIGLU_BWD && epi != EPI_SWIGLU_FWD && !g.defer_reduce) {
     const size_t ce = epi == EPI_H16 || epi == EPI_CE_BWD || epi == EPI_CE_FWD ? 2 : 4;  // C element size

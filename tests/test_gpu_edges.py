@@ -133,3 +133,43 @@ def test_decode_prompt_chunks(B, P, fmt, kw):
     picks, dist = om.decode(cfg, W, prompt, n, temperature=0.8, top_p=1.0, uniforms=u, forced=got)
     assert np.abs(dist).max() < 1e-5, (np.argwhere(picks != got), np.abs(dist).max())
     m.close()
+
+
+# One shape per tile of the entry point's GEMM: 256x256, 256x128, 128x128 and 128x64 with a last tile that
+# overlaps the one before it (M, N odd multiples of 64), 64x64 on 64-deep steps, and the K-divided tiles of
+# 64x64, 64x32 and 32x32, with fewer K steps than waves (K = 64, 192) and an uneven share of them (K = 576,
+# 1088).  C has rows and columns of its own around it.  fp32 sums of K products: 1e-5 of the largest.
+@pytest.mark.parametrize("M,N,K", [(3136, 4160, 128), (3136, 2112, 64), (1856, 1472, 192), (1088, 1024, 64),
+                                   (2496, 832, 128), (576, 1024, 2112), (384, 1024, 1088), (320, 768, 576),
+                                   (64, 64, 64), (64, 1024, 192)])
+@pytest.mark.parametrize("layout,epi,fmt", [(0, 0, "bf16"), (0, 3, "fp16"), (1, 1, "fp16"), (2, 1, "fp16"),
+                                            (2, 2, "bf16"), (2, 4, "fp16"), (3, 1, "bf16"), (3, 2, "fp16")])
+def test_gemm_tiles(M, N, K, layout, epi, fmt):
+    dt, tdt, _, u = FMT[fmt]
+    g = torch.Generator(device="cuda").manual_seed(M + N + K + layout)
+    rnd = lambda *sh: torch.randn(sh, generator=g, device="cuda")  # noqa: E731
+    A, B = rnd(M, K).to(tdt), rnd(K, N).to(tdt)
+    ref = 0.5 * (A.double() @ B.double())
+    a = A.t().contiguous() if layout & 1 else A
+    b = B if layout & 2 else B.t().contiguous()
+    ld = 2 * N + 8 if epi == 4 else N + 8
+    half = epi in (0, 4)
+    c = torch.full((M + 1, ld), 3.0, device="cuda", dtype=tdt if half else torch.float32)
+    R = rnd(M, 2 * N).to(tdt) if epi == 4 else rnd(M, N) if epi == 3 else None
+    if epi == 2:
+        ref = ref + 3.0
+    elif epi == 3:
+        ref = ref + R.double()
+    elif epi == 4:
+        h1, h3 = R.double()[:, :N], R.double()[:, N:]
+        sg = torch.sigmoid(h1)
+        ref = torch.cat([ref * h3 * sg * (1 + h1 * (1 - sg)), ref * h1 * sg], 1)
+    call(L.ne_k_gemm, dt, layout, epi, M, N, K, ptr(a), a.shape[1], ptr(b), b.shape[1], ptr(c), ld, ptr(R),
+         R.shape[1] if R is not None else 0, 0.5, None)
+    W = ref.shape[1]
+    assert (c[M] == 3.0).all() and (c[:, W:] == 3.0).all()
+    d = c[:M, :W].double() - ref
+    if half:
+        assert float(d.norm() / ref.norm()) < u
+    else:
+        assert float(d.abs().max() / ref.abs().max()) < 1e-5
