@@ -517,14 +517,22 @@ __global__ void gqa_reduce_kernel(AttnArgs a) {
   flag_overflow(a.ovf, bad);
 }
 
-// NW waves per block, RG groups of 16 queries per wave; key tiles of 64 up to the diagonal.
-// Block (bx, by, bz) of a dQ grid nbx blocks wide; lds: [buffer][K tile, V tile].
+// NW waves per block, RG groups of 16 queries per wave; key tiles of 64 up to the diagonal, each in
+// two halves of 32 keys: scores, their gradients and the half's dQ products, so that only a half's
+// scores are live and RG = 2 fits 256 VGPRs (two waves per SIMD).  LDS reads bound this half of the
+// backward: a wave reads 48 KB per key tile whatever RG, against 48 RG MFMAs (4 waves x 48 KB at 128
+// bytes a cycle is twice the MFMAs' cycles at RG = 1).  The
+// backward launch at batch 8 x 2048 (16 / 8 heads of 128, fp16): 815 us with whole tiles and RG = 1,
+// 671 with halves and RG = 2.
+// Block (bx, by, bz) of a dQ grid nbx blocks wide, the last rows first; with S not a multiple of the
+// block's rows the block with the first queries starts below 0, and its waves there only copy.
+// lds: [buffer][K tile, V tile].
 template <typename HT, int HD, int NW, int RG>
-__device__ __forceinline__ void dq_block(const AttnArgs &a, int bx, int by, int bz, int nbx,
+__device__ __forceinline__ void dq_block(const AttnArgs &a, int bx, int by, int bz,
                                          h16_t (*lds)[2 * BLK * (HD + 16)]) {
   constexpr int RP = HD + 16, NK = HD / 32, ND = HD / 16, NT = NW * 64, TILE = BLK * RP;
   constexpr int ROWS = NW * 16 * RG;  // queries per block
-  const int q0 = (nbx - 1 - bx) * ROWS;  // longest rows first
+  const int q0 = a.S - (bx + 1) * ROWS;  // longest rows first
   const int kb_last = (q0 + ROWS - 1) / BLK;
   const int h = by, b = bz;
   const int kvh = h / (a.NH / a.NKV);
@@ -532,6 +540,7 @@ __device__ __forceinline__ void dq_block(const AttnArgs &a, int bx, int by, int 
   const int g = lane >> 4, c16 = lane & 15;
   const long tb = (long)b * a.S;
   const int qw = q0 + w * 16 * RG;
+  const bool act = qw >= 0;  // q0 is a multiple of 32: a wave's queries are all in or all out
   int qi[RG];
   typename HT::v8 qf[RG][NK], df[RG][NK];
   float lse2[RG], dl[RG];
@@ -539,7 +548,7 @@ __device__ __forceinline__ void dq_block(const AttnArgs &a, int bx, int by, int 
 #pragma unroll
   for (int r = 0; r < RG; r++) {
     qi[r] = qw + r * 16 + c16;
-    const long tq = tb + qi[r];
+    const long tq = tb + max(qi[r], 0);
 #pragma unroll
     for (int kk = 0; kk < NK; kk++) {
       qf[r][kk] = ld8<HT>(a.q + tq * a.ldq + h * HD + kk * 32 + g * 8);
@@ -564,57 +573,57 @@ __device__ __forceinline__ void dq_block(const AttnArgs &a, int bx, int by, int 
       cp.load(0, a.k, a.ldk, tb + (kb + 1) * BLK, kvh * HD);
       cp.load(1, a.v, a.ldv, tb + (kb + 1) * BLK, kvh * HD);
     }
-    if (kb * BLK <= qw + 16 * RG - 1) {
-      const h16_t *Ks = lds[cur], *Vs = lds[cur] + TILE;
-      f32x4 sp[RG][4], dp[RG][4];
+    const h16_t *Ks = lds[cur], *Vs = lds[cur] + TILE;
 #pragma unroll
-      for (int nb = 0; nb < 4; nb++)
+    for (int c = 0; c < 2; c++) {
+      const int k0 = kb * BLK + 32 * c;  // the half's first key
+      if (!act || k0 > qw + 16 * RG - 1) continue;
+      f32x4 sp[RG][2], dp[RG][2];
+#pragma unroll
+      for (int n = 0; n < 2; n++)
 #pragma unroll
         for (int r = 0; r < RG; r++) {
-          sp[r][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-          dp[r][nb] = f32x4{-dl[r], -dl[r], -dl[r], -dl[r]};  // the MFMAs leave dP - delta
+          sp[r][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+          dp[r][n] = f32x4{-dl[r], -dl[r], -dl[r], -dl[r]};  // the MFMAs leave dP - delta
         }
 #pragma unroll
       for (int kk = 0; kk < NK; kk++)
 #pragma unroll
-        for (int nb = 0; nb < 4; nb++) {
-          const typename HT::v8 kfrag = ld8<HT>(Ks + (nb * 16 + c16) * RP + kk * 32 + g * 8);
-          const typename HT::v8 vfrag = ld8<HT>(Vs + (nb * 16 + c16) * RP + kk * 32 + g * 8);
+        for (int n = 0; n < 2; n++) {
+          const typename HT::v8 kfrag = ld8<HT>(Ks + (c * 32 + n * 16 + c16) * RP + kk * 32 + g * 8);
+          const typename HT::v8 vfrag = ld8<HT>(Vs + (c * 32 + n * 16 + c16) * RP + kk * 32 + g * 8);
 #pragma unroll
           for (int r = 0; r < RG; r++) {
-            sp[r][nb] = HT::mfma16(kfrag, qf[r][kk], sp[r][nb]);
-            dp[r][nb] = HT::mfma16(vfrag, df[r][kk], dp[r][nb]);
+            sp[r][n] = HT::mfma16(kfrag, qf[r][kk], sp[r][n]);
+            dp[r][n] = HT::mfma16(vfrag, df[r][kk], dp[r][n]);
           }
         }
-      // sp[r][nb][i] = score(key kb*64 + nb*16 + 4g + i, query qi[r])
+      // sp[r][n][i] = score(key k0 + n*16 + 4g + i, query qi[r])
       // Only the last key tile crosses this wave's queries: the others skip the mask.
-      const bool diag = kb * BLK + BLK - 1 > qw;  // some key of the tile above some query
-      typename HT::v8 sb[RG][2];
+      const bool diag = k0 + 31 > qw;  // some key of the half above some query
+      typename HT::v8 sb[RG];
       auto elem = [&](auto masked) {
 #pragma unroll
         for (int r = 0; r < RG; r++) {
 #pragma unroll
-          for (int nb = 0; nb < 4; nb++)
+          for (int n = 0; n < 2; n++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-              float p = fexp2(fmaf(sp[r][nb][i], sl2, -lse2[r]));
-              if (decltype(masked)::value && kb * BLK + nb * 16 + g * 4 + i > qi[r]) p = 0.f;
-              dp[r][nb][i] = p * dp[r][nb][i];
+              float p = fexp2(fmaf(sp[r][n][i], sl2, -lse2[r]));
+              if (decltype(masked)::value && k0 + n * 16 + g * 4 + i > qi[r]) p = 0.f;
+              dp[r][n][i] = p * dp[r][n][i];
             }
-          sb[r][0] = pack_acc<HT>(dp[r][0], dp[r][1]);
-          sb[r][1] = pack_acc<HT>(dp[r][2], dp[r][3]);
+          sb[r] = pack_acc<HT>(dp[r][0], dp[r][1]);
         }
       };
       if (diag) elem(Bool<true>{});
       else elem(Bool<false>{});
 #pragma unroll
-      for (int c = 0; c < 2; c++)
+      for (int d = 0; d < ND; d++) {
+        const typename HT::v8 kt = tr8<HT, RP>(Ks, c, d * 16);
 #pragma unroll
-        for (int d = 0; d < ND; d++) {
-          const typename HT::v8 kt = tr8<HT, RP>(Ks, c, d * 16);
-#pragma unroll
-          for (int r = 0; r < RG; r++) dq[r][d] = HT::mfma16(kt, sb[r][c], dq[r][d]);
-        }
+        for (int r = 0; r < RG; r++) dq[r][d] = HT::mfma16(kt, sb[r], dq[r][d]);
+      }
     }
     if (kb < kb_last) {
       cp.template store<RP>(0, lds[cur ^ 1]);
@@ -623,6 +632,7 @@ __device__ __forceinline__ void dq_block(const AttnArgs &a, int bx, int by, int 
     __syncthreads();
   }
   // dq[r][d][i] = dQ[query qi[r]][dim d*16 + 4g + i]
+  if (!act) return;
 #pragma unroll
   for (int r = 0; r < RG; r++)
 #pragma unroll
@@ -642,9 +652,9 @@ int check(const AttnArgs &a) {
 
 // Block shape (waves NW, 16-row groups per wave RG) by the work-group count it gives.
 // Two row groups per wave halve the LDS reads per MFMA and double the accumulators: the
-// forward still fits two waves per SIMD with them (used for long sequences); the dK/dV and
-// dQ kernels would drop to one, which costs more than the LDS traffic saves, so they keep
-// one group.  4 waves while 64-row blocks give 256 work-groups, else 2 (short sequences
+// forward and the dQ blocks still fit two waves per SIMD with them (used for long sequences);
+// the dK/dV blocks would drop to one, which costs more than the LDS traffic saves, so they
+// keep one group.  4 waves while 64-row blocks give 256 work-groups, else 2 (short sequences
 // would leave most CUs idle).
 enum { SHAPE_2x1 = 0, SHAPE_4x1 = 1, SHAPE_4x2 = 2 };
 int pick_shape(const AttnArgs &a) {
@@ -680,40 +690,46 @@ int fwd_t(const AttnArgs &a, hipStream_t s) {
 // idle: without the per-query-head split there is one block row per KV head), the rest dQ
 // query blocks.  The two kinds depend only on delta (computed before), so they run side by
 // side: at short sequences each alone leaves half the CUs idle.
-template <typename HT, int HD, int NW, int RG, bool SPLIT>
-__global__ __launch_bounds__(NW * 64) void attn_bwd_kernel(AttnArgs a, int nkv, int nky) {
+// RGQ: 16-query groups per wave of the dQ blocks (the dK / dV blocks have one of 16 keys).
+template <typename HT, int HD, int NW, int RGQ, bool SPLIT>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void attn_bwd_kernel(AttnArgs a, int nkv,
+                                                                                                   int nky) {
   __shared__ __attribute__((aligned(16))) h16_t lds[2][2 * BLK * (HD + 16)];
   __shared__ __attribute__((aligned(16))) float lse_s[2][BLK], ndl_s[2][BLK];
   int bx, by, bz;
   xcd_block(bx, by, bz);
   if (bx < nkv) {
-    if (by < nky) dkdv_block<HT, HD, NW, RG, SPLIT>(a, bx, by, bz, lds, lse_s, ndl_s);
+    if (by < nky) dkdv_block<HT, HD, NW, 1, SPLIT>(a, bx, by, bz, lds, lse_s, ndl_s);
   } else {
-    dq_block<HT, HD, NW, RG>(a, bx - nkv, by, bz, gridDim.x - nkv, lds);
+    dq_block<HT, HD, NW, RGQ>(a, bx - nkv, by, bz, lds);
   }
 }
 
-template <typename HT, int HD, int NW, int RG>
+template <typename HT, int HD, int NW, int RGQ>
 int bwd_hd(const AttnArgs &a, hipStream_t s) {
-  const int nblk = a.S / (16 * NW * RG);  // key blocks of dK / dV = query blocks of dQ
-  const dim3 grid(2 * nblk, a.NH, a.B);
+  const int nblk = a.S / (16 * NW);                              // key blocks of dK / dV
+  const int nq = (a.S + 16 * NW * RGQ - 1) / (16 * NW * RGQ);  // query blocks of dQ
+  const dim3 grid(nblk + nq, a.NH, a.B);
   if (a.part && a.NH != a.NKV) {
-    hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RG, true>), grid, dim3(NW * 64), 0, s, a, nblk, a.NH);
+    hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, true>), grid, dim3(NW * 64), 0, s, a, nblk, a.NH);
     NE_HIP(hipGetLastError());
     if (!a.defer_gqa) {
       const long n4 = (long)a.B * a.S * a.NKV * HD / 4;
       hipLaunchKernelGGL(gqa_reduce_kernel<HT>, dim3((int)std::min<long>((n4 + 255) / 256, 4096)), dim3(256), 0, s, a);
     }
   } else {
-    hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RG, false>), grid, dim3(NW * 64), 0, s, a, nblk, a.NKV);
+    hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, false>), grid, dim3(NW * 64), 0, s, a, nblk, a.NKV);
   }
   return ne_hip_status(hipGetLastError(), "attn_bwd");
 }
 
 template <typename HT, int HD>
 int bwd_shape(const AttnArgs &a, hipStream_t s) {
-  if (pick_shape(a) != SHAPE_2x1) return bwd_hd<HT, HD, 4, 1>(a, s);
-  return bwd_hd<HT, HD, 2, 1>(a, s);
+  if (pick_shape(a) == SHAPE_2x1) return bwd_hd<HT, HD, 2, 1>(a, s);
+  // dQ blocks of 128 queries (two groups a wave) while there is one a CU: batch 3 x 1088 (432 of
+  // them) 151 -> 142 us, batch 8 x 2048 815 -> 671
+  const long dq128 = (long)((a.S + 127) / 128) * a.NH * a.B;
+  return dq128 >= 256 ? bwd_hd<HT, HD, 4, 2>(a, s) : bwd_hd<HT, HD, 4, 1>(a, s);
 }
 
 template <typename HT>
