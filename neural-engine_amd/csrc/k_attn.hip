@@ -92,15 +92,17 @@ struct TileCopy {
   static constexpr int RSTEP = NT / CPR;  // rows between a thread's chunks
   static_assert(NT % CPR == 0 && CH % NT == 0, "tile copy: threads must tile the 64 x HD tile");
   u16x8 v[NSRC][PER];
+  // thread of the NT that copy a tile (blocks of several groups of NT copy a tile a group)
+  __device__ __forceinline__ static int tid() { return threadIdx.x & (NT - 1); }
   __device__ __forceinline__ void load(int s, const h16_t *__restrict__ src, long ld, long t0, int col) {
     const h16_t *b = src + t0 * ld + col;
-    const long off = (long)(threadIdx.x / CPR) * ld + (threadIdx.x % CPR) * 8;
+    const long off = (long)(tid() / CPR) * ld + (tid() % CPR) * 8;
 #pragma unroll
     for (int i = 0; i < PER; i++) v[s][i] = *(const u16x8 *)(b + off + (long)i * RSTEP * ld);
   }
   template <int RP>
   __device__ __forceinline__ void store(int s, h16_t *dst) {
-    h16_t *d = dst + (threadIdx.x / CPR) * RP + (threadIdx.x % CPR) * 8;
+    h16_t *d = dst + (tid() / CPR) * RP + (tid() % CPR) * 8;
 #pragma unroll
     for (int i = 0; i < PER; i++) *(u16x8 *)(d + i * RSTEP * RP) = v[s][i];
   }
@@ -326,10 +328,15 @@ __global__ void attn_delta_kernel(AttnArgs a, long rows) {
 // (reduced by gqa_reduce_kernel); otherwise it loops over the query heads of its kv head
 // (block row by) and writes dK (fp32) and dV (16-bit) directly.  Query tiles of 64 from the
 // block's diagonal on.
-// Block (bx, by, bz) of the dK / dV grid; lds: [buffer][Q tile, dO tile].
-template <typename HT, int HD, int NW, int RG, bool SPLIT>
-__device__ __forceinline__ void dkdv_block(const AttnArgs &a, int bx, int by, int bz, h16_t (*lds)[2 * BLK * (HD + 16)],
-                                           float (*lse_s)[BLK], float (*ndl_s)[BLK]) {
+// HG > 1 (not SPLIT): HG groups of NW waves take the query heads of the KV head in turn, each with
+// LDS tiles of its own, and their sums meet at the end in group order: short sequences leave CUs
+// idle while a block's chain of (head, query tile) steps is what takes the time.
+// Block (bx, by, bz) of the dK / dV grid; lds: [HG][buffer][Q tile, dO tile].
+template <typename HT, int HD, int NW, int RG, bool SPLIT, int HG>
+__device__ __forceinline__ void dkdv_block(const AttnArgs &a, int bx, int by, int bz,
+                                           h16_t (*lds_all)[2][2 * BLK * (HD + 16)], float (*lse_all)[2][BLK],
+                                           float (*ndl_all)[2][BLK]) {
+  static_assert(HG == 1 || !SPLIT, "head groups: whole KV heads");
   constexpr int RP = HD + 16, NK = HD / 32, ND = HD / 16, NT = NW * 64, TILE = BLK * RP;
   constexpr int ROWS = NW * 16 * RG;  // keys per block
   const int nqb = a.S / BLK;
@@ -337,9 +344,14 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs &a, int bx, int by, in
   const int qb_first = k0 / BLK;
   const int ratio = a.NH / a.NKV;
   const int kvh = SPLIT ? by / ratio : by, b = bz;
-  const int h_begin = SPLIT ? by : kvh * ratio, h_end = SPLIT ? by + 1 : (kvh + 1) * ratio;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int hg = HG == 1 ? 0 : threadIdx.x / NT;  // this wave's head group
+  const int nh = SPLIT ? 1 : ratio / HG;          // its heads (the launcher: ratio % HG == 0)
+  const int h_begin = SPLIT ? by : kvh * ratio + hg * nh, h_end = h_begin + nh;
+  const int tid = HG == 1 ? threadIdx.x : threadIdx.x % NT;
+  const int lane = threadIdx.x & 63, w = tid >> 6;
   const int g = lane >> 4, c16 = lane & 15;
+  h16_t(*lds)[2 * TILE] = lds_all[hg];
+  float(*lse_s)[BLK] = lse_all[hg], (*ndl_s)[BLK] = ndl_all[hg];
   const long tb = (long)b * a.S;
   const int kw = k0 + w * 16 * RG;  // first key of this wave
   int ki[RG];
@@ -368,8 +380,8 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs &a, int bx, int by, in
     const int h = h_begin + it / per_head, qb = qb_first + it % per_head;
     cp.load(0, a.q, a.ldq, tb + qb * BLK, h * HD);
     cp.load(1, a.dout, a.lddo, tb + qb * BLK, h * HD);
-    if (threadIdx.x < BLK) {
-      const long t = tb + qb * BLK + threadIdx.x;
+    if (tid < BLK) {
+      const long t = tb + qb * BLK + tid;
       lse_r = a.lse[t * a.NH + h] * LOG2E;
       dl_r = a.delta[t * a.NH + h];
     }
@@ -377,9 +389,9 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs &a, int bx, int by, in
   auto put = [&](int buf) {
     cp.template store<RP>(0, lds[buf]);
     cp.template store<RP>(1, lds[buf] + TILE);
-    if (threadIdx.x < BLK) {
-      lse_s[buf][threadIdx.x] = lse_r;
-      ndl_s[buf][threadIdx.x] = -dl_r;
+    if (tid < BLK) {
+      lse_s[buf][tid] = lse_r;
+      ndl_s[buf][tid] = -dl_r;
     }
   };
   fetch(0);
@@ -454,6 +466,32 @@ __device__ __forceinline__ void dkdv_block(const AttnArgs &a, int bx, int by, in
     }
     if (it + 1 < n_it) put(cur ^ 1);
     __syncthreads();
+  }
+  if constexpr (HG > 1) {  // groups 1.. leave their sums (lane for lane) in their own tiles
+    static_assert(RG * ND * 2 * 4 * NT * 4 <= 2 * TILE * 2 * 2, "a group's sums fit its tiles");
+    f32x4 *mine = (f32x4 *)lds_all[hg][0];
+    if (hg > 0) {
+#pragma unroll
+      for (int r = 0; r < RG; r++)
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+          mine[((r * ND + d) * 2) * NT + tid] = dk[r][d];
+          mine[((r * ND + d) * 2 + 1) * NT + tid] = dv[r][d];
+        }
+    }
+    __syncthreads();
+    if (hg > 0) return;
+#pragma unroll
+    for (int q = 1; q < HG; q++) {
+      const f32x4 *o = (const f32x4 *)lds_all[q][0];
+#pragma unroll
+      for (int r = 0; r < RG; r++)
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+          dk[r][d] += o[((r * ND + d) * 2) * NT + tid];
+          dv[r][d] += o[((r * ND + d) * 2 + 1) * NT + tid];
+        }
+    }
   }
   // dv[r][d][i] = dV[key ki[r]][dim d*16 + 4g + i]
   bool bad = false;
@@ -690,42 +728,53 @@ int fwd_t(const AttnArgs &a, hipStream_t s) {
 // idle: without the per-query-head split there is one block row per KV head), the rest dQ
 // query blocks.  The two kinds depend only on delta (computed before), so they run side by
 // side: at short sequences each alone leaves half the CUs idle.
-// RGQ: 16-query groups per wave of the dQ blocks (the dK / dV blocks have one of 16 keys).
-template <typename HT, int HD, int NW, int RGQ, bool SPLIT>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void attn_bwd_kernel(AttnArgs a, int nkv,
-                                                                                                   int nky) {
-  __shared__ __attribute__((aligned(16))) h16_t lds[2][2 * BLK * (HD + 16)];
-  __shared__ __attribute__((aligned(16))) float lse_s[2][BLK], ndl_s[2][BLK];
+// RGQ: 16-query groups per wave of the dQ blocks (the dK / dV blocks have one of 16 keys).  HG: head
+// groups of the dK / dV blocks, NW waves each; the dQ blocks have HG * NW waves.
+template <typename HT, int HD, int NW, int RGQ, bool SPLIT, int HG>
+__global__ __launch_bounds__(HG * NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void attn_bwd_kernel(AttnArgs a,
+                                                                                                        int nkv,
+                                                                                                        int nky) {
+  __shared__ __attribute__((aligned(16))) h16_t lds[HG][2][2 * BLK * (HD + 16)];
+  __shared__ __attribute__((aligned(16))) float lse_s[HG][2][BLK], ndl_s[HG][2][BLK];
   int bx, by, bz;
   xcd_block(bx, by, bz);
   if (bx < nkv) {
-    if (by < nky) dkdv_block<HT, HD, NW, 1, SPLIT>(a, bx, by, bz, lds, lse_s, ndl_s);
+    if (by < nky) dkdv_block<HT, HD, NW, 1, SPLIT, HG>(a, bx, by, bz, lds, lse_s, ndl_s);
   } else {
-    dq_block<HT, HD, NW, RGQ>(a, bx - nkv, by, bz, lds);
+    dq_block<HT, HD, HG * NW, RGQ>(a, bx - nkv, by, bz, lds[0]);
   }
 }
 
-template <typename HT, int HD, int NW, int RGQ>
+template <typename HT, int HD, int NW, int RGQ, int HG = 1>
 int bwd_hd(const AttnArgs &a, hipStream_t s) {
-  const int nblk = a.S / (16 * NW);                              // key blocks of dK / dV
-  const int nq = (a.S + 16 * NW * RGQ - 1) / (16 * NW * RGQ);  // query blocks of dQ
-  const dim3 grid(nblk + nq, a.NH, a.B);
-  if (a.part && a.NH != a.NKV) {
-    hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, true>), grid, dim3(NW * 64), 0, s, a, nblk, a.NH);
-    NE_HIP(hipGetLastError());
-    if (!a.defer_gqa) {
-      const long n4 = (long)a.B * a.S * a.NKV * HD / 4;
-      hipLaunchKernelGGL(gqa_reduce_kernel<HT>, dim3((int)std::min<long>((n4 + 255) / 256, 4096)), dim3(256), 0, s, a);
+  constexpr int QROWS = 16 * NW * HG * RGQ;
+  const int nblk = a.S / (16 * NW);              // key blocks of dK / dV
+  const int nq = (a.S + QROWS - 1) / QROWS;  // query blocks of dQ
+  const dim3 grid(nblk + nq, a.NH, a.B), block(HG * NW * 64);
+  if constexpr (HG == 1)
+    if (a.part && a.NH != a.NKV) {
+      hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, true, 1>), grid, block, 0, s, a, nblk, a.NH);
+      NE_HIP(hipGetLastError());
+      if (!a.defer_gqa) {
+        const long n4 = (long)a.B * a.S * a.NKV * HD / 4;
+        hipLaunchKernelGGL(gqa_reduce_kernel<HT>, dim3((int)std::min<long>((n4 + 255) / 256, 4096)), dim3(256), 0, s, a);
+      }
+      return ne_hip_status(hipGetLastError(), "attn_bwd");
     }
-  } else {
-    hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, false>), grid, dim3(NW * 64), 0, s, a, nblk, a.NKV);
-  }
+  hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, false, HG>), grid, block, 0, s, a, nblk, a.NKV);
   return ne_hip_status(hipGetLastError(), "attn_bwd");
 }
 
 template <typename HT, int HD>
 int bwd_shape(const AttnArgs &a, hipStream_t s) {
-  if (pick_shape(a) == SHAPE_2x1) return bwd_hd<HT, HD, 2, 1>(a, s);
+  if (pick_shape(a) == SHAPE_2x1) {
+    // Two head groups a dK / dV block (one block a CU: 150 KB of LDS at heads of 128) while all
+    // blocks run at once.  256 tokens, 16 / 8
+    // heads of 128 (128 blocks): 21.5 -> 16.2 us.
+    const long blocks = (long)a.B * (a.S / 32 * a.NKV + a.S / 64 * a.NH);
+    if (!a.part && a.NH / a.NKV % 2 == 0 && blocks <= 256) return bwd_hd<HT, HD, 2, 1, 2>(a, s);
+    return bwd_hd<HT, HD, 2, 1>(a, s);
+  }
   // dQ blocks of 128 queries (two groups a wave) while there is one a CU: batch 3 x 1088 (432 of
   // them) 151 -> 142 us, batch 8 x 2048 815 -> 671
   const long dq128 = (long)((a.S + 127) / 128) * a.NH * a.B;
