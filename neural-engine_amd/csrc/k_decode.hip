@@ -19,6 +19,7 @@
 //  * batch 5..32: v_mfma_f32_16x16x4_f32, 16 weight rows x 16 sequences per MFMA tile,
 //    K split over the 4 waves of a block and over grid.y (fp32 partials, ordered reduction).
 #include <math.h>
+#include <type_traits>
 
 #include "common.h"
 #include "ne_ctx.h"
@@ -50,6 +51,7 @@ struct Dec {
   float *ws;              // MFMA split-K partials
   long ws_elems;
   float *gate;            // [Rp, H] SwiGLU gate (MFMA path)
+  h16_t *xn3, *att3, *gate3;  // bf16 weights, MFMA path: the bf16 parts (part_at) of xn, att, gate
   float *amv;             // argmax partials [Bmax][nblk]
   int32_t *ami;
   int lm_nblk;
@@ -68,6 +70,52 @@ struct Dec {
   struct Graph { int B, mode; hipGraphExec_t gen; };  // mode: PICK_*
   std::vector<Graph> graphs;
 };
+
+// x = hi + mid + lo, three bf16 values obtained by truncation: hi keeps the top 8 significant
+// bits of x, mid the next 8 of the remainder x - hi, lo what is left, so the sum is exact and
+// each product of a bf16 weight with a part is exact in fp32.
+__device__ __forceinline__ void split3(float x, uint16_t &hi, uint16_t &mid, uint16_t &lo) {
+  const uint32_t u = __float_as_uint(x) & 0xFFFF0000u;
+  const float r1 = x - __uint_as_float(u);
+  const uint32_t u1 = __float_as_uint(r1) & 0xFFFF0000u;
+  const float r2 = r1 - __uint_as_float(u1);
+  hi = (uint16_t)(u >> 16);
+  mid = (uint16_t)(u1 >> 16);
+  lo = (uint16_t)(__float_as_uint(r2) >> 16);
+}
+
+// The parts of a row-major [rows, K] matrix as gemv_bf3_kernel reads them: for each tile of 16 rows and
+// step of 32 columns three 1 KB fragments (hi, mid, lo) in lane order (16 (k / 8 % 4) + row % 16, 8
+// columns each), so that a fragment is one contiguous read.  As row-major planes each load of a wave
+// touched 16 rows a power of two apart.
+__device__ __forceinline__ long part_at(long K, long row, long k) {
+  return ((row >> 4) * (K >> 5) + (k >> 5)) * 1536 + (((k >> 3) & 3) * 16 + (row & 15)) * 8 + (k & 7);
+}
+// The three parts of element (row, k), or of 4 from k on (a multiple of 4); p may be null.
+__device__ __forceinline__ void put3(h16_t *p, long K, long row, long k, float v) {
+  if (!p) return;
+  uint16_t h, m, l;
+  split3(v, h, m, l);
+  h16_t *q = p + part_at(K, row, k);
+  q[0] = h;
+  q[512] = m;
+  q[1024] = l;
+}
+__device__ __forceinline__ void put3(h16_t *p, long K, long row, long k, const float4 &v) {
+  if (!p) return;
+  const float f[4] = {v.x, v.y, v.z, v.w};
+  u16x4 h, m, l;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    uint16_t a, b, c;
+    split3(f[i], a, b, c);
+    h[i] = a; m[i] = b; l[i] = c;
+  }
+  h16_t *q = p + part_at(K, row, k);
+  *(u16x4 *)q = h;
+  *(u16x4 *)(q + 512) = m;
+  *(u16x4 *)(q + 1024) = l;
+}
 
 // ------------------------------------------------------------------ GEMV, batch <= 4 ----
 
@@ -253,13 +301,13 @@ __device__ __forceinline__ f32x4 mfma_f32(float a, float b, const f32x4 &c) {
 // blockIdx.z takes the rows NT * 16 * z .. of x (a prompt chunk has more than NT * 16).
 // GATE (one split; W = [W1; W3], gate_n rows each): the block's rows are j0..j0+7 of W1 and
 // the same of W3 (j0 = 8 * blockIdx.x), and it writes out[b, j] = silu(h1) * h3
-// (generate.py:190).  WV waves per block split the K range; each loads up to 8 weight chunks
-// ahead of their use.
+// (generate.py:190).  WV waves per block split the K range (a multiple of 32 each).
 template <typename HT, int NT, bool GATE, int WV = 4>
 __global__ __launch_bounds__(WV * 64) void gemv_mfma_kernel(const h16_t *__restrict__ W, long ldw,
                                                         const float *__restrict__ x, long ldx, int K, int ksplit,
                                                         float *out, long ldo, const float *resid, float alpha,
-                                                        float *ws, int N, int B, int Bp, long gate_n) {
+                                                        float *ws, int N, int B, int Bp, long gate_n,
+                                                        h16_t *out3) {
   __shared__ f32x4 red[WV][NT][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int g = lane >> 4, r = lane & 15;
@@ -271,26 +319,40 @@ __global__ __launch_bounds__(WV * 64) void gemv_mfma_kernel(const h16_t *__restr
 #pragma unroll
   for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   const h16_t *wr = W + row * ldw;
-  for (int base = kbeg; base < kend; base += 8 * 32) {
-    u16x8 wv[8];
+  // G chunks of 32: the weights and the x rows all loaded before the first MFMA (the barrier keeps
+  // them there), no load behind another's use.
+  auto group = [&](int base, auto gc) {
+    constexpr int G = decltype(gc)::value;
+    u16x8 wv[G];
+    float4 xa[G][NT][2];
 #pragma unroll
-    for (int i = 0; i < 8; i++)
-      if (base + i * 32 < kend) wv[i] = __builtin_nontemporal_load((const u16x8 *)(wr + base + i * 32 + g * 8));
+    for (int i = 0; i < G; i++) wv[i] = __builtin_nontemporal_load((const u16x8 *)(wr + base + i * 32 + g * 8));
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int k0 = base + i * 32;
-      if (k0 < kend) {
+    for (int i = 0; i < G; i++)
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
-          const float *xr = x + (long)((blockIdx.z * NT + t) * 16 + r) * ldx + k0 + g * 8;
-          const float4 a0 = *(const float4 *)xr, a1 = *(const float4 *)(xr + 4);
-          const float xv[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-#pragma unroll
-          for (int j = 0; j < 8; j++) acc[t] = mfma_f32(HT::f(wv[i][j]), xv[j], acc[t]);
-        }
+      for (int t = 0; t < NT; t++) {
+        const float *xr = x + (long)((blockIdx.z * NT + t) * 16 + r) * ldx + base + i * 32 + g * 8;
+        xa[i][t][0] = *(const float4 *)xr;
+        xa[i][t][1] = *(const float4 *)(xr + 4);
       }
-    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < G; i++)
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const float4 a0 = xa[i][t][0], a1 = xa[i][t][1];
+        const float xv[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+#pragma unroll
+        for (int j = 0; j < 8; j++) acc[t] = mfma_f32(HT::f(wv[i][j]), xv[j], acc[t]);
+      }
+  };
+  int base = kbeg;
+  for (; base + 4 * 32 <= kend; base += 4 * 32) group(base, std::integral_constant<int, 4>{});
+  if (base + 2 * 32 <= kend) {
+    group(base, std::integral_constant<int, 2>{});
+    base += 2 * 32;
   }
+  if (base < kend) group(base, std::integral_constant<int, 1>{});
 #pragma unroll
   for (int t = 0; t < NT; t++) red[w][t][lane] = acc[t];
   __syncthreads();
@@ -313,7 +375,9 @@ __global__ __launch_bounds__(WV * 64) void gemv_mfma_kernel(const h16_t *__restr
           float *op = &o.x;
 #pragma unroll
           for (int i = 0; i < 4; i++) op[i] = s[i] * (1.f / (1.f + expf(-s[i]))) * h3[i];
-          *(float4 *)(out + b * ldo + (long)blockIdx.x * 8 + g * 4) = o;
+          const long j = (long)blockIdx.x * 8 + g * 4;
+          *(float4 *)(out + b * ldo + j) = o;
+          put3(out3, gate_n, b, j, o);
         }
       } else if (ws) {
         *(f32x4 *)(ws + ((long)blockIdx.y * Bp + b) * N + n) = s;
@@ -331,24 +395,12 @@ __global__ __launch_bounds__(WV * 64) void gemv_mfma_kernel(const h16_t *__restr
 
 // ------------------------------------------- GEMV, batch 5..32, bf16 weights, exact ----
 
-// x = hi + mid + lo, three bf16 values obtained by truncation: hi keeps the top 8 significant
-// bits of x, mid the next 8 of the remainder x - hi, lo what is left, so the sum is exact and
-// each product of a bf16 weight with a part is exact in fp32.
-__device__ __forceinline__ void split3(float x, uint16_t &hi, uint16_t &mid, uint16_t &lo) {
-  const uint32_t u = __float_as_uint(x) & 0xFFFF0000u;
-  const float r1 = x - __uint_as_float(u);
-  const uint32_t u1 = __float_as_uint(r1) & 0xFFFF0000u;
-  const float r2 = r1 - __uint_as_float(u1);
-  hi = (uint16_t)(u >> 16);
-  mid = (uint16_t)(u1 >> 16);
-  lo = (uint16_t)(__float_as_uint(r2) >> 16);
-}
-
 enum { BF3_WS = 0, BF3_GATE = 1, BF3_PLAIN = 2 };
 
 // Products of bf16 weight rows W [N, K] with fp32 x rows [Bp, K] (row stride ldx) on
-// v_mfma_f32_16x16x32_bf16: each x value is split into three bf16 parts (split3) and every
-// weight fragment meets the three, so the sums are of the exact products (fp32 accumulation,
+// v_mfma_f32_16x16x32_bf16: each x value comes as three bf16 parts (split3) in
+// fragment order (part_at), written by the kernel that made the value, and every weight fragment
+// meets the three, so the sums are of the exact products (fp32 accumulation,
 // as the fp32-MFMA GEMV).  A block has 4 * NTW waves: wave w takes batch tile w / 4 (16
 // sequences) and K slice w % 4 of the block's K range (KS steps of 32), holds that slice of x
 // as bf16 parts in registers for all its RT row tiles of 16 weight rows, and the four K
@@ -362,9 +414,9 @@ enum { BF3_WS = 0, BF3_GATE = 1, BF3_PLAIN = 2 };
 // blockIdx.z takes the x rows 16 * NTW * z .. (a prompt chunk has more than 16 * NTW).
 template <int NTW, int RT, int KS, int MODE>
 __global__ __launch_bounds__(NTW * 256) void gemv_bf3_kernel(const h16_t *__restrict__ W, long ldw,
-                                                             const float *__restrict__ x, long ldx,
+                                                             const h16_t *__restrict__ x, int K,
                                                              float *__restrict__ out, long ldo, int N, int B,
-                                                             int Bp, long gate_n) {
+                                                             int Bp, long gate_n, h16_t *__restrict__ out3) {
   __shared__ f32x4 red[3][NTW][RT][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int ksl = w & 3, t = w >> 2;
@@ -379,40 +431,46 @@ __global__ __launch_bounds__(NTW * 256) void gemv_bf3_kernel(const h16_t *__rest
       return (long)blockIdx.x * 16 * RT + rt * 16 + r16;
     }
   };
-  // the weight stream first: every fragment of the wave in flight at once
-  u16x8 wf[RT][KS];
-#pragma unroll
-  for (int rt = 0; rt < RT; rt++) {
+  // The weight stream first: PF row tiles of the wave in flight (all of them up to 16 fragments).
+  // The scheduling barriers keep the loads where they are written: left to itself the compiler
+  // moved them down to their uses (48 VGPRs for 16 fragments and the x parts).  With the x parts in
+  // fragment order: the W1|W3 launch of Qwen3-0.6B at batch 32 9.6 -> 8.6 us at best, 96 positions
+  // 115.6 -> 112.2 ms (116.1 without the barriers).
+  constexpr int PF = RT * KS <= 16 ? RT : 3;
+  u16x8 wf[PF][KS];
+  auto wload = [&](int slot, int rt) {
     const h16_t *wr = W + wrow(rt) * ldw + kb;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) wf[rt][ks] = __builtin_nontemporal_load((const u16x8 *)(wr + ks * 32));
-  }
+    for (int ks = 0; ks < KS; ks++) wf[slot][ks] = __builtin_nontemporal_load((const u16x8 *)(wr + ks * 32));
+  };
+#pragma unroll
+  for (int rt = 0; rt < PF; rt++) wload(rt, rt);
   const int b = (blockIdx.z * NTW + t) * 16 + r16;
   u16x8 xh[KS], xm[KS], xl[KS];
   {
-    const float *xr = x + (long)b * ldx + kb;
+    const h16_t *xr = x + ((long)(blockIdx.z * NTW + t) * (K >> 5) + (blockIdx.y * 4 + ksl) * KS) * 1536 + lane * 8;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      const float4 a0 = *(const float4 *)(xr + ks * 32), a1 = *(const float4 *)(xr + ks * 32 + 4);
-      const float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        uint16_t h, m, l;
-        split3(v[e], h, m, l);
-        xh[ks][e] = h; xm[ks][e] = m; xl[ks][e] = l;
-      }
+      xh[ks] = *(const u16x8 *)(xr + ks * 1536);
+      xm[ks] = *(const u16x8 *)(xr + ks * 1536 + 512);
+      xl[ks] = *(const u16x8 *)(xr + ks * 1536 + 1024);
     }
   }
+  __builtin_amdgcn_sched_barrier(0);
   f32x4 acc[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; rt++) {
     acc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      const bf16x8 a = H16B::op(wf[rt][ks]);
+      const bf16x8 a = H16B::op(wf[rt % PF][ks]);
       acc[rt] = H16B::mfma16(a, H16B::op(xh[ks]), acc[rt]);
       acc[rt] = H16B::mfma16(a, H16B::op(xm[ks]), acc[rt]);
       acc[rt] = H16B::mfma16(a, H16B::op(xl[ks]), acc[rt]);
+    }
+    if constexpr (PF < RT) {
+      if (rt + PF < RT) wload(rt % PF, rt + PF);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
   // acc[rt][i] = sum over this K slice for weight row (tile rt) 4g + i, sequence b
@@ -444,7 +502,9 @@ __global__ __launch_bounds__(NTW * 256) void gemv_bf3_kernel(const h16_t *__rest
           const float h1 = acc[rt][i], h3 = acc[rt + HALF][i];
           op[i] = h1 * (1.f / (1.f + expf(-h1))) * h3;
         }
-        *(float4 *)(out + (long)b * ldo + (long)blockIdx.x * 16 * HALF + rt * 16 + g * 4) = o;
+        const long j = (long)blockIdx.x * 16 * HALF + rt * 16 + g * 4;
+        *(float4 *)(out + (long)b * ldo + j) = o;
+        put3(out3, gate_n, b, j, o);
       }
     }
   } else {
@@ -464,7 +524,7 @@ __global__ __launch_bounds__(NTW * 256) void gemv_bf3_kernel(const h16_t *__rest
 template <int KS>
 __global__ __launch_bounds__(256) void gemv_reduce_rows_kernel(const float *__restrict__ ws, int ksplit, int Bp, int N,
                                                                float *out, long ldo, const float *resid, float alpha,
-                                                               const float *gn, float *xn, float eps) {
+                                                               const float *gn, float *xn, float eps, h16_t *xn3) {
   __shared__ float red[4];
   const int b = blockIdx.x, tid = threadIdx.x;
   float ss = 0.f;
@@ -511,10 +571,18 @@ __global__ __launch_bounds__(256) void gemv_reduce_rows_kernel(const float *__re
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       const int n = tid + 256 * e;
-      if (n < N) xn[(long)b * N + n] = rv[e] / rms * gn[n];
+      if (n < N) {
+        const float v = rv[e] / rms * gn[n];
+        xn[(long)b * N + n] = v;
+        put3(xn3, N, b, n, v);
+      }
     }
   } else {  // read back what this thread wrote
-    for (int n = tid; n < N; n += 256) xn[(long)b * N + n] = out[(long)b * ldo + n] / rms * gn[n];
+    for (int n = tid; n < N; n += 256) {
+      const float v = out[(long)b * ldo + n] / rms * gn[n];
+      xn[(long)b * N + n] = v;
+      put3(xn3, N, b, n, v);
+    }
   }
 }
 
@@ -525,7 +593,7 @@ __global__ __launch_bounds__(256) void gemv_reduce_rows_kernel(const float *__re
 template <typename HT>
 __global__ void dec_token_kernel(const int32_t *__restrict__ prompt, int ctx, const DecState *__restrict__ st,
                                  int32_t *tok, const h16_t *__restrict__ E, float *x, int D, int B,
-                                 const float *__restrict__ gn, float *xn, float eps) {
+                                 const float *__restrict__ gn, float *xn, float eps, h16_t *xn3) {
   __shared__ float red[4];
   const int b = blockIdx.x;
   const int pos = st->pos;
@@ -542,7 +610,11 @@ __global__ void dec_token_kernel(const int32_t *__restrict__ prompt, int ctx, co
   if (threadIdx.x == 0) tok[b] = t;
   if (gn) {  // the RMSNorm of the row (generate.py:81-84), read by the batch-5..32 QKV GEMV
     const float rms = sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)D + eps);
-    for (int i = threadIdx.x; i < D; i += blockDim.x) xn[(long)b * D + i] = x[(long)b * D + i] / rms * gn[i];
+    for (int i = threadIdx.x; i < D; i += blockDim.x) {
+      const float v = x[(long)b * D + i] / rms * gn[i];
+      xn[(long)b * D + i] = v;
+      put3(xn3, D, b, i, v);
+    }
   }
 }
 
@@ -559,7 +631,7 @@ __global__ __launch_bounds__(256) void dec_attn_kernel(const float *__restrict__
                                                        float *kc, float *vc, float *att, int NH, int NKV, int ctx,
                                                        const DecState *__restrict__ st, float eps, double scale,
                                                        const float *__restrict__ qws, int qnz, int Bp, int p0,
-                                                       int nc) {
+                                                       int nc, h16_t *att3) {
   extern __shared__ float sc[];  // [RATIO][ctx]
   constexpr int C4 = HD / 4, NG = 256 / C4, HALF = HD / 2;
   __shared__ float4 qs[RATIO][C4];
@@ -711,7 +783,9 @@ __global__ __launch_bounds__(256) void dec_attn_kernel(const float *__restrict__
       o.x += p.x; o.y += p.y; o.z += p.z; o.w += p.w;
     }
     o.x *= inv; o.y *= inv; o.z *= inv; o.w *= inv;
-    *(float4 *)(att + (long)ri * NH * HD + (long)(qh0 + r) * HD + c * 4) = o;
+    const long k = (long)(qh0 + r) * HD + c * 4;
+    *(float4 *)(att + (long)ri * NH * HD + k) = o;
+    put3(att3, NH * HD, ri, k, o);
   }
 }
 
@@ -720,7 +794,7 @@ __global__ __launch_bounds__(256) void dec_attn_kernel(const float *__restrict__
 template <typename HT>
 __global__ __launch_bounds__(256) void pre_token_kernel(const int32_t *__restrict__ prompt, int ctx, int p0, int nc,
                                                         const h16_t *__restrict__ E, float *x, int D,
-                                                        const float *__restrict__ gn, float *xn, float eps) {
+                                                        const float *__restrict__ gn, float *xn, float eps, h16_t *xn3) {
   __shared__ float red[4];
   const long i = blockIdx.x;
   const int t = prompt[(i / nc) * ctx + p0 + i % nc];
@@ -734,7 +808,11 @@ __global__ __launch_bounds__(256) void pre_token_kernel(const int32_t *__restric
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
   const float rms = sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)D + eps);
-  for (int k = threadIdx.x; k < D; k += 256) xn[i * D + k] = x[i * D + k] / rms * gn[k];
+  for (int k = threadIdx.x; k < D; k += 256) {
+    const float v = x[i * D + k] / rms * gn[k];
+    xn[i * D + k] = v;
+    put3(xn3, D, i, k, v);
+  }
 }
 
 // Keys (QK-norm, RoPE) and values of a prompt chunk into the cache, from the qnz split-K slices
@@ -1263,6 +1341,7 @@ inline int pad_rows(int rows) { return rows <= 16 ? 16 : (rows + 31) / 32 * 32; 
 int gemv_big(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float *x, long ldx, float *wsp, long cap,
              float *out, long ldo, const float *resid, float alpha, int *nz_out, const float *gn = nullptr,
              float *xn = nullptr, bool gate = false) {
+  Dec *d = (Dec *)c->dec;
   if ((gate ? N % 8 : N % 16) || K % 128)
     return ne_fail(NE_ERR_ARG, "decode gemv: N=%d K=%d (need N%%16 (gate: %%8), K%%128)", N, K);
   if (gate && wsp) return ne_fail(NE_ERR_ARG, "decode gemv: the gate form has one split");
@@ -1277,7 +1356,7 @@ int gemv_big(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float
   NE_CHECK(DISPATCH_H16(c->dt, [&] {
     auto go = [&](auto kernel, int threads) {
       hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, c->st, W, (long)K, x, ldx, K, ks, out, ldo, resid, alpha,
-                         wsp, N, B, Bp, (long)N);
+                         wsp, N, B, Bp, (long)N, gate ? d->gate3 : nullptr);
     };
     if (Bp == 16) {
       if (wide) go(gemv_mfma_kernel<HT, 1, true, 8>, 512);
@@ -1297,7 +1376,7 @@ int gemv_big(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float
   if (wsp) {
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(B), dim3(256), 0, c->st, wsp, ks, Bp, N, out, ldo, resid, alpha, gn, xn,
-                         c->c.norm_eps);
+                         c->c.norm_eps, d->xn3);
     };
     if (N > 1024) go(gemv_reduce_rows_kernel<0>);
     else if (ks == 1) go(gemv_reduce_rows_kernel<1>);
@@ -1314,10 +1393,10 @@ int gemv_big(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float
 // 1 after launching; 0: not applicable, nothing launched).  mode BF3_WS: the split-K partials
 // go to d->ws and *nz receives the split count; BF3_GATE: W = [W1; W3] (N rows each), gate
 // [Bp, N] -> out; BF3_PLAIN: out [Bp, ldo] = products.
-int gemv_bf3(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float *x, long ldx, int mode, float *out,
+int gemv_bf3(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const h16_t *x3, int mode, float *out,
              long ldo, int *nz) {
   Dec *d = (Dec *)c->dec;
-  if (c->dt != NE_BF16 || K % 128) return 0;
+  if (c->dt != NE_BF16 || K % 128 || !x3) return 0;
   int ks = 0, rt = 2, ksplit = 1;
   if (mode == BF3_WS) {
     for (int cand : {2, 3, 1})
@@ -1343,7 +1422,8 @@ int gemv_bf3(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float
   const long ldd = mode == BF3_WS ? N : ldo;
   bool done = false;
   auto go = [&](auto kernel, int nt) {
-    hipLaunchKernelGGL(kernel, grid, dim3(nt * 256), 0, c->st, W, (long)K, x, ldx, dst, ldd, N, B, Bp, (long)N);
+    hipLaunchKernelGGL(kernel, grid, dim3(nt * 256), 0, c->st, W, (long)K, x3, K, dst, ldd, N, B, Bp, (long)N,
+                       mode == BF3_GATE ? d->gate3 : nullptr);
     done = true;
   };
 #define NE_BF3(NTW_)                                                                                 \
@@ -1381,15 +1461,15 @@ int gemv_bf3(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float
 
 // Wo / W2 on gemv_bf3_kernel with the split-K sum, residual and RMSNorm of gemv_big's
 // workspace form (gemv_reduce_rows_kernel); returns 0 when not applicable.
-int gemv_bf3_resid(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const float *x, long ldx, float *out, long ldo,
+int gemv_bf3_resid(ne_ctx *c, int B, int Bp, const h16_t *W, int N, int K, const h16_t *x3, float *out, long ldo,
                    const float *resid, float alpha, const float *gn, float *xn) {
   Dec *d = (Dec *)c->dec;
   int ks = 0;
-  const int rc = gemv_bf3(c, B, Bp, W, N, K, x, ldx, BF3_WS, nullptr, 0, &ks);
+  const int rc = gemv_bf3(c, B, Bp, W, N, K, x3, BF3_WS, nullptr, 0, &ks);
   if (rc <= 0) return rc;
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(B), dim3(256), 0, c->st, d->ws, ks, Bp, N, out, ldo, resid, alpha, gn, xn,
-                       c->c.norm_eps);
+                       c->c.norm_eps, d->xn3);
   };
   if (N > 1024) go(gemv_reduce_rows_kernel<0>);
   else if (ks == 1) go(gemv_reduce_rows_kernel<1>);
@@ -1410,7 +1490,8 @@ void attn_go(ne_ctx *c, dim3 grid, size_t sh, const float *gq, const float *gk, 
   const double scale = 1.0 / sqrt((double)c->HD);
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(256), sh, c->st, qkv, c->QKV, gq, gk, d->cosb, d->sinb, kc, vc, d->att, c->NH,
-                       c->NKV, d->ctx, d->st, c->c.norm_eps, scale, qkv, qnz, Bp, p0, nc);
+                       c->NKV, d->ctx, d->st, c->c.norm_eps, scale, qkv, qnz, Bp, p0, nc,
+                       KCOL && !nc ? nullptr : d->att3);
   };
   if (nc > 0) go(dec_attn_kernel<HD, R, KCOL, true>);
   else go(dec_attn_kernel<HD, R, KCOL, false>);
@@ -1456,16 +1537,16 @@ int big_layer_tail(ne_ctx *c, int rows, int Bp, const LayerOff &o, const float *
   const long cap = d->ws_elems;
   const h16_t *Pb = c->Pb;
   const float *g_ffn = c->P + o.g_ffn;
-  int rc = gemv_bf3_resid(c, rows, Bp, Pb + o.wo, D, Q, d->att, Q, d->x, D, d->x, alpha, g_ffn, d->xn);
+  int rc = gemv_bf3_resid(c, rows, Bp, Pb + o.wo, D, Q, d->att3, d->x, D, d->x, alpha, g_ffn, d->xn);
   if (rc < 0) return rc;
   if (!rc)
     NE_CHECK(gemv_big(c, rows, Bp, Pb + o.wo, D, Q, d->att, Q, d->ws, cap, d->x, D, d->x, alpha, nullptr, g_ffn, d->xn));
-  rc = gemv_bf3(c, rows, Bp, Pb + o.w13, H, D, d->xn, D, BF3_GATE, d->gate, H, nullptr);
+  rc = gemv_bf3(c, rows, Bp, Pb + o.w13, H, D, d->xn3, BF3_GATE, d->gate, H, nullptr);
   if (rc < 0) return rc;
   if (!rc)
     NE_CHECK(gemv_big(c, rows, Bp, Pb + o.w13, H, D, d->xn, D, nullptr, 0, d->gate, H, nullptr, 1.f, nullptr, nullptr,
                       nullptr, true));
-  rc = gemv_bf3_resid(c, rows, Bp, Pb + o.w2, D, H, d->gate, H, d->x, D, d->x, alpha, g_next, d->xn);
+  rc = gemv_bf3_resid(c, rows, Bp, Pb + o.w2, D, H, d->gate3, d->x, D, d->x, alpha, g_next, d->xn);
   if (rc < 0) return rc;
   if (!rc)
     NE_CHECK(gemv_big(c, rows, Bp, Pb + o.w2, D, H, d->gate, H, d->ws, cap, d->x, D, d->x, alpha, nullptr, g_next, d->xn));
@@ -1475,7 +1556,7 @@ int big_layer_tail(ne_ctx *c, int rows, int Bp, const LayerOff &o, const float *
 // The QKV products of the rows of xn into d->ws; *qnz receives their split-K slice count.
 int big_qkv(ne_ctx *c, int rows, int Bp, const LayerOff &o, int *qnz) {
   Dec *d = (Dec *)c->dec;
-  const int rc = gemv_bf3(c, rows, Bp, c->Pb + o.wqkv, c->QKV, c->D, d->xn, c->D, BF3_WS, nullptr, 0, qnz);
+  const int rc = gemv_bf3(c, rows, Bp, c->Pb + o.wqkv, c->QKV, c->D, d->xn3, BF3_WS, nullptr, 0, qnz);
   if (rc < 0) return rc;
   if (!rc)
     NE_CHECK(gemv_big(c, rows, Bp, c->Pb + o.wqkv, c->QKV, c->D, d->xn, c->D, d->ws, d->ws_elems, nullptr, 0, nullptr,
@@ -1498,7 +1579,7 @@ int enqueue_prompt(ne_ctx *c, int B, int n_pos) {
     const int nc = std::min(per, n_pos - p0), rows = B * nc, Bp = pad_rows(rows);
     auto token = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, c->st, d->prompt, d->ctx, p0, nc, c->Pb + c->off_E, d->x,
-                         c->D, c->P + c->lo[0].g_att, d->xn, eps);
+                         c->D, c->P + c->lo[0].g_att, d->xn, eps, d->xn3);
     };
     if (c->dt == NE_FP16) token(pre_token_kernel<H16F>);
     else token(pre_token_kernel<H16B>);
@@ -1541,10 +1622,10 @@ int enqueue_position(ne_ctx *c, int B, bool gen, int mode) {
   const float *g0 = small ? nullptr : Pf + c->lo[0].g_att;
   if (c->dt == NE_FP16)
     hipLaunchKernelGGL(dec_token_kernel<H16F>, dim3(B), dim3(256), 0, c->st, d->prompt, d->ctx, d->st, d->tok,
-                       Pb + c->off_E, d->x, D, B, g0, d->xn, eps);
+                       Pb + c->off_E, d->x, D, B, g0, d->xn, eps, d->xn3);
   else
     hipLaunchKernelGGL(dec_token_kernel<H16B>, dim3(B), dim3(256), 0, c->st, d->prompt, d->ctx, d->st, d->tok,
-                       Pb + c->off_E, d->x, D, B, g0, d->xn, eps);
+                       Pb + c->off_E, d->x, D, B, g0, d->xn, eps, d->xn3);
   NE_HIP(hipGetLastError());
   for (int l = 0; l < c->L; l++) {
     const LayerOff &o = c->lo[l];
@@ -1572,7 +1653,7 @@ int enqueue_position(ne_ctx *c, int B, bool gen, int mode) {
         hipLaunchKernelGGL(dec_argmax_kernel, dim3(B), dim3(1024), 0, c->st, d->amv, d->ami, V / (4 * pick_rpw(V)),
                            d->st, d->ctx, d->tok, d->out);
     } else {
-      const int rc = gemv_bf3(c, B, d->Bp, Pb + c->off_E, V, D, d->xn, D, BF3_PLAIN, d->logits, V, nullptr);
+      const int rc = gemv_bf3(c, B, d->Bp, Pb + c->off_E, V, D, d->xn3, BF3_PLAIN, d->logits, V, nullptr);
       if (rc < 0) return rc;
       if (!rc) NE_CHECK(gemv_big(c, B, d->Bp, Pb + c->off_E, V, D, d->xn, D, nullptr, 0, d->logits, V, nullptr, 1.f, nullptr));
       if (greedy) {
@@ -1633,6 +1714,8 @@ int decode_alloc(ne_ctx *c) {
   const size_t o_qkv = take(Bp * (Q + 2 * NKV * HD) * 4), o_att = take(Rp * Q * 4);
   const size_t o_lg = take(Bp * V * 4);
   const size_t o_ws = take((size_t)d->ws_elems * 4), o_gate = take(Rp * H * 4);
+  const size_t parts = c->dt == NE_BF16 ? 3 * Rp * 2 : 0;  // bytes a column of the bf16-part planes
+  const size_t o_xn3 = take(parts * D), o_att3 = take(parts * Q), o_gate3 = take(parts * H);
   const size_t o_amv = take(Bp * (size_t)d->lm_nblk * 4), o_ami = take(Bp * (size_t)d->lm_nblk * 4);
   const size_t o_tok = take(Bp * 4), o_out = take(Bp * ctx * 4), o_pr = take(Bp * ctx * 4), o_u = take(Bp * ctx * 8);
   // row chunks of at least 1024 columns, a multiple of 4 (16-byte accesses)
@@ -1649,6 +1732,11 @@ int decode_alloc(ne_ctx *c) {
   d->logits = (float *)(base + o_lg);
   d->ws = (float *)(base + o_ws);
   d->gate = (float *)(base + o_gate);
+  if (parts) {
+    d->xn3 = (h16_t *)(base + o_xn3);
+    d->att3 = (h16_t *)(base + o_att3);
+    d->gate3 = (h16_t *)(base + o_gate3);
+  }
   d->amv = (float *)(base + o_amv); d->ami = (int32_t *)(base + o_ami);
   d->tok = (int32_t *)(base + o_tok); d->out = (int32_t *)(base + o_out); d->prompt = (int32_t *)(base + o_pr);
   d->unif = (double *)(base + o_u);
