@@ -212,7 +212,7 @@ __device__ __forceinline__ float store_out(const GemmArgs &g, int row, int col, 
 enum { KM_TAIL = 0, KM_EVEN = 1, KM_PAD = 2 };
 
 // One output tile (mt, nt) of split kz: the body of the plain and the grouped kernel.
-template <typename HT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC, int EPI, int KMODE>
+template <typename HT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC, int EPI, int KMODE, bool RAG>
 __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const int nt, const int kz) {
   constexpr int NTHREADS = WM * WN * 64;
   constexpr int TM = BM / WM, TN = BN / WN;
@@ -229,10 +229,11 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
-  // The last tile of an M (N) that is not a multiple of BM (BN) is moved back to end with the
+  // RAG: the last tile of an M (N) that is not a multiple of BM (BN) is moved back to end with the
   // matrix: the K loop needs no bounds, and the epilogue skips the 32-wide fragments that the tile
-  // before it writes (M and N are multiples of 64).
-  const int n0 = min(nt * BN, g.N - BN), m0 = min(mt * BM, g.M - BM);
+  // before it writes (M and N are multiples of 64).  Not on the 256-row tiles: the checks cost their
+  // 16-bit epilogue 8% (16,384 x 4096 x 1024: 148 -> 160 us).
+  const int n0 = RAG ? min(nt * BN, g.N - BN) : nt * BN, m0 = RAG ? min(mt * BM, g.M - BM) : mt * BM;
   const int m_own = mt * BM, n_own = nt * BN;
   const h16_t *A = (const h16_t *)g.A;
   const h16_t *B = (const h16_t *)g.B;
@@ -439,7 +440,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const
     for (int i = 0; i < FM; i++)
 #pragma unroll
       for (int j = 0; j < FN; j++) {
-        if (m0 + wm * TM + i * 32 < m_own || n0 + wn * TN + j * 32 < n_own) continue;
+        if (RAG && (m0 + wm * TM + i * 32 < m_own || n0 + wn * TN + j * 32 < n_own)) continue;
         const int col = n0 + wn * TN + j * 32 + (lane & 31);
 #pragma unroll
         for (int e = 0; e < 16; e++) {
@@ -483,7 +484,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const
         const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
         const long grow = m0 + (row / 32) * TM + i * 32 + row % 32;
         const int gcol = n0 + c8 * 8;
-        if (grow < m_own || gcol < n_own) continue;
+        if (RAG && (grow < m_own || gcol < n_own)) continue;
         if constexpr (EPI == EPI_SWIGLU_BWD) {
           const h16_t *hb = (const h16_t *)g.R;
           h16_t *db = (h16_t *)g.C;
@@ -535,7 +536,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const
   for (int i = 0; i < FM; i++) {
 #pragma unroll
     for (int j = 0; j < FN; j++) {
-      if (m0 + wm * TM + i * 32 < m_own || n0 + wn * TN + j * 32 < n_own) continue;
+      if (RAG && (m0 + wm * TM + i * 32 < m_own || n0 + wn * TN + j * 32 < n_own)) continue;
       const int col = n0 + wn * TN + j * 32 + (lane & 31);
 #pragma unroll
       for (int e = 0; e < 16; e++) {
@@ -594,7 +595,7 @@ __device__ __forceinline__ void grouped_tile(int u, int num_m, int num_n, int &m
   nt = r / gsz;
 }
 
-template <typename HT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC, int EPI, int KMODE>
+template <typename HT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC, int EPI, int KMODE, bool RAG>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g) {
   // The K splits (grid.z) take part in the stretches: an XCD runs all the tiles of a split
   // (tile fastest in the sequence), so a split's slice of the shared operand is fetched into one
@@ -605,7 +606,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs g) {
   const int u = xcd_stretch(blockIdx.x + num_n * (blockIdx.y + num_m * blockIdx.z), plane * gridDim.z);
   int mt, nt;
   grouped_tile(u % plane, num_m, num_n, mt, nt);
-  gemm_body<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KMODE>(g, mt, nt, u / plane);
+  gemm_body<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KMODE, RAG>(g, mt, nt, u / plane);
 }
 
 // Several GEMMs of one shape class in one launch (the weight gradients of a layer): problem
@@ -619,7 +620,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_group_kernel(GemmGroup gg) 
   const GemmArgs &g = gg.g[p];
   int mt, nt;
   grouped_tile(u - gg.first[p], g.M / BM, g.N / BN, mt, nt);
-  gemm_body<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KM_TAIL>(g, mt, nt, 0);
+  gemm_body<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KM_TAIL, false>(g, mt, nt, 0);
 }
 
 // Small outputs without a split-K workspace (the kernel-level entry point on a short step): a
@@ -775,20 +776,19 @@ namespace {
 // Work-groups of the ordered split-K reduction of an M x N output.
 int reduce_blocks(int M, int N) { return (int)std::min<long>(((long)M * N / 4 + 255) / 256, 2048); }
 
-template <typename HT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC, int EPI>
+template <typename HT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC, int EPI, bool RAG = false>
 int launch_t(GemmArgs g, hipStream_t s) {
-  if (g.M < BM || g.N < BN || ((g.sq || EPI == EPI_CE_FWD || EPI == EPI_CE_BWD || EPI == EPI_SWIGLU_FWD) &&
-                               (g.M % BM || g.N % BN)))
+  if (g.M < BM || g.N < BN || ((!RAG || g.sq) && (g.M % BM || g.N % BN)))
     return ne_fail(NE_ERR_ARG, "gemm: a %dx%d tile does not fit %dx%d", BM, BN, g.M, g.N);
   g.n_tiles = g.part_ld > 0 ? g.part_ld : g.N / BN;
   dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, g.split);
   if constexpr (EPI == EPI_CE_FWD || EPI == EPI_CE_BWD) {  // never split
     if ((g.K / BK) % 2 == 0)
-      hipLaunchKernelGGL((gemm_kernel<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KM_EVEN>), grid, dim3(WM * WN * 64), 0, s, g);
+      hipLaunchKernelGGL((gemm_kernel<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KM_EVEN, RAG>), grid, dim3(WM * WN * 64), 0, s, g);
     else
-      hipLaunchKernelGGL((gemm_kernel<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KM_PAD>), grid, dim3(WM * WN * 64), 0, s, g);
+      hipLaunchKernelGGL((gemm_kernel<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KM_PAD, RAG>), grid, dim3(WM * WN * 64), 0, s, g);
   } else {
-    hipLaunchKernelGGL((gemm_kernel<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KM_TAIL>), grid, dim3(WM * WN * 64), 0, s, g);
+    hipLaunchKernelGGL((gemm_kernel<HT, BM, BN, BK, WM, WN, AKC, BKC, EPI, KM_TAIL, RAG>), grid, dim3(WM * WN * 64), 0, s, g);
   }
   NE_HIP(hipGetLastError());
   if (g.split > 1 && !g.defer_reduce) {
@@ -827,8 +827,8 @@ int launch_e(GemmArgs g, int tile, hipStream_t s) {
   if (tile == TILE_256x128) return launch_t<HT, 256, 128, 64, 4, 2, AKC, BKC, EPI>(g, s);
   if (tile == TILE_128) return launch_t<HT, 128, 128, 64, 2, 2, AKC, BKC, EPI>(g, s);
   if constexpr (EPI != EPI_CE_FWD && EPI != EPI_CE_BWD && EPI != EPI_SWIGLU_FWD) {
-    if (tile == TILE_128W8) return launch_t<HT, 128, 128, 64, 4, 2, AKC, BKC, EPI>(g, s);
-    if (tile == TILE_128x64) return launch_t<HT, 128, 64, 64, 4, 2, AKC, BKC, EPI>(g, s);
+    if (tile == TILE_128W8) return launch_t<HT, 128, 128, 64, 4, 2, AKC, BKC, EPI, true>(g, s);
+    if (tile == TILE_128x64) return launch_t<HT, 128, 64, 64, 4, 2, AKC, BKC, EPI, true>(g, s);
     if (tile == KWAVE_64) return launch_kwave<HT, 64, 64, 4, 2, AKC, BKC, EPI>(g, s);
     if (tile == KWAVE_64x32) return launch_kwave<HT, 64, 32, 8, 2, AKC, BKC, EPI>(g, s);
     if (tile == KWAVE_32) return launch_kwave<HT, 32, 32, 8, 2, AKC, BKC, EPI>(g, s);
@@ -888,12 +888,12 @@ int gemm_tile(int M, int N, int K) {
 // Block tile of a shape without a split-K workspace (the kernel-level entry points), from the
 // time of every tile at some 70 shapes of 64 to 4096 rows (fp16, MI355X; us, the tile that the
 // workspace form's rule gives -> this one's).  mn: an operand is M/N-contiguous.  Tile counts
-// round up: a ragged last tile overlaps the one before it.
-//  * The 256-row tiles while they leave at most a quarter of the CUs idle: 3264x4096x1024 79.6 ->
-//    36.9, 6144x1024x2048 (TN) 47.9 -> 38.1 (the SwiGLU backward's staged epilogue wants more than
+// round up: a ragged last tile overlaps the one before it (RAG of gemm_body).
+//  * The 256-row tiles, of whole multiples, while they leave at most a quarter of the CUs idle:
+//    6144x1024x2048 (TN) 47.9 -> 38.1 (the SwiGLU backward's staged epilogue wants more than
 //    one work-group a CU: 2048x3072x1024, 192 tiles, 34.2 on this one, 30.9 on 128x128).
 //  * 128x128 on 8 waves (two work-groups of 4 waves a CU hide no more, and below 256 tiles a CU
-//    has one; above 256 the 4-wave form): 4096x1024x151936 (NN) 1760 -> 1626, 3264x1024x4096 (NN) 96.3 -> 42.3.
+//    has one; above 256 the 4-wave form): 4096x1024x151936 (NN) 1760 -> 1626, 3264x1024x4096 (NN) 96.3 -> 42.3, 3264x4096x1024 79.6 -> 41.5.
 //  * Fewer tiles than that: 128x64 while it is one a CU (2048x1024x6144 (NN) 54.8 -> 45.6,
 //    1024x2048x3264 (TN) 35.1 -> 28.4), else 64x64 if it is two (2496x832x3456 (NN) 40.2 -> 28.6).
 //  * One 64x64 tile a CU or less: the K range over a block's waves, in smaller tiles as they get
@@ -906,9 +906,9 @@ int gemm_tile_nows(int layout, int epi, int M, int N, int K) {
   const bool mn = layout != GEMM_NT;
   auto tiles = [&](int bm, int bn) { return M < bm || N < bn ? 0L : (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   const long t128 = tiles(128, 128), t128x64 = tiles(128, 64), t64 = tiles(64, 64);
-  if (tiles(256, 256) >= 192) return TILE_256;
-  if (tiles(256, 128) >= (epi == EPI_SWIGLU_BWD ? 256 : 192)) return TILE_256x128;
-  if (t128 >= 176) return t128 > 256 ? TILE_128 : TILE_128W8;
+  if (M % 256 == 0 && N % 256 == 0 && tiles(256, 256) >= 192) return TILE_256;
+  if (M % 256 == 0 && N % 128 == 0 && tiles(256, 128) >= (epi == EPI_SWIGLU_BWD ? 256 : 192)) return TILE_256x128;
+  if (t128 >= 176) return t128 > 256 && M % 128 == 0 && N % 128 == 0 ? TILE_128 : TILE_128W8;
   if (t64 > 256) {
     if (t128x64 >= 128 && t128x64 <= 256) return TILE_128x64;
     return t128 >= 128 && t64 > 512 ? TILE_128W8 : TILE_64;
@@ -1069,7 +1069,7 @@ int gemm_launch(int dt, int layout, int epi, GemmArgs g, hipStream_t s, int *spl
   if (epi == EPI_SWIGLU_FWD && (!g.C || !g.C2 || g.ldc < g.N || g.ldc2 < g.N / 2 || g.N % 128))
     return ne_fail(NE_ERR_ARG, "gemm: the SwiGLU forward needs h13 [M,N] and gate [M,N/2] outputs, N %% 128 == 0");
   const bool whole = epi == EPI_CE_FWD || epi == EPI_CE_BWD || epi == EPI_SWIGLU_FWD;  // whole tiles only
-  if (!g.ws && !g.sq && !g.defer_reduce && !whole) {
+  if (!g.ws && !g.sq && !g.defer_reduce && !whole && !ragged_main(g.M, g.N, g.K) && !ragged_main(g.N, g.M, g.K)) {
     g.split = 1;
     if (split_out) *split_out = 1;
     const int tile = gemm_tile_nows(layout, epi, g.M, g.N, g.K);
