@@ -31,6 +31,7 @@ struct H16B {
     u += 0x7FFFu + ((u >> 16) & 1u);
     return (h16_t)(u >> 16);
   }
+  __device__ static __forceinline__ h16_t fma_h(float a, float b, float c) { return h(fmaf(a, b, c)); }
   __device__ static __forceinline__ bool bad(h16_t v) { return (v & 0x7F80u) == 0x7F80u; }
   __device__ static __forceinline__ v8 op(const u16x8 &v) { return __builtin_bit_cast(v8, v); }
   __device__ static __forceinline__ f32x16 mfma32(const v8 &a, const v8 &b, const f32x16 &c) {
@@ -47,6 +48,13 @@ struct H16F {
   typedef f16x8 v8;
   __device__ static __forceinline__ float f(h16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
   __device__ static __forceinline__ h16_t h(float x) { return __builtin_bit_cast(h16_t, (_Float16)x); }
+  // a * b + c rounded once, to fp16.  The compiler picks this instruction for a rounded product sum in
+  // some kernels and rounds to fp32 first in others; written out where kernels promise the same bits.
+  __device__ static __forceinline__ h16_t fma_h(float a, float b, float c) {
+    uint32_t o = 0;  // the instruction keeps the upper half of its destination
+    asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "+v"(o) : "v"(a), "v"(b), "v"(c));
+    return (h16_t)o;
+  }
   // inf or nan after conversion (|x| beyond the fp16 range)
   __device__ static __forceinline__ bool bad(h16_t v) { return (v & 0x7C00u) == 0x7C00u; }
   __device__ static __forceinline__ v8 op(const u16x8 &v) { return __builtin_bit_cast(v8, v); }

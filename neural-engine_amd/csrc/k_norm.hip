@@ -360,8 +360,10 @@ __global__ __launch_bounds__(RG * RMS_NT) void rmsnorm_bwd_kernel(
 // out[j] += sum_r part[r * n + j] for r in [0, rows): the deterministic second pass of the
 // per-block gain-gradient partials.  Block = 64 columns x 16 row groups; row group g sums
 // rows g, g+16, ... in order, then the 16 group sums are added in group order, so the
-// result does not depend on scheduling.  grid.y selects one of two (part, rows, out) sets.
-constexpr int CS_COLS = 64, CS_GROUPS = 16;
+// result does not depend on scheduling.  grid.y selects one of two (part, rows, out) sets.  A group has
+// CS_DEPTH rows in flight: many tokens leave many QK-norm rows (3264 tokens of 16 heads of 128: 13,056), and
+// the sum is one chain (with 4 in flight a step of 3264 tokens and two layers took 2316 us, now 2217).
+constexpr int CS_COLS = 64, CS_GROUPS = 16, CS_DEPTH = 16;
 __global__ __launch_bounds__(CS_COLS * CS_GROUPS) void colsum_kernel(const float *__restrict__ part0, int rows0,
                                                                      float *__restrict__ out0,
                                                                      const float *__restrict__ part1, int rows1,
@@ -375,13 +377,12 @@ __global__ __launch_bounds__(CS_COLS * CS_GROUPS) void colsum_kernel(const float
   float s = 0.f;
   if (j < n) {
     int r = grp;
-    for (; r + 3 * CS_GROUPS < rows; r += 4 * CS_GROUPS) {
-      const float a = part[(long)r * n + j], b = part[(long)(r + CS_GROUPS) * n + j];
-      const float d = part[(long)(r + 2 * CS_GROUPS) * n + j], e = part[(long)(r + 3 * CS_GROUPS) * n + j];
-      s += a;
-      s += b;
-      s += d;
-      s += e;
+    for (; r + (CS_DEPTH - 1) * CS_GROUPS < rows; r += CS_DEPTH * CS_GROUPS) {
+      float v[CS_DEPTH];
+#pragma unroll
+      for (int i = 0; i < CS_DEPTH; i++) v[i] = part[(long)(r + i * CS_GROUPS) * n + j];
+#pragma unroll
+      for (int i = 0; i < CS_DEPTH; i++) s += v[i];
     }
     for (; r < rows; r += CS_GROUPS) s += part[(long)r * n + j];
   }
@@ -407,13 +408,12 @@ __global__ __launch_bounds__(CS_COLS * CS_GROUPS) void colsum_batch_kernel(const
   float s = 0.f;
   if (j < n) {
     int r = grp;
-    for (; r + 3 * CS_GROUPS < rows; r += 4 * CS_GROUPS) {
-      const float a = part[(long)r * n + j], b = part[(long)(r + CS_GROUPS) * n + j];
-      const float d = part[(long)(r + 2 * CS_GROUPS) * n + j], e = part[(long)(r + 3 * CS_GROUPS) * n + j];
-      s += a;
-      s += b;
-      s += d;
-      s += e;
+    for (; r + (CS_DEPTH - 1) * CS_GROUPS < rows; r += CS_DEPTH * CS_GROUPS) {
+      float v[CS_DEPTH];
+#pragma unroll
+      for (int i = 0; i < CS_DEPTH; i++) v[i] = part[(long)(r + i * CS_GROUPS) * n + j];
+#pragma unroll
+      for (int i = 0; i < CS_DEPTH; i++) s += v[i];
     }
     for (; r < rows; r += CS_GROUPS) s += part[(long)r * n + j];
   }
@@ -556,34 +556,135 @@ __global__ __launch_bounds__(256) void qk_prep_fwd_kernel(h16_t *__restrict__ qk
   flag_overflow(ovf_qkv, bad);
 }
 
-// Backward of qk_prep: inverse rotation (TD/cpu_ops.h:510-537), then the exact per-head RMSNorm
-// backward.  HBM-bound: reads dq, dk (fp32) and the q and k columns of qkv, writes their
-// columns of dqkv.  A head slot (one head of one token) is HD/8 consecutive lanes owning 8
-// elements each, so every access is 16 bytes; a block takes tok_per_block tokens and its slots run
-// over the (token, head) items of those, so a lane meets the same 8 columns of a head every time
-// and keeps their q- and k-gain sums in registers for the whole block: they meet in LDS once, at its
-// end, and leave as one partial row of q and one of k per block (reduced by colsum_kernel) or,
-// without `part` (the kernel entry point has no scratch), as one atomic per channel and block.
-// Before (one head per block, 8-byte accesses, the atomics of every head's blocks on the same
-// lines, about 22 ns each, one after the other) the entry point took 171 us for 16,384 tokens of
-// 16 + 8 heads of 128, 697 us for 3,264 tokens and 53 us for 256; now 96 (408 MB: 4.2 TB/s), 25 and
-// 8.5 us.  In a training step (partial rows, no atomics) 256 tokens take the same 5.9 us.
-// With kvpart (per-query-head dK/dV partials, [2][T, NH*HD]) a k slot sums its query heads'
-// dK partials in head order, and NKV further slots per token sum dV into dqkv's v columns.
-template <typename HT, bool QKN, int HD>
+// Backward of qk_prep: inverse rotation (TD/cpu_ops.h:510-537), then the exact
+// per-head RMSNorm backward; gain gradients reduced per block, one atomic per channel.
+// Block = 256 threads = 256/(HD/2) token rows of one head slot; grid.y = head slot.
+template <typename HT, bool QKN>
 __global__ __launch_bounds__(256) void qk_prep_bwd_kernel(
     const float *__restrict__ dq, const float *__restrict__ dk, const h16_t *__restrict__ qkv, long ld,
     const float *__restrict__ cosb, const float *__restrict__ sinb, const float *__restrict__ gq,
     const float *__restrict__ gk, const float *__restrict__ rq, const float *__restrict__ rk,
     h16_t *__restrict__ dqkv, float *__restrict__ dgq, float *__restrict__ dgk, float dg_scale, int T,
-    int S, int NH, int NKV, int tok_per_block, int *ovf, float *__restrict__ part,
+    int S, int NH, int NKV, int HD, int tok_per_block, int *ovf, float *__restrict__ part,
     const float *__restrict__ kvpart, int *ovf_v) {
+  bool bad = false;
+  __shared__ float red[256 * 2];
+  const int half = HD / 2;
+  const int i = threadIdx.x % half;
+  const int sub = threadIdx.x / half, nsub = 256 / half;
+  const int h = blockIdx.y;
+  const int ratio = NH / NKV;
+  if (h >= NH + NKV) {
+    // dV of kv head h - NH - NKV: the head-order sum of its query heads' partials (kvpart's
+    // second half), rounded to 16 bits into dqkv's v columns
+    const int kvh = h - NH - NKV;
+    const float *pv = kvpart + (long)T * NH * HD;
+    const long t0 = (long)blockIdx.x * tok_per_block, t1 = min((long)T, t0 + tok_per_block);
+    for (long t = t0 + sub; t < t1; t += nsub) {
+      float2 sv = make_float2(0.f, 0.f);
+      for (int r = 0; r < ratio; r++) {
+        const float2 y = *(const float2 *)(pv + t * NH * HD + (long)(kvh * ratio + r) * HD + 2 * i);
+        sv.x += y.x; sv.y += y.y;
+      }
+      const h16_t o0 = HT::h(sv.x), o1 = HT::h(sv.y);
+      bad |= HT::bad(o0) | HT::bad(o1);
+      *(uint32_t *)(dqkv + t * ld + (long)(NH + NKV) * HD + (long)kvh * HD + 2 * i) = (uint32_t)o0 | ((uint32_t)o1 << 16);
+    }
+    flag_overflow(ovf_v, bad);
+    return;
+  }
+  const bool isq = h < NH;
+  const int hh = isq ? h : h - NH;
+  const long col = (isq ? 0 : (long)NH * HD) + (long)hh * HD + 2 * i;
+  const float *gg = isq ? gq : gk;
+  float g0 = 0.f, g1 = 0.f;
+  if (QKN) {
+    g0 = gg[2 * i];
+    g1 = gg[2 * i + 1];
+  }
+  float a0 = 0.f, a1 = 0.f;
+  const long t0 = (long)blockIdx.x * tok_per_block;
+  const long t1 = min((long)T, t0 + tok_per_block);
+  for (long t = t0 + sub; t < t1; t += nsub) {
+    float2 dd;
+    if (isq) {
+      dd = *(const float2 *)(dq + t * (long)NH * HD + (long)hh * HD + 2 * i);
+    } else if (kvpart) {  // dK: the head-order sum of the query heads' partials
+      dd = make_float2(0.f, 0.f);
+      for (int r = 0; r < ratio; r++) {
+        const float2 y = *(const float2 *)(kvpart + t * (long)NH * HD + (long)(hh * ratio + r) * HD + 2 * i);
+        dd.x += y.x; dd.y += y.y;
+      }
+    } else {
+      dd = *(const float2 *)(dk + t * (long)NKV * HD + (long)hh * HD + 2 * i);
+    }
+    const int pos = t % S;
+    const float c = cosb[pos * half + i], s = sinb[pos * half + i];
+    float d0 = dd.x * c + dd.y * s;
+    float d1 = dd.y * c - dd.x * s;
+    if (QKN) {
+      const uint32_t pr = *(const uint32_t *)(qkv + t * ld + col);
+      const float x0 = HT::f((h16_t)(pr & 0xFFFF)), x1 = HT::f((h16_t)(pr >> 16));
+      const float r = isq ? rq[t * NH + hh] : rk[t * NKV + hh];
+      float dot = d0 * x0 * g0 + d1 * x1 * g1;
+      dot = half == 64 ? group_sum<64>(dot) : group_sum<32>(dot);  // HD = 128 or 64
+      const float cc = r * r * r * dot / (float)HD;
+      a0 += d0 * x0 * r;
+      a1 += d1 * x1 * r;
+      d0 = r * g0 * d0 - x0 * cc;
+      d1 = r * g1 * d1 - x1 * cc;
+    }
+    const h16_t o0 = HT::h(d0), o1 = HT::h(d1);
+    bad |= HT::bad(o0) | HT::bad(o1);
+    *(uint32_t *)(dqkv + t * ld + col) = (uint32_t)o0 | ((uint32_t)o1 << 16);
+  }
+  flag_overflow(ovf, bad);
+  if (QKN) {
+    red[threadIdx.x * 2] = a0;
+    red[threadIdx.x * 2 + 1] = a1;
+    __syncthreads();
+    if (sub == 0) {
+      float s0 = 0.f, s1 = 0.f;
+      for (int k = 0; k < nsub; k++) {
+        s0 += red[(k * half + i) * 2];
+        s1 += red[(k * half + i) * 2 + 1];
+      }
+      if (part) {  // layout [head slot][token block][HD], reduced by colsum_kernel
+        float *pp = part + ((long)h * gridDim.x + blockIdx.x) * HD;
+        pp[2 * i] = dg_scale * s0;
+        pp[2 * i + 1] = dg_scale * s1;
+      } else {
+        float *dg = isq ? dgq : dgk;
+        atomicAdd(dg + 2 * i, dg_scale * s0);
+        atomicAdd(dg + 2 * i + 1, dg_scale * s1);
+      }
+    }
+  }
+}
+
+// The same backward where there are no partials to write or read (the kernel entry point: it has no
+// scratch) and every access can be 16 bytes (the launcher checks).  HBM-bound: reads dq, dk (fp32) and
+// the q and k columns of qkv, writes their columns of dqkv.  A head slot (one head of one token) is
+// HD/8 consecutive lanes owning 8 elements each; a block takes tok_per_block tokens and its slots run
+// over the (token, head) items of those, so a lane meets the same 8 columns of a head every time and
+// keeps their q- and k-gain sums in registers for the whole block: they meet in LDS once, at its end,
+// and leave as one atomic per channel and block.  The kernel above (one head per block, 4- and 8-byte
+// accesses, the atomics of every head's blocks on the same lines, about 22 ns each, one after the other)
+// takes 171 us for 16,384 tokens of 16 + 8 heads of 128, 698 us for 3264 and 52 us for 256; this one 95
+// (408 MB: 4.3 TB/s), 25 and 7.6 us.  The same products in the same order of sums as that kernel (a lane's
+// 4 pairs are the butterfly's first two strides; fused multiply-adds written out): the same dqkv bits.
+template <typename HT, bool QKN, int HD>
+__global__ __launch_bounds__(256) void qk_prep_bwd_wide_kernel(
+    const float *__restrict__ dq, const float *__restrict__ dk, const h16_t *__restrict__ qkv, long ld,
+    const float *__restrict__ cosb, const float *__restrict__ sinb, const float *__restrict__ gq,
+    const float *__restrict__ gk, const float *__restrict__ rq, const float *__restrict__ rk,
+    h16_t *__restrict__ dqkv, float *__restrict__ dgq, float *__restrict__ dgk, float dg_scale, int T,
+    int S, int NH, int NKV, int tok_per_block, int *ovf) {
   constexpr int TPH = HD / 8, HALF = HD / 2, SPB = 256 / TPH;  // lanes per slot, slots per block
   const int j = threadIdx.x % TPH;
-  const int ratio = NH / NKV;
-  const int slots = kvpart ? NH + 2 * NKV : NH + NKV;
+  const int slots = NH + NKV;
   const int t0 = blockIdx.x * tok_per_block, nt = min(tok_per_block, T - t0);
-  bool bad = false, bad_v = false;
+  bool bad = false;
   float gqv[8], gkv[8], aq[8], ak[8];
 #pragma unroll
   for (int e = 0; e < 8; e++) {
@@ -591,107 +692,73 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_kernel(
     gqv[e] = QKN ? gq[8 * j + e] : 0.f;
     gkv[e] = QKN ? gk[8 * j + e] : 0.f;
   }
-  // An item's loads are issued before the item before it is worked on: two items, and for GQA
-  // partials two query heads of each, are in flight per lane.
+  // An item's loads are issued before the item before it is worked on: two items are in flight per lane.
   struct Item {
-    float4 d[2][2];  // dq / dk, or the partials of the first two query heads
-    float4 c4, s4;
+    float4 d[2], c4, s4;
     u16x8 pr;
     float r;
   };
   const int n = nt * slots;
-  auto place = [&](int w, long &t, int &h, int &hh, long &col) {
-    t = t0 + w / slots;
-    h = w % slots;
-    hh = h < NH ? h : h < NH + NKV ? h - NH : h - NH - NKV;
-    col = (h < NH ? 0 : h < NH + NKV ? (long)NH * HD : (long)(NH + NKV) * HD) + (long)hh * HD + 8 * j;
-  };
-  auto partials = [&](long t, int h, int hh) {
-    return kvpart + (h >= NH + NKV ? (long)T * NH * HD : 0) + t * (long)NH * HD + (long)hh * ratio * HD + 8 * j;
-  };
   auto load = [&](int w, Item &it) {
-    long t, col;
-    int h, hh;
-    place(w, t, h, hh, col);
+    const long t = t0 + w / slots;
+    const int h = w % slots;
     const bool isq = h < NH;
-    const float *p = isq      ? dq + t * (long)NH * HD + (long)hh * HD + 8 * j
-                     : kvpart ? partials(t, h, hh)
-                              : dk + t * (long)NKV * HD + (long)hh * HD + 8 * j;
-    it.d[0][0] = *(const float4 *)p;
-    it.d[0][1] = *(const float4 *)(p + 4);
-    if (!isq && kvpart && ratio > 1) {
-      it.d[1][0] = *(const float4 *)(p + HD);
-      it.d[1][1] = *(const float4 *)(p + HD + 4);
-    } else {
-      it.d[1][0] = it.d[1][1] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    if (h >= NH + NKV) return;
+    const float *p = isq ? dq + (t * NH + h) * HD + 8 * j : dk + (t * NKV + h - NH) * HD + 8 * j;
+    it.d[0] = *(const float4 *)p;
+    it.d[1] = *(const float4 *)(p + 4);
     const long pos = t % S;
     it.c4 = *(const float4 *)(cosb + pos * HALF + 4 * j);
     it.s4 = *(const float4 *)(sinb + pos * HALF + 4 * j);
     if (QKN) {
-      it.pr = *(const u16x8 *)(qkv + t * ld + col);
-      it.r = isq ? rq[t * NH + hh] : rk[t * NKV + hh];
+      it.pr = *(const u16x8 *)(qkv + t * ld + (long)h * HD + 8 * j);  // the k heads follow the q heads
+      it.r = isq ? rq[t * NH + h] : rk[t * NKV + h - NH];
     }
   };
   // whole head slots are active or idle together, so the sums below stay within a slot
   auto finish = [&](int w, const Item &it) {
-    long t, col;
-    int h, hh;
-    place(w, t, h, hh, col);
+    const long t = t0 + w / slots;
+    const int h = w % slots;
     const bool isq = h < NH;
-    float d[8] = {it.d[0][0].x + it.d[1][0].x, it.d[0][0].y + it.d[1][0].y, it.d[0][0].z + it.d[1][0].z,
-                  it.d[0][0].w + it.d[1][0].w, it.d[0][1].x + it.d[1][1].x, it.d[0][1].y + it.d[1][1].y,
-                  it.d[0][1].z + it.d[1][1].z, it.d[0][1].w + it.d[1][1].w};
-    if (!isq && kvpart)
-      for (int r = 2; r < ratio; r++) {
-        const float *p = partials(t, h, hh) + (long)r * HD;
-        const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 4);
-        d[0] += a.x; d[1] += a.y; d[2] += a.z; d[3] += a.w;
-        d[4] += b.x; d[5] += b.y; d[6] += b.z; d[7] += b.w;
-      }
-    u16x8 o;
-    if (h >= NH + NKV) {
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        o[e] = HT::h(d[e]);
-        bad_v |= HT::bad(o[e]);
-      }
-      *(u16x8 *)(dqkv + t * ld + col) = o;
-      return;
-    }
     const float cv[4] = {it.c4.x, it.c4.y, it.c4.z, it.c4.w}, sv[4] = {it.s4.x, it.s4.y, it.s4.z, it.s4.w};
+    const float in[8] = {it.d[0].x, it.d[0].y, it.d[0].z, it.d[0].w, it.d[1].x, it.d[1].y, it.d[1].z, it.d[1].w};
+    u16x8 o;
+    if (!QKN) {
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const float d0 = d[2 * q] * cv[q] + d[2 * q + 1] * sv[q];
-      const float d1 = d[2 * q + 1] * cv[q] - d[2 * q] * sv[q];
-      d[2 * q] = d0;
-      d[2 * q + 1] = d1;
-    }
-    if (QKN) {
+      for (int q = 0; q < 4; q++) {
+        o[2 * q] = HT::fma_h(in[2 * q], cv[q], in[2 * q + 1] * sv[q]);
+        o[2 * q + 1] = HT::fma_h(in[2 * q + 1], cv[q], -(in[2 * q] * sv[q]));
+      }
+    } else {
       const float r = it.r;
-      float x[8], dot = 0.f;
+      float d[8], x[8], dx[8], pair[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        d[2 * q] = fmaf(in[2 * q], cv[q], in[2 * q + 1] * sv[q]);
+        d[2 * q + 1] = fmaf(in[2 * q + 1], cv[q], -(in[2 * q] * sv[q]));
+      }
 #pragma unroll
       for (int e = 0; e < 8; e++) {
         x[e] = HT::f(it.pr[e]);
-        dot += d[e] * x[e] * (isq ? gqv[e] : gkv[e]);
+        dx[e] = d[e] * x[e];
       }
-      dot = group_sum<TPH>(dot);
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        pair[q] = fmaf(dx[2 * q], isq ? gqv[2 * q] : gkv[2 * q], dx[2 * q + 1] * (isq ? gqv[2 * q + 1] : gkv[2 * q + 1]));
+      const float dot = group_sum<TPH>((pair[0] + pair[1]) + (pair[2] + pair[3]));
       const float cc = r * r * r * dot / (float)HD;
 #pragma unroll
       for (int e = 0; e < 8; e++) {
-        const float a = d[e] * x[e] * r;
+        const float a = dx[e] * r;
         aq[e] += isq ? a : 0.f;
         ak[e] += isq ? 0.f : a;
-        d[e] = r * (isq ? gqv[e] : gkv[e]) * d[e] - x[e] * cc;
+        float v = fmaf(r * (isq ? gqv[e] : gkv[e]), d[e], -(x[e] * cc));
+        asm volatile("" : "+v"(v));  // rounded to fp32 first
+        o[e] = HT::h(v);
       }
     }
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      o[e] = HT::h(d[e]);
-      bad |= HT::bad(o[e]);
-    }
-    *(u16x8 *)(dqkv + t * ld + col) = o;
+    for (int e = 0; e < 8; e++) bad |= HT::bad(o[e]);
+    *(u16x8 *)(dqkv + t * ld + (long)h * HD + 8 * j) = o;
   };
   int w = threadIdx.x / TPH;
   Item ia, ib;
@@ -703,7 +770,6 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_kernel(
     if (w + SPB < n) finish(w + SPB, ib);
   }
   flag_overflow(ovf, bad);
-  flag_overflow(ovf_v, bad_v);
   if constexpr (QKN) {
     __shared__ float comb[SPB][2 * HD];
     const int sb = threadIdx.x / TPH;
@@ -718,9 +784,7 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_kernel(
       float v = 0.f;
 #pragma unroll
       for (int k = 0; k < SPB; k++) v += comb[k][i];
-      v *= dg_scale;
-      if (part) part[i < HD ? (long)blockIdx.x * HD + i : ((long)gridDim.x + blockIdx.x) * HD + i - HD] = v;
-      else atomicAdd(i < HD ? dgq + i : dgk + i - HD, v);
+      atomicAdd(i < HD ? dgq + i : dgk + i - HD, dg_scale * v);
     }
   }
 }
@@ -767,10 +831,13 @@ namespace {
 int rms_rows(int T) { return std::max(1, (T + 1023) / 1024); }  // rows per block: <= 1024 blocks
 // Rows per block of the form that adds its gain sums with atomics: <= 256 blocks of 4 row groups.
 int rms_rows_atomic(int T) { return 4 * std::max(1, (T + 1023) / 1024); }
-// Tokens per block of the QK-prep backward: as few as one on short steps (a block is a chain of
-// dependent loads per 16 or 32 head slots), at most 1024 blocks on long ones; at most 512 where
-// every block ends in atomics on the same lines.
-int qk_tpb(int T, bool atomics) {
+// Tokens per block of the QK-prep backward: on short steps one per thread group (HD/2 threads a
+// token), so a block runs one pass and there are 4x-8x more blocks (256 tokens: 10.3 us with
+// 16 tokens a block, four passes of dependent loads); 128 on long steps.
+int qk_tpb(int T, int HD) { return T <= 4096 ? 512 / HD : 128; }
+// Of its wide form: as few as one on short steps (a block is a chain of dependent loads per 16 or 32 head
+// slots), at most 1024 blocks on long ones; at most 512 where every block ends in atomics on the same lines.
+int qk_tpb_wide(int T, bool atomics) {
   const int most = atomics ? 512 : 1024;
   return std::max(atomics ? 2 : 1, (T + most - 1) / most);
 }
@@ -778,8 +845,10 @@ int qk_tpb(int T, bool atomics) {
 
 long rmsnorm_bwd_part_elems(int T, int D) { return (long)((T + rms_rows(T) - 1) / rms_rows(T)) * D; }
 int rmsnorm_bwd_part_rows(int T) { return (T + rms_rows(T) - 1) / rms_rows(T); }
-void qk_prep_bwd_part_rows(int T, int *rows_q, int *rows_k) {
-  *rows_q = *rows_k = (T + qk_tpb(T, false) - 1) / qk_tpb(T, false);
+void qk_prep_bwd_part_rows(int T, int NH, int NKV, int HD, int *rows_q, int *rows_k) {
+  const int nbx = (T + qk_tpb(T, HD) - 1) / qk_tpb(T, HD);
+  *rows_q = NH * nbx;
+  *rows_k = NKV * nbx;
 }
 
 int launch_colsum_batch(const ColsumJob *jobs_dev, int njobs, int max_n, hipStream_t s) {
@@ -788,8 +857,8 @@ int launch_colsum_batch(const ColsumJob *jobs_dev, int njobs, int max_n, hipStre
                      s, jobs_dev);
   return ne_hip_status(hipGetLastError(), "colsum_batch");
 }
-long qk_prep_bwd_part_elems(int T, int HD) {
-  return (long)((T + qk_tpb(T, false) - 1) / qk_tpb(T, false)) * 2 * HD;
+long qk_prep_bwd_part_elems(int T, int NH, int NKV, int HD) {
+  return (long)((T + qk_tpb(T, HD) - 1) / qk_tpb(T, HD)) * (NH + NKV) * HD;
 }
 
 int launch_rmsnorm_bwd(int dt, const float *dy, const float *x, const float *g, const float *r,
@@ -858,28 +927,40 @@ int launch_qk_prep_bwd(int dt, const float *dq, const float *dk, const h16_t *qk
                        int T, int S, int NH, int NKV, int HD, int *ovf, float *part, hipStream_t s,
                        bool defer_colsum, const float *kvpart, int *ovf_v) {
   if (HD != 64 && HD != 128) return ne_fail(NE_ERR_ARG, "qk_prep: head_dim %d not in {64,128}", HD);
-  if (kvpart && NH % NKV) return ne_fail(NE_ERR_ARG, "qk_prep: bad layout for the dK/dV partials");
-  if (T <= 0) return 0;
-  const bool atomics = gq && !part;
-  const int tpb = qk_tpb(T, atomics);
+  if (T <= 0) return ne_fail(NE_ERR_ARG, "qk_prep: T = %d", T);
+  if (kvpart && (ld % 2 || NH % NKV)) return ne_fail(NE_ERR_ARG, "qk_prep: bad layout for the dK/dV partials");
+  // The wide form: no partials, 16-byte rows, and enough tokens: without gains (no atomics to save) 192
+  // tokens of 16 + 8 heads of 128 take 3.7 us on one head a block and 2.9 on this, 2048 tokens 17.2 and
+  // 7.1, but 64 tokens 2.8 and 3.5.
+  const uintptr_t align = (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)qkv | (uintptr_t)dqkv | (uintptr_t)cosb | (uintptr_t)sinb;
+  if (!part && !kvpart && ld % 8 == 0 && !(align & 15) && (gq || T >= 192)) {
+    const int tpb = qk_tpb_wide(T, gq != nullptr);
+    return DISPATCH_H16(dt, [&] {
+      auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((T + tpb - 1) / tpb), dim3(256), 0, s, dq, dk, qkv, ld, cosb, sinb, gq, gk, rq,
+                           rk, dqkv, dgq, dgk, dg_scale, T, S, NH, NKV, tpb, ovf);
+      };
+      if (HD == 128) {
+        if (gq) go(qk_prep_bwd_wide_kernel<HT, true, 128>);
+        else go(qk_prep_bwd_wide_kernel<HT, false, 128>);
+      } else {
+        if (gq) go(qk_prep_bwd_wide_kernel<HT, true, 64>);
+        else go(qk_prep_bwd_wide_kernel<HT, false, 64>);
+      }
+      return ne_hip_status(hipGetLastError(), "qk_prep_bwd");
+    }());
+  }
+  const int tpb = qk_tpb(T, HD);
   const int nbx = (T + tpb - 1) / tpb;
+  dim3 grid(nbx, NH + NKV + (kvpart ? NKV : 0));
   NE_CHECK(DISPATCH_H16(dt, [&] {
-    auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(nbx), dim3(256), 0, s, dq, dk, qkv, ld, cosb, sinb, gq, gk, rq, rk, dqkv, dgq,
-                         dgk, dg_scale, T, S, NH, NKV, tpb, ovf, part, kvpart, ovf_v);
-    };
-    if (HD == 128) {
-      if (gq) go(qk_prep_bwd_kernel<HT, true, 128>);
-      else go(qk_prep_bwd_kernel<HT, false, 128>);
-    } else {
-      if (gq) go(qk_prep_bwd_kernel<HT, true, 64>);
-      else go(qk_prep_bwd_kernel<HT, false, 64>);
-    }
+    if (gq) hipLaunchKernelGGL((qk_prep_bwd_kernel<HT, true>), grid, dim3(256), 0, s, dq, dk, qkv, ld, cosb, sinb, gq, gk, rq, rk, dqkv, dgq, dgk, dg_scale, T, S, NH, NKV, HD, tpb, ovf, part, kvpart, ovf_v);
+    else hipLaunchKernelGGL((qk_prep_bwd_kernel<HT, false>), grid, dim3(256), 0, s, dq, dk, qkv, ld, cosb, sinb, gq, gk, rq, rk, dqkv, dgq, dgk, dg_scale, T, S, NH, NKV, HD, tpb, ovf, part, kvpart, ovf_v);
     return ne_hip_status(hipGetLastError(), "qk_prep_bwd");
   }()));
   if (gq && part && !defer_colsum) {
     hipLaunchKernelGGL(colsum_kernel, dim3((HD + CS_COLS - 1) / CS_COLS, 2), dim3(CS_COLS * CS_GROUPS), 0, s, part,
-                       nbx, dgq, part + (long)nbx * HD, nbx, dgk, HD);
+                       NH * nbx, dgq, part + (long)NH * nbx * HD, NKV * nbx, dgk, HD);
     NE_HIP(hipGetLastError());
   }
   return 0;

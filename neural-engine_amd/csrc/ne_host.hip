@@ -508,7 +508,7 @@ extern "C" ne_ctx *ne_create(const ne_config *cfg) {
   // gain-gradient partials of every norm site (2L+1 RMSNorms, L QK-norm pairs), summed by one
   // ordered launch at the end of the backward
   c->rms_slab = rmsnorm_bwd_part_elems(c->T, c->D);
-  c->qk_slab = c->c.qk_norm ? qk_prep_bwd_part_elems(c->T, c->HD) : 0;
+  c->qk_slab = c->c.qk_norm ? qk_prep_bwd_part_elems(c->T, c->NH, c->NKV, c->HD) : 0;
   pl.add(&c->gpart, (size_t)(2 * c->L + 1) * c->rms_slab + (size_t)c->L * c->qk_slab);
   c->cs_njobs = 2 * c->L + 1 + (c->c.qk_norm ? 2 * c->L : 0);
   pl.add(&c->cs_jobs, (size_t)c->cs_njobs);
@@ -540,7 +540,7 @@ extern "C" ne_ctx *ne_create(const ne_config *cfg) {
     }
     if (c->c.qk_norm) {
       int rq, rk;
-      qk_prep_bwd_part_rows(c->T, &rq, &rk);
+      qk_prep_bwd_part_rows(c->T, c->NH, c->NKV, c->HD, &rq, &rk);
       for (int l = 0; l < c->L; l++) {
         jobs.push_back({qk_part(c, l), c->G + c->lo[l].gq, rq, c->HD});
         jobs.push_back({qk_part(c, l) + (long)rq * c->HD, c->G + c->lo[l].gk, rk, c->HD});

@@ -139,7 +139,7 @@ int launch_rmsnorm_fwd(int dt, const float *x, const float *g, h16_t *y, float *
 // Gain gradients: with `part` (scratch of *_part_elems floats) per-block partials are summed
 // in a second, ordered pass (deterministic); without it blocks add atomically.
 long rmsnorm_bwd_part_elems(int T, int D);
-long qk_prep_bwd_part_elems(int T, int HD);
+long qk_prep_bwd_part_elems(int T, int NH, int NKV, int HD);
 // With sp.n > 0, dy is formed from split-K partials (SplitIn) instead of read.  With
 // defer_colsum the partials are left for one colsum_batch launch (ColsumJob) later.  With
 // ref_formula dx follows the reference's formula (gain factor on the projection term too).
@@ -155,7 +155,7 @@ struct ColsumJob {
   int rows, n;
 };
 int rmsnorm_bwd_part_rows(int T);                              // partial rows of one rmsnorm_bwd
-void qk_prep_bwd_part_rows(int T, int *rows_q, int *rows_k);
+void qk_prep_bwd_part_rows(int T, int NH, int NKV, int HD, int *rows_q, int *rows_k);
 int launch_colsum_batch(const ColsumJob *jobs_dev, int njobs, int max_n, hipStream_t s);
 // With sp.n > 0 the 16-bit input (h13 / qkv, the GEMM's output) is formed from split-K
 // partials and written before use; ovf_h13 / ovf_qkv take the GEMM's overflow flag.

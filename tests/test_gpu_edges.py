@@ -80,6 +80,62 @@ def test_qk_prep_bwd_edges(fmt, T, S, NH, NKV, HD, pad, qk):
         assert rel_l2(host(dgq), 1 + 2 * dgqr) < 1e-4 and rel_l2(host(dgk), 1 + 2 * dgkr) < 1e-4
 
 
+# The sums behind dqkv have one order, whichever form runs (16-byte rows: the wide one; a pitch or a base that
+# is not: one head a block, which the training step uses too): a head's products by pairs, the pairs in a
+# butterfly of strides 1, 2, 4 ..., fused multiply-adds where written here.  Restated in numpy (a float64
+# product of two float32 values is exact), so every element has the same bits; the two forms' borders
+# (191 / 192 tokens without gains), one token, and an empty last pass.
+@pytest.mark.parametrize("fmt", ["fp16", "bf16"])
+@pytest.mark.parametrize("T,NH,NKV,HD,qk", [(512, 16, 8, 128, True), (1, 16, 8, 128, True), (512, 10, 5, 64, True),
+                                            (191, 12, 12, 64, False), (192, 12, 12, 64, False), (1025, 16, 8, 128, False)])
+def test_qk_prep_bwd_bits(fmt, T, NH, NKV, HD, qk):
+    dt, tdt, rnd, _ = FMT[fmt]
+    f32 = np.float32
+    Q, KV, N = NH * HD, NKV * HD, NH + NKV
+    rng = np.random.default_rng(T + HD)
+    qkv = rnd(rng.standard_normal((T, Q + 2 * KV)).astype(f32))
+    gq, gk = ((1 + 0.3 * rng.standard_normal(HD)).astype(f32) for _ in range(2))
+    rq, rk = (rng.uniform(0.5, 2, (T, n)).astype(f32) for n in (NH, NKV))
+    cos, sin = (t.astype(f32) for t in om.rope_tables(T, HD, 1e4))
+    dq, dk = rng.standard_normal((T, Q)).astype(f32), rng.standard_normal((T, KV)).astype(f32)
+
+    def fma64(a, b, c):
+        return a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)
+
+    y = np.concatenate([dq, dk], 1).reshape(T, N, HD // 2, 2)
+    c, s = cos[:, None], sin[:, None]
+    rot = np.stack([fma64(y[..., 0], c, y[..., 1] * s), fma64(y[..., 1], c, -(y[..., 0] * s))], -1)
+    if qk:
+        d, x = rot.astype(f32), qkv[:, :Q + KV].reshape(T, N, HD // 2, 2)
+        g = np.concatenate([np.tile(gq, (NH, 1)), np.tile(gk, (NKV, 1))]).reshape(N, HD // 2, 2)
+        r = np.concatenate([rq, rk], 1)[..., None]
+        dx = d * x
+        dot = fma64(dx[..., 0], g[..., 0], dx[..., 1] * g[..., 1]).astype(f32)
+        while dot.shape[-1] > 1:
+            dot = dot[..., 0::2] + dot[..., 1::2]
+        cc = (r * r * r * dot / f32(HD))[..., None]
+        ref = rnd(fma64(r[..., None] * g, d, -(x * cc)).astype(f32))
+    else:  # fp16: the rotation is rounded once
+        ref = rot.astype(np.float16).astype(f32) if fmt == "fp16" else rnd(rot.astype(f32))
+    ref = ref.reshape(T, Q + KV)
+    P = lambda a: ptr(dev(a)) if qk else None  # noqa: E731
+    for pitch, base in ((0, 0), (8, 0), (2, 0), (8, 2)):  # elements beyond a row; of the arrays' start
+        ld = Q + 2 * KV + pitch
+        buf, out = zeros(T * ld + base, tdt), zeros(T * ld + base, tdt)
+        buf[base:].view(T, ld)[:, :Q + 2 * KV] = dev(qkv, tdt)
+        dgq, dgk = (dev(np.ones(HD, f32)) for _ in range(2))
+        call(L.ne_k_qk_prep_bwd, dt, ptr(dev(dq)), ptr(dev(dk)), ptr(buf[base:]), ld, ptr(dev(cos)), ptr(dev(sin)),
+             P(gq), P(gk), P(rq), P(rk), ptr(out[base:]), ptr(dgq) if qk else None, ptr(dgk) if qk else None, 2.0, T, T,
+             NH, NKV, HD, None)
+        got = host(out)[base:].reshape(T, ld)
+        assert np.array_equal(got[:, :Q + KV], ref), (pitch, base, int((got[:, :Q + KV] != ref).sum()))
+        assert not got[:, Q + KV:].any()
+        if qk:
+            a = dx.astype(np.float64) * r[..., None]
+            for got_g, h in ((dgq, slice(0, NH)), (dgk, slice(NH, N))):
+                assert rel_l2(host(got_g), 1 + 2 * a[:, h].sum((0, 1)).reshape(HD)) < 1e-4
+
+
 # Sampling runs a row of logits in chunks of at least 1024 columns: one chunk, two, a last chunk shorter
 # than the others; peaked (gain 8) and flat (gain 1) distributions, with and without the top-p mask.
 # A pick may differ from the oracle's only where its uniform lies within 1e-5 of the boundary between

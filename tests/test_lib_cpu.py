@@ -55,6 +55,14 @@ def test_kernel_entry_points_validate_shapes_before_launch():
     assert rc == -1
 
 
+def test_qk_prep_bwd_refuses_no_tokens():
+    L = ne.lib()
+    for T in (0, -3):
+        rc = L.ne_k_qk_prep_bwd(1, None, None, None, 64, None, None, None, None, None, None, None, None, None, 1.0,
+                                T, 64, 2, 1, 64, None)
+        assert rc == -1 and b"T =" in L.ne_last_error()
+
+
 def test_swiglu_forward_epilogue_arguments_checked_on_host():
     """The W1|W3 GEMM's SwiGLU-forward epilogue (epi 7) needs both outputs and layout 0; the
     checks run before any launch."""
