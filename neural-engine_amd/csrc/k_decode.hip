@@ -1202,13 +1202,15 @@ __global__ __launch_bounds__(SAMP_NT) void samp_pick_kernel(SampArgs a) {
   }
   __syncthreads();
   const double u = a.unif[(long)b * a.ctx + step] * (double)total;
-  // the first chunk that passes u; where rounding lets none pass, the last one that holds mass
+  // the first chunk that passes u; a uniform of 1 or more (no draw from [0, 1) rounds up to the total) takes
+  // the last one that holds mass
   if (own && (double)incl > u && !((double)(incl - own) > u)) {
     s_chunk = tid;
     s_before = incl - own;
   }
   __syncthreads();
   const bool none = s_chunk < 0;
+  __syncthreads();  // every wave has read s_chunk before one writes it again
   if (none && own && incl == total) {
     s_chunk = tid;
     s_before = incl - own;

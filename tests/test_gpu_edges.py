@@ -159,6 +159,10 @@ def test_decode_sampling_chunks(V, B, gain, top_p):
     lo = m.decode(prompt, 1, temp, 1.0, np.zeros((B, 1)))
     hi = m.decode(prompt, 1, temp, 1.0, np.full((B, 1), 1 - 2.0 ** -53))
     assert (lo == 0).all() and (hi > V - 64).all()
+    # a uniform of 1 or more lies past every token: the last one that holds mass
+    one = m.decode(prompt, 1, temp, top_p, np.full((B, 1), 1.0))
+    np.testing.assert_array_equal(one, m.decode(prompt, 1, temp, top_p, np.full((B, 1), 1 - 2.0 ** -53)))
+    np.testing.assert_array_equal(one, m.decode(prompt, 1, temp, top_p, np.full((B, 1), 7.0)))
     m.set("rms_final", np.full(cfg.dim, np.nan, np.float32))
     assert (m.decode(prompt, 2, temp, top_p, u[:, :2]) == 0).all()
     m.close()
