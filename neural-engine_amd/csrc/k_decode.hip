@@ -929,7 +929,8 @@ __global__ __launch_bounds__(256) void dec_argmax_part_kernel(const float *__res
 // threshold) a sample of 151,936 logits took 747 us at batch 1; the chain takes 34 us (seven launches of 4-6 us: latency).
 //
 // Masses are sums of fixed-point values, p * 2^62 as an integer (p <= 1; exact for p >= 2^-38,
-// smaller ones lose less than 2^-62 each): integer sums do not depend on the order of the atomics
+// smaller ones are off by less than 2^-62 each, and every p above 0 counts at least one unit, so that
+// a uniform of 0 picks the first of them): integer sums do not depend on the order of the atomics
 // that form them, so the same logits and uniform always give the same token.
 
 struct SampArgs {
@@ -954,7 +955,9 @@ constexpr double SAMP_ONE = 4611686018427387904.0;  // 2^62
 constexpr uint32_t SAMP_P1 = 0x3f800000u;       // the bits of p = 1, the largest
 
 __device__ __forceinline__ unsigned long long samp_mass(float p) {
-  return p > 0.f ? (unsigned long long)((double)p * SAMP_ONE) : 0ull;  // 0 for NaN
+  if (!(p > 0.f)) return 0ull;  // also NaN
+  const unsigned long long m = (unsigned long long)((double)p * SAMP_ONE);
+  return m ? m : 1ull;
 }
 
 template <typename T>

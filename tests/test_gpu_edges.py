@@ -168,6 +168,26 @@ def test_decode_sampling_chunks(V, B, gain, top_p):
     m.close()
 
 
+# A uniform of 0 picks the first token whose probability is above 0, however small (numpy: the first index
+# with cdf > 0): logits spread so that probabilities run down to the smallest normal float32.
+@pytest.mark.parametrize("top_p", [1.0, 0.9])
+def test_decode_sampling_tiny_probabilities(top_p):
+    B, V = 4, 2112
+    cfg = om.tiny(vocab=V)
+    P = {k: om.round_bf16(v) for k, v in om.init_params(cfg, seed=3).items()}
+    P["rms_final"] = np.full_like(P["rms_final"], 60.0)
+    rng = np.random.default_rng(5)
+    prompt, u = rng.integers(0, V, (B, 4)).astype(np.int32), np.zeros((B, 1))
+    want, _, logits = om.decode(cfg, P, prompt, 1, return_logits=True)
+    first = np.exp(np.float64(logits[0][:, 0]) - np.float64(logits[0]).max(1))
+    assert ((first > 2.0 ** -110) & (first < 2.0 ** -64)).any()  # token 0, far from 1 and above 0
+    m = ne.Model.from_oracle(cfg, decode_batch=B, decode_ctx=8, dtype=ne.NE_BF16)
+    m.set_params(P)
+    got = m.decode(prompt, 1, 1.0, top_p, u)
+    np.testing.assert_array_equal(got, om.decode(cfg, P, prompt, 1, temperature=1.0, top_p=top_p, uniforms=u))
+    m.close()
+
+
 # The prompt before its last position runs in chunks of up to 256 rows (sequence x position): rows below 16
 # and 32 and at several 32s, chunk borders, the last chunk with one position, batches of both K-cache
 # layouts, and the one or two positions that a small batch takes one at a time.  Picks as in
