@@ -102,11 +102,13 @@ int ne_get_tensor(ne_ctx *ctx, int kind, int tensor_id, float *host, size_t n);
  * residual / RoPE / GQA ops, cross_entropy_loss (TD/cpu_ops.h:348-382), the dW sgemms and
  * embed_backward. */
 int ne_train_step(ne_ctx *ctx, const int32_t *tokens, float loss_scale, float *loss_out);
-/* Replay the step, and each position of ne_decode, from captured HIP graphs (default on;
- * the step's graph is used only while ne_overlap_weight_grads is off and per-kernel
- * profiling is disabled: the two-stream step runs faster from eager launches).  The step's graph is
- * captured on first use per (fresh accumulation, loss_scale, internal gradient scale), the
- * decode graphs per (batch size; greedy, sampling, sampling with top-p); they replace the reference's
+/* Replay the step, and each position of ne_decode that does not run in a prompt chunk, from
+ * captured HIP graphs (default on; the step's graph is used only while ne_overlap_weight_grads
+ * is off and per-kernel profiling is disabled: the two-stream step runs faster from eager
+ * launches).  Chunks launch eagerly: the positions before a prompt's last, from 3 of them on
+ * at batch <= 4 and from 2 on above.  The step's graph is captured on first use per (fresh
+ * accumulation, loss_scale, internal gradient scale), the decode graphs per (batch size;
+ * prompt position, greedy, sampling, sampling with top-p); they replace the reference's
  * per-kernel ANE dispatch (TD/io.h:190-229).  Off: every kernel is launched eagerly. */
 int ne_use_graphs(ne_ctx *ctx, int on);
 /* Run the step's weight-gradient GEMMs (and the embedding gradient of the classifier) on a

@@ -7,9 +7,10 @@
 // the KV cache and all accumulation are fp32.
 //
 // Every kernel reads the position from device memory (DecState), so the launch sequence of
-// one generated position does not depend on it: it is captured once as a HIP graph and replayed
-// per position.  The prompt's positions before the last run in chunks of up to 256 rows (sequence x
-// position) through the batch 5..32 GEMVs (enqueue_prompt).
+// one position does not depend on it: it is captured once as a HIP graph (one for prompt
+// positions, one for generated ones) and replayed per position.  A longer prompt's positions before
+// the last run in chunks of up to 256 rows (sequence x position) through the batch 5..32 GEMVs
+// (enqueue_prompt).
 //
 // GEMVs are HBM-bound (each weight byte is read once per position whatever the batch):
 //  * batch <= 4: VALU kernel.  The block stages its input rows in LDS (fusing the RMSNorm or
@@ -33,8 +34,9 @@ struct DecState {
   float top_p;
 };
 
-// How a position's token is chosen: the first maximum, or sampled without or with a top-p mask.
-enum { PICK_GREEDY = 0, PICK_SAMPLE = 1, PICK_TOPP = 2 };
+// How a position's token is chosen: not at all (a prompt position before the last), the first maximum, or
+// sampled without or with a top-p mask.
+enum { PICK_NONE = -1, PICK_GREEDY = 0, PICK_SAMPLE = 1, PICK_TOPP = 2 };
 
 constexpr int VB = 4;            // largest batch of the VALU GEMV path
 constexpr int PROMPT_ROWS = 256; // most rows of a prompt chunk
@@ -67,7 +69,7 @@ struct Dec {
   float *cosb, *sinb;     // [ctx, HD/2]
   DecState *st;
   void *arena;
-  struct Graph { int B, mode; hipGraphExec_t gen; };  // mode: PICK_*
+  struct Graph { int B, mode; hipGraphExec_t exec; };  // mode: PICK_*
   std::vector<Graph> graphs;
 };
 
@@ -1612,11 +1614,11 @@ int enqueue_prompt(ne_ctx *c, int B, int n_pos) {
   return 0;
 }
 
-// Enqueue the kernels of one position for B sequences.  gen: also the final norm, LM head
-// and token choice.  Position-independent (everything position-dependent is read from
+// Enqueue the kernels of one position for B sequences, with the final norm, LM head and token choice
+// unless mode is PICK_NONE.  Position-independent (everything position-dependent is read from
 // d->st), so it can be captured once and replayed.
-int enqueue_position(ne_ctx *c, int B, bool gen, int mode) {
-  const bool greedy = mode == PICK_GREEDY;
+int enqueue_position(ne_ctx *c, int B, int mode) {
+  const bool gen = mode != PICK_NONE, greedy = mode == PICK_GREEDY;
   Dec *d = (Dec *)c->dec;
   const int D = c->D, H = c->H, Q = c->Q, NKV = c->NKV, HD = c->HD, QKV = c->QKV, V = c->V;
   const float eps = c->c.norm_eps, alpha = c->c.res_alpha;
@@ -1682,7 +1684,7 @@ int enqueue_position(ne_ctx *c, int B, bool gen, int mode) {
 int capture(ne_ctx *c, int B, int mode, hipGraphExec_t *exec) {
   hipGraph_t graph = nullptr;
   NE_HIP(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
-  const int rc = enqueue_position(c, B, true, mode);
+  const int rc = enqueue_position(c, B, mode);
   const hipError_t ec = hipStreamEndCapture(c->st, &graph);
   if (rc) {
     if (graph) (void)hipGraphDestroy(graph);
@@ -1771,7 +1773,7 @@ void decode_free(ne_ctx *c) {
   Dec *d = (Dec *)c->dec;
   if (!d) return;
   for (auto &g : d->graphs) {
-    if (g.gen) hipGraphExecDestroy(g.gen);
+    if (g.exec) hipGraphExecDestroy(g.exec);
   }
   if (d->arena) hipFree(d->arena);
   delete d;
@@ -1779,7 +1781,7 @@ void decode_free(ne_ctx *c) {
 }
 
 namespace {
-int replay(ne_ctx *c, int B, int n_new, int mode);
+int positions(ne_ctx *c, int B, int n, int mode);
 }
 
 int decode_run(ne_ctx *c, const int32_t *prompt, int B, int P, int n_new, float temp, float top_p,
@@ -1817,12 +1819,8 @@ int decode_run(ne_ctx *c, const int32_t *prompt, int B, int P, int n_new, float 
   NE_HIP(hipStreamSynchronize(c->st));  // host staging vectors are released at return
 
   if (by_chunk) NE_CHECK(enqueue_prompt(c, B, P - 1));
-  else for (int pos = 0; pos < P - 1; pos++) NE_CHECK(enqueue_position(c, B, false, mode));
-  if (!c->use_graphs) {  // eager launches (tracers that do not follow graph launches)
-    for (int j = 0; j < n_new; j++) NE_CHECK(enqueue_position(c, B, true, mode));
-  } else {
-    NE_CHECK(replay(c, B, n_new, mode));
-  }
+  else NE_CHECK(positions(c, B, P - 1, PICK_NONE));
+  NE_CHECK(positions(c, B, n_new, mode));
   std::vector<int32_t> o((size_t)d->Bp * d->ctx);
   NE_HIP(hipMemcpyAsync(o.data(), d->out, o.size() * 4, hipMemcpyDeviceToHost, c->st));
   NE_HIP(hipStreamSynchronize(c->st));
@@ -1833,19 +1831,27 @@ int decode_run(ne_ctx *c, const int32_t *prompt, int B, int P, int n_new, float 
 
 namespace {
 
-// Replay the captured graph of a generated position (captured on first use per batch size and mode).
-int replay(ne_ctx *c, int B, int n_new, int mode) {
+// The next n positions: the captured graph of one (captured on first use per batch size and mode) replayed
+// n times, or eager launches where graphs are off (tracers that do not follow graph launches).  The one or
+// two prompt positions of a short prompt replay theirs too: eagerly their 140 launches each took longer than
+// their kernels (batch 1, Qwen3-0.6B, a prompt of 3 tokens and 1 new: 1.75 ms replayed, 1.81-1.88 eager).
+int positions(ne_ctx *c, int B, int n, int mode) {
   Dec *d = (Dec *)c->dec;
+  if (!c->use_graphs) {
+    for (int j = 0; j < n; j++) NE_CHECK(enqueue_position(c, B, mode));
+    return 0;
+  }
+  if (n <= 0) return 0;
   Dec::Graph *gr = nullptr;
   for (auto &g : d->graphs)
     if (g.B == B && g.mode == mode) gr = &g;
   if (!gr) {
     Dec::Graph g = {B, mode, nullptr};
-    NE_CHECK(capture(c, B, mode, &g.gen));
+    NE_CHECK(capture(c, B, mode, &g.exec));
     d->graphs.push_back(g);
     gr = &d->graphs.back();
   }
-  for (int j = 0; j < n_new; j++) NE_HIP(hipGraphLaunch(gr->gen, c->st));
+  for (int j = 0; j < n; j++) NE_HIP(hipGraphLaunch(gr->exec, c->st));
   return 0;
 }
 

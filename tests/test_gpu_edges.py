@@ -192,7 +192,7 @@ def test_decode_sampling_tiny_probabilities(top_p):
 # and 32 and at several 32s, chunk borders, the last chunk with one position, batches of both K-cache
 # layouts, and the one or two positions that a small batch takes one at a time.  Picks as in
 # test_decode_sampling_chunks.
-@pytest.mark.parametrize("B,P,fmt,kw", [(1, 2, "bf16", {}), (1, 4, "fp16", {}), (2, 40, "bf16", dict(qk_norm=True)),
+@pytest.mark.parametrize("B,P,fmt,kw", [(1, 2, "bf16", {}), (1, 3, "bf16", {}), (1, 4, "fp16", {}), (2, 40, "bf16", dict(qk_norm=True)),
                                         (3, 87, "fp16", dict(head_dim=128, qk_norm=True)), (4, 66, "bf16", {}),
                                         (5, 53, "bf16", dict(head_dim=128, n_heads=2, qk_norm=True)),
                                         (5, 2, "fp16", {}), (17, 17, "fp16", dict(n_heads=8)),
