@@ -358,12 +358,13 @@ __global__ __launch_bounds__(RG * RMS_NT) void rmsnorm_bwd_kernel(
 }
 
 // out[j] += sum_r part[r * n + j] for r in [0, rows): the deterministic second pass of the
-// per-block gain-gradient partials.  Block = 64 columns x 16 row groups; row group g sums
+// per-block gain-gradient partials.  Block = 16 columns x 16 row groups; row group g sums
 // rows g, g+16, ... in order, then the 16 group sums are added in group order, so the
 // result does not depend on scheduling.  grid.y selects one of two (part, rows, out) sets.  A group has
-// CS_DEPTH rows in flight: many tokens leave many QK-norm rows (3264 tokens of 16 heads of 128: 13,056), and
-// the sum is one chain (with 4 in flight a step of 3264 tokens and two layers took 2316 us, now 2217).
-constexpr int CS_COLS = 64, CS_GROUPS = 16, CS_DEPTH = 16;
+// CS_DEPTH rows in flight, and blocks are narrow: the sum is one chain a column, and QK-norm sites leave many
+// rows of few columns (3264 tokens of 16 heads of 128: 13,056 of 128).  A step of 1024 tokens and two layers:
+// 37.4 us with 4 rows in flight and 64 columns a block, 24.8 with 32 rows, 21.8 with 16 columns as well.
+constexpr int CS_COLS = 16, CS_GROUPS = 16, CS_DEPTH = 32;
 __global__ __launch_bounds__(CS_COLS * CS_GROUPS) void colsum_kernel(const float *__restrict__ part0, int rows0,
                                                                      float *__restrict__ out0,
                                                                      const float *__restrict__ part1, int rows1,
@@ -376,15 +377,14 @@ __global__ __launch_bounds__(CS_COLS * CS_GROUPS) void colsum_kernel(const float
   const int j = blockIdx.x * CS_COLS + c;
   float s = 0.f;
   if (j < n) {
-    int r = grp;
-    for (; r + (CS_DEPTH - 1) * CS_GROUPS < rows; r += CS_DEPTH * CS_GROUPS) {
+    for (int r = grp; r < rows; r += CS_DEPTH * CS_GROUPS) {
       float v[CS_DEPTH];
 #pragma unroll
-      for (int i = 0; i < CS_DEPTH; i++) v[i] = part[(long)(r + i * CS_GROUPS) * n + j];
+      for (int i = 0; i < CS_DEPTH; i++) v[i] = r + i * CS_GROUPS < rows ? part[(long)(r + i * CS_GROUPS) * n + j] : 0.f;
 #pragma unroll
-      for (int i = 0; i < CS_DEPTH; i++) s += v[i];
+      for (int i = 0; i < CS_DEPTH; i++)
+        if (r + i * CS_GROUPS < rows) s += v[i];
     }
-    for (; r < rows; r += CS_GROUPS) s += part[(long)r * n + j];
   }
   red[grp][c] = s;
   __syncthreads();
@@ -407,15 +407,14 @@ __global__ __launch_bounds__(CS_COLS * CS_GROUPS) void colsum_batch_kernel(const
   if (blockIdx.x * CS_COLS >= n) return;  // uniform: this job has fewer columns
   float s = 0.f;
   if (j < n) {
-    int r = grp;
-    for (; r + (CS_DEPTH - 1) * CS_GROUPS < rows; r += CS_DEPTH * CS_GROUPS) {
+    for (int r = grp; r < rows; r += CS_DEPTH * CS_GROUPS) {
       float v[CS_DEPTH];
 #pragma unroll
-      for (int i = 0; i < CS_DEPTH; i++) v[i] = part[(long)(r + i * CS_GROUPS) * n + j];
+      for (int i = 0; i < CS_DEPTH; i++) v[i] = r + i * CS_GROUPS < rows ? part[(long)(r + i * CS_GROUPS) * n + j] : 0.f;
 #pragma unroll
-      for (int i = 0; i < CS_DEPTH; i++) s += v[i];
+      for (int i = 0; i < CS_DEPTH; i++)
+        if (r + i * CS_GROUPS < rows) s += v[i];
     }
-    for (; r < rows; r += CS_GROUPS) s += part[(long)r * n + j];
   }
   red[grp][c] = s;
   __syncthreads();
