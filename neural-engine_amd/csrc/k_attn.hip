@@ -690,7 +690,7 @@ int check(const AttnArgs &a) {
 
 // Block shape (waves NW, 16-row groups per wave RG) by the work-group count it gives.
 // Two row groups per wave halve the LDS reads per MFMA and double the accumulators: the
-// forward and the dQ blocks still fit two waves per SIMD with them (used for long sequences);
+// forward and the dQ blocks still fit two waves per SIMD with them (two_query_groups);
 // the dK/dV blocks would drop to one, which costs more than the LDS traffic saves, so they
 // keep one group.  4 waves while 64-row blocks give 256 work-groups, else 2 (short sequences
 // would leave most CUs idle).
@@ -730,10 +730,14 @@ int fwd_t(const AttnArgs &a, hipStream_t s) {
 // side: at short sequences each alone leaves half the CUs idle.
 // RGQ: 16-query groups per wave of the dQ blocks (the dK / dV blocks have one of 16 keys).  HG: head
 // groups of the dK / dV blocks, NW waves each; the dQ blocks have HG * NW waves.
+// bf16 heads of 64 on 4 waves keep three waves per SIMD (168 VGPRs): left to itself the compiler took 172
+// for the wider dQ blocks and two waves (batch 4 x 1024, 10 / 5 heads: 73 us on blocks of 64 queries, 84 at
+// two waves, 75 at three, with 36 bytes of spills).  fp16 takes two: at three, with more blocks beside each
+// other on a CU, a launch of one round is slower (12 heads, 1 x 2048: 58 us at two, 68 at three).
 template <typename HT, int HD, int NW, int RGQ, bool SPLIT, int HG>
-__global__ __launch_bounds__(HG * NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void attn_bwd_kernel(AttnArgs a,
-                                                                                                        int nkv,
-                                                                                                        int nky) {
+__global__ __launch_bounds__(HG * NW * 64)
+    __attribute__((amdgpu_waves_per_eu(HD == 64 && NW == 4 && HT::id == H16B::id ? 3 : 2))) void attn_bwd_kernel(
+        AttnArgs a, int nkv, int nky) {
   __shared__ __attribute__((aligned(16))) h16_t lds[HG][2][2 * BLK * (HD + 16)];
   __shared__ __attribute__((aligned(16))) float lse_s[HG][2][BLK], ndl_s[HG][2][BLK];
   int bx, by, bz;
@@ -765,6 +769,27 @@ int bwd_hd(const AttnArgs &a, hipStream_t s) {
   return ne_hip_status(hipGetLastError(), "attn_bwd");
 }
 
+// dQ blocks of 128 queries (two groups a wave) instead of 64: half the LDS reads, but half the blocks, so
+// that a launch of few rounds ends with a nearly empty one.  From the time of both at batch 1 to 8 x 192 to
+// 2048, 8 to 16 heads, fp16 and bf16 (us, 64 -> 128 queries a block):
+//  * at least one such block a CU (256);
+//  * heads of 128: not below 448 tokens (320 with 4 query heads per KV head): 16 / 8 heads 8 x 192 24.3 -> 26.7,
+//    8 x 320 41 -> 45, but 8 x 448 60 -> 57, 3 x 1088 147 -> 137, 8 x 2048 659 -> 594; without GQA the dK / dV
+//    blocks are as many as the dQ blocks and it takes 512: 8 / 8 heads 2 x 2048 106 -> 110, 8 x 1024 117 -> 112.
+//    With 4 query heads per KV head the longer dK / dV blocks decide and it goes either way by size: 16 / 4 heads
+//    8 x 448 70 -> 78, 8 x 512 90 -> 83;
+//  * heads of 64: fp16 12 heads 8 x 2048 297 -> 278.  In bf16 the wider block spills a few registers at three
+//    waves per SIMD: not without GQA (12 heads 4 x 1344 78 -> 87), otherwise up to 512 blocks (10 / 5 heads
+//    3 x 1088 79 -> 61, 16 / 4 heads 4 x 1024 137 -> 115; 10 / 5 heads 8 x 1024, 640 blocks, 78 -> 84).
+template <typename HT, int HD>
+bool two_query_groups(const AttnArgs &a) {
+  const long blocks = (long)((a.S + 127) / 128) * a.NH * a.B;
+  const int ratio = a.NH / a.NKV;
+  if (HD == 128) return a.S >= (ratio >= 4 ? 320 : 448) && blocks >= (ratio == 1 ? 512 : 256);
+  if (HT::id == H16F::id) return blocks >= 256;
+  return ratio > 1 && blocks >= 256 && blocks <= 512;
+}
+
 template <typename HT, int HD>
 int bwd_shape(const AttnArgs &a, hipStream_t s) {
   if (pick_shape(a) == SHAPE_2x1) {
@@ -775,10 +800,7 @@ int bwd_shape(const AttnArgs &a, hipStream_t s) {
     if (!a.part && a.NH / a.NKV % 2 == 0 && blocks <= 256) return bwd_hd<HT, HD, 2, 1, 2>(a, s);
     return bwd_hd<HT, HD, 2, 1>(a, s);
   }
-  // dQ blocks of 128 queries (two groups a wave) while there is one a CU: batch 3 x 1088 (432 of
-  // them) 151 -> 142 us, batch 8 x 2048 815 -> 671
-  const long dq128 = (long)((a.S + 127) / 128) * a.NH * a.B;
-  return dq128 >= 256 ? bwd_hd<HT, HD, 4, 2>(a, s) : bwd_hd<HT, HD, 4, 1>(a, s);
+  return two_query_groups<HT, HD>(a) ? bwd_hd<HT, HD, 4, 2>(a, s) : bwd_hd<HT, HD, 4, 1>(a, s);
 }
 
 template <typename HT>
