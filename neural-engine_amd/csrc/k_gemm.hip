@@ -886,36 +886,57 @@ int gemm_tile(int M, int N, int K) {
 }
 
 // Block tile of a shape without a split-K workspace (the kernel-level entry points), from the
-// time of every tile at some 70 shapes of 64 to 4096 rows (fp16, MI355X; us, the tile that the
-// workspace form's rule gives -> this one's).  mn: an operand is M/N-contiguous.  Tile counts
-// round up: a ragged last tile overlaps the one before it (RAG of gemm_body).
+// time of every tile at some 700 products of 64 to 16,384 rows, fp16 and bf16 (MI355X; us, the tile that
+// the workspace form's rule gives -> this one's, or the two sides of a line).  mn: an operand is
+// M/N-contiguous; reads: the epilogue reads an M x N operand.  Tile counts round up: a ragged last tile
+// overlaps the one before it (RAG of gemm_body).
 //  * The 256-row tiles, of whole multiples, while they leave at most a quarter of the CUs idle:
 //    6144x1024x2048 (TN) 47.9 -> 38.1 (the SwiGLU backward's staged epilogue wants more than
 //    one work-group a CU: 2048x3072x1024, 192 tiles, 34.2 on this one, 30.9 on 128x128).
 //  * 128x128 on 8 waves (two work-groups of 4 waves a CU hide no more, and below 256 tiles a CU
-//    has one; above 256 the 4-wave form): 4096x1024x151936 (NN) 1760 -> 1626, 3264x1024x4096 (NN) 96.3 -> 42.3, 3264x4096x1024 79.6 -> 41.5.
+//    has one): 4096x1024x151936 (NN) 1760 -> 1626, 3264x1024x4096 (NN) 96.3 -> 42.3, 3264x4096x1024 79.6 ->
+//    41.5.  Whole tiles keep the 4-wave form above 256, and below with an M/N-contiguous operand and a plain
+//    output, but for long K loops of NN (8 waves and 4: 768x4096x1024 (NN) 14.1 and 12.9, 4096x1024x3264 (TN)
+//    38.8 and 36.0).  Ragged, 8 waves pay where their rounds are full: just above one tile a CU a second
+//    round is nearly empty (3392x1280x832 16.6 -> 19.6, 64x64 again up to 320 tiles; longer K loops gain all
+//    the same), as just above two of a residual (9856x832x1728 52.7 -> 58.6, 48.1 on 128x64).
+//  * An epilogue that reads is exposed where a CU has one large tile and hidden where it has three small
+//    ones: up to 768 64x64 tiles those, unless K is long (768x4096x1024 + residual 22.6 and 19.6,
+//    1600x1728x832 SwiGLU backward 17.2 and 14.5, 3264x1024x4096 + residual, 816 tiles, 45 and 55).
 //  * Fewer tiles than that: 128x64 while it is one a CU (2048x1024x6144 (NN) 54.8 -> 45.6,
-//    1024x2048x3264 (TN) 35.1 -> 28.4), else 64x64 if it is two (2496x832x3456 (NN) 40.2 -> 28.6).
+//    1024x2048x3264 (TN) 35.1 -> 28.4) and K is not a handful of steps (768x2048x192 (TN) 6.1 and 5.7), else
+//    64x64 if it is two (2496x832x3456 (NN) 40.2 -> 28.6).
 //  * One 64x64 tile a CU or less: the K range over a block's waves, in smaller tiles as they get
 //    fewer (kwave; 256x768x2048 9.5 -> 5.6, 256x1024x6144 (NN) 30.6 -> 16.4, 384x1024x4096 (NN)
-//    21.7 -> 13.7, 1024x1024x6144 (NN) 32.9 -> 26.6), except where the K loop is short (or, at 129
-//    and more tiles, both operands are K-contiguous: 1024x1024x2048 10.3, 12.0 with it), and
+//    21.7 -> 13.7, 1024x1024x6144 (NN) 32.9 -> 26.6; 32x32 while that is one a CU, 384x768x2048 (NN) 11.2 on
+//    288 of them and 8.6 on 64x32), except where the K loop is short (or, at 129
+//    and more tiles, both operands are K-contiguous: 1024x1024x2048 10.3, 12.0 with it; or the epilogue
+//    reads four values an output and writes two: 768x1024x2048 SwiGLU backward 18.0 with it, 15.1 without,
+//    768x1024x6144 31.7 and 33.4), and
 //    except for 16-bit outputs of the forward layout: EPI_SWIGLU_FWD promises their bits, and it
 //    sums K in one chain.
 int gemm_tile_nows(int layout, int epi, int M, int N, int K) {
-  const bool mn = layout != GEMM_NT;
+  const bool mn = layout != GEMM_NT, reads = epi == EPI_RESID || epi == EPI_SWIGLU_BWD;
+  const bool whole = M % 128 == 0 && N % 128 == 0;
   auto tiles = [&](int bm, int bn) { return M < bm || N < bn ? 0L : (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   const long t128 = tiles(128, 128), t128x64 = tiles(128, 64), t64 = tiles(64, 64);
   if (M % 256 == 0 && N % 256 == 0 && tiles(256, 256) >= 192) return TILE_256;
   if (M % 256 == 0 && N % 128 == 0 && tiles(256, 128) >= (epi == EPI_SWIGLU_BWD ? 256 : 192)) return TILE_256x128;
-  if (t128 >= 176) return t128 > 256 && M % 128 == 0 && N % 128 == 0 ? TILE_128 : TILE_128W8;
+  if (reads && t64 > 512 && t64 <= 768 && K <= 3072) return TILE_64;
+  if (!whole && t128 > 256 && t128 <= 320 && K <= 1536) return TILE_64;
+  if (!whole && epi == EPI_RESID && t128 > 512 && t128 <= 640) return TILE_128x64;
+  if (t128 >= 176) {
+    const bool four = mn && !reads && (epi == EPI_H16 || layout != GEMM_NN || K <= 1024);
+    return whole && (t128 > 256 || four) ? TILE_128 : TILE_128W8;
+  }
   if (t64 > 256) {
-    if (t128x64 >= 128 && t128x64 <= 256) return TILE_128x64;
+    if (t128x64 >= 128 && t128x64 <= 256) return K >= 384 || reads ? TILE_128x64 : TILE_64;
     return t128 >= 128 && t64 > 512 ? TILE_128W8 : TILE_64;
   }
   if (!mn && epi == EPI_H16) return TILE_64;
-  if (t64 > 128) return mn && K >= 2048 ? KWAVE_64 : TILE_64;
+  if (t64 > 128) return mn && (epi == EPI_SWIGLU_BWD ? K > 4096 : K >= 2048) ? KWAVE_64 : TILE_64;
   if (t64 > 80) return K >= 1024 ? KWAVE_64x32 : TILE_64;
+  if (t64 > 64 && (mn || K >= 1024)) return K >= 512 ? KWAVE_64x32 : TILE_64;
   return K >= 512 || t64 <= 16 ? KWAVE_32 : TILE_64;
 }
 

@@ -215,15 +215,23 @@ def test_decode_prompt_chunks(B, P, fmt, kw):
     m.close()
 
 
-# One shape per tile of the entry point's GEMM: 256x256, 256x128, 128x128 and 128x64 with a last tile that
-# overlaps the one before it (M, N odd multiples of 64), 64x64 on 64-deep steps, and the K-divided tiles of
-# 64x64, 64x32 and 32x32, with fewer K steps than waves (K = 64, 192) and an uneven share of them (K = 576,
-# 1088).  C has rows and columns of its own around it.  fp32 sums of K products: 1e-5 of the largest.
+# The entry point's GEMM at the sizes where its tile changes.  Two edges of the ragged 8-wave 128x128 tile (M, N
+# odd multiples of 64: the last tile overlaps the one before it), 64x64 on 64-deep steps, ragged 128x64 for the
+# epilogues that read, and the K-divided tiles of 64x64, 64x32 and 32x32, with fewer K steps than waves
+# (K = 64, 192) and an uneven share of them (K = 576, 1088).  Then 256x256, 256x128 (also at the SwiGLU backward's
+# 256 tiles, and below it, where that epilogue takes 128x128 on 4 waves), 128x128 on 4 waves (289 and exactly 256
+# tiles) and on 8 (143 tiles), 64x64 for 289 ragged tiles and 8 waves again with a long K, 128x64 for a ragged
+# residual of 575 tiles, 128x64 with K = 448, and the K-divided 64x32 at 80 tiles and 64x64 for the SwiGLU backward.
+# C has rows and columns of its own around it.  fp32 sums of K products: 1e-5 of the largest.
 @pytest.mark.parametrize("M,N,K", [(3136, 4160, 128), (3136, 2112, 64), (1856, 1472, 192), (1088, 1024, 64),
                                    (2496, 832, 128), (576, 1024, 2112), (384, 1024, 1088), (320, 768, 576),
-                                   (64, 64, 64), (64, 1024, 192)])
+                                   (64, 64, 64), (64, 1024, 192),
+                                   (3072, 4096, 128), (2048, 4224, 64), (2048, 3200, 64), (2176, 2176, 128),
+                                   (2048, 2048, 192), (1408, 1600, 128), (2112, 2112, 128), (2112, 2112, 2112),
+                                   (3136, 2880, 64), (1088, 1024, 448), (320, 1024, 576), (576, 1024, 4160)])
 @pytest.mark.parametrize("layout,epi,fmt", [(0, 0, "bf16"), (0, 3, "fp16"), (1, 1, "fp16"), (2, 1, "fp16"),
-                                            (2, 2, "bf16"), (2, 4, "fp16"), (3, 1, "bf16"), (3, 2, "fp16")])
+                                            (2, 2, "bf16"), (2, 4, "fp16"), (3, 1, "bf16"), (3, 2, "fp16"),
+                                            (2, 0, "fp16"), (2, 0, "bf16"), (2, 4, "bf16")])
 def test_gemm_tiles(M, N, K, layout, epi, fmt):
     dt, tdt, _, u = FMT[fmt]
     g = torch.Generator(device="cuda").manual_seed(M + N + K + layout)
