@@ -1503,7 +1503,7 @@ void attn_go(ne_ctx *c, dim3 grid, size_t sh, const float *gq, const float *gk, 
                        KCOL && !nc ? nullptr : d->att3);
   };
   if (nc > 0) go(dec_attn_kernel<HD, R, KCOL, true>);
-  else go(dec_attn_kernel<HD, R, KCOL, false>);
+  else if constexpr (!KCOL || R == 1) go(dec_attn_kernel<HD, R, KCOL, false>);  // launch_attn: one head a block
 }
 
 template <int HD, int R>

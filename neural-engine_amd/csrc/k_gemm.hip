@@ -434,13 +434,12 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const
     return;
   }
 
-  if (g.split > 1) {  // fp32 partial tile -> workspace slice kz
+  if (!RAG && g.split > 1) {  // fp32 partial tile -> workspace slice kz
     float *ws = g.ws + (long)kz * g.M * g.N;
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
       for (int j = 0; j < FN; j++) {
-        if (RAG && (m0 + wm * TM + i * 32 < m_own || n0 + wn * TN + j * 32 < n_own)) continue;
         const int col = n0 + wn * TN + j * 32 + (lane & 31);
 #pragma unroll
         for (int e = 0; e < 16; e++) {
@@ -542,12 +541,12 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &g, const int mt, const
       for (int e = 0; e < 16; e++) {
         const int row = m0 + wm * TM + i * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
         const float o = store_out<HT, EPI, SQ_INLINE>(g, row, col, acc[i][j][e] * alpha, bad);
-        if constexpr (epi_sq<EPI>() && SQ_INLINE) sq += o * o;
+        if constexpr (epi_sq<EPI>() && !RAG && SQ_INLINE) sq += o * o;
       }
     }
   }
   flag_overflow(g.ovf, bad);
-  if constexpr (epi_sq<EPI>())
+  if constexpr (epi_sq<EPI>() && !RAG)
     if (g.sq) {
       if constexpr (!SQ_INLINE) {
         asm volatile("" ::: "memory");
@@ -714,19 +713,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_kwave_kernel(GemmArgs g) {
         red[(i * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)) * RP + j * 32 + (lane & 31)] = acc[i][j][e];
   __syncthreads();
   bool bad = false;
-  float sq = 0.f;
 #pragma unroll
   for (int c = 0; c < BM * BN / (NW * 64); c++) {
     const int el = threadIdx.x + c * NW * 64, row = el / BN, col = el % BN;
     float s = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; w++) s += ((const float *)(lds + w * PER_WAVE))[row * RP + col];
-    const float o = store_out<HT, EPI>(g, m0 + row, n0 + col, s * g.alpha, bad);
-    if constexpr (epi_sq<EPI>()) sq += o * o;
+    store_out<HT, EPI>(g, m0 + row, n0 + col, s * g.alpha, bad);
   }
   flag_overflow(g.ovf, bad);
-  if constexpr (epi_sq<EPI>())
-    if (g.sq) block_sumsq_store<NW>(sq, g.sq + (long)mt * (g.N / BN) + nt);
 }
 
 // Ordered sum of the split-K partials (split 0 first) followed by the epilogue; four
@@ -778,8 +773,10 @@ int reduce_blocks(int M, int N) { return (int)std::min<long>(((long)M * N / 4 + 
 
 template <typename HT, int BM, int BN, int BK, int WM, int WN, bool AKC, bool BKC, int EPI, bool RAG = false>
 int launch_t(GemmArgs g, hipStream_t s) {
-  if (g.M < BM || g.N < BN || ((!RAG || g.sq) && (g.M % BM || g.N % BN)))
+  if (g.M < BM || g.N < BN || (!RAG && (g.M % BM || g.N % BN)))
     return ne_fail(NE_ERR_ARG, "gemm: a %dx%d tile does not fit %dx%d", BM, BN, g.M, g.N);
+  if (RAG && (g.split > 1 || g.sq))
+    return ne_fail(NE_ERR_ARG, "gemm: the tiles that may overlap have one split and no sums of squares");
   g.n_tiles = g.part_ld > 0 ? g.part_ld : g.N / BN;
   dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, g.split);
   if constexpr (EPI == EPI_CE_FWD || EPI == EPI_CE_BWD) {  // never split
@@ -815,7 +812,9 @@ constexpr int tile_bn(int t) { return t == TILE_256 ? 256 : t == TILE_64 ? 64 : 
 
 template <typename HT, int BM, int BN, int NW, int DEPTH, bool AKC, bool BKC, int EPI>
 int launch_kwave(const GemmArgs &g, hipStream_t s) {
-  if (g.M % BM || g.N % BN) return ne_fail(NE_ERR_ARG, "gemm: a %dx%d tile does not fit %dx%d", BM, BN, g.M, g.N);
+  if (g.M % BM || g.N % BN || g.split > 1 || g.sq)
+    return ne_fail(NE_ERR_ARG, "gemm: a K-divided %dx%d tile does not fit %dx%d (one split, no sums of squares)", BM, BN,
+                   g.M, g.N);
   const int blocks = (g.M / BM) * (g.N / BN);
   hipLaunchKernelGGL((gemm_kwave_kernel<HT, BM, BN, NW, DEPTH, AKC, BKC, EPI>), dim3(blocks), dim3(NW * 64), 0, s, g);
   return ne_hip_status(hipGetLastError(), "gemm (K over waves)");
