@@ -894,14 +894,19 @@ int gemm_tile(int M, int N, int K) {
 //    one work-group a CU: 2048x3072x1024, 192 tiles, 34.2 on this one, 30.9 on 128x128).
 //  * 128x128 on 8 waves (two work-groups of 4 waves a CU hide no more, and below 256 tiles a CU
 //    has one): 4096x1024x151936 (NN) 1760 -> 1626, 3264x1024x4096 (NN) 96.3 -> 42.3, 3264x4096x1024 79.6 ->
-//    41.5.  Whole tiles keep the 4-wave form above 256, and below with an M/N-contiguous operand and a plain
-//    output, but for long K loops of NN (8 waves and 4: 768x4096x1024 (NN) 14.1 and 12.9, 4096x1024x3264 (TN)
-//    38.8 and 36.0).  Ragged, 8 waves pay where their rounds are full: just above one tile a CU a second
-//    round is nearly empty (3392x1280x832 16.6 -> 19.6, 64x64 again up to 320 tiles; longer K loops gain all
-//    the same), as just above two of a residual (9856x832x1728 52.7 -> 58.6, 48.1 on 128x64).
+//    41.5.  Whole tiles keep the 4-wave form above 256, and below for 16-bit outputs of short K loops with an
+//    M/N-contiguous operand (1792x1792x512 (NN) 9.4 on 8 waves, 9.1 on 4).  With longer ones 4 waves gain up to
+//    4% on operands that the caches hold and lose 6-19% on operands from HBM (4096x1024x768 (NN) 11.6 and 11.2,
+//    from HBM 13.0 and 13.8; 1024x3072x6144 (TN) 54.6 and 56.9, from HBM 56.4 and 65.1), and accumulating they
+//    lose 30-60% (1024x3072x2048 (TN) += 35.4 and 47.6).  Ragged, 8 waves pay where their rounds are full: just
+//    above one tile a CU a second round is nearly empty (3392x1280x832 16.6 -> 19.6, 64x64 again up to 320
+//    tiles; longer K loops gain all the same), as just above two of a residual (9856x832x1728 52.7 -> 58.6,
+//    48.1 on 128x64).
 //  * An epilogue that reads is exposed where a CU has one large tile and hidden where it has three small
-//    ones: up to 768 64x64 tiles those, unless K is long (768x4096x1024 + residual 22.6 and 19.6,
-//    1600x1728x832 SwiGLU backward 17.2 and 14.5, 3264x1024x4096 + residual, 816 tiles, 45 and 55).
+//    ones: up to 768 64x64 tiles those, while K is short (+ residual 768x4096x1024 22.6 -> 19.6, 1024x3072x2048 (NN)
+//    28.4 and 29.0, from HBM 35.6 and 38.7; += 1408x1920x128 (NN) 16.5 -> 11.1, 896x3328x1536 (NN) 31.4 -> 29.9;
+//    SwiGLU backward 1600x1728x832 17.2 -> 14.5, 1024x3072x2048 25.3 and 27.1, from HBM 27.8 and 34.9), and up to
+//    1024 of a ragged NT accumulation of few K steps (2496x1536x64 17.4 -> 11.8, 1856x1856x256 19.8 -> 15.3).
 //  * Fewer tiles than that: 128x64 while it is one a CU (2048x1024x6144 (NN) 54.8 -> 45.6,
 //    1024x2048x3264 (TN) 35.1 -> 28.4) and K is not a handful of steps (768x2048x192 (TN) 6.1 and 5.7), else
 //    64x64 if it is two (2496x832x3456 (NN) 40.2 -> 28.6).
@@ -915,17 +920,18 @@ int gemm_tile(int M, int N, int K) {
 //    except for 16-bit outputs of the forward layout: EPI_SWIGLU_FWD promises their bits, and it
 //    sums K in one chain.
 int gemm_tile_nows(int layout, int epi, int M, int N, int K) {
-  const bool mn = layout != GEMM_NT, reads = epi == EPI_RESID || epi == EPI_SWIGLU_BWD;
+  const bool mn = layout != GEMM_NT, reads = epi == EPI_RESID || epi == EPI_F32_ACC || epi == EPI_SWIGLU_BWD;
   const bool whole = M % 128 == 0 && N % 128 == 0;
   auto tiles = [&](int bm, int bn) { return M < bm || N < bn ? 0L : (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   const long t128 = tiles(128, 128), t128x64 = tiles(128, 64), t64 = tiles(64, 64);
   if (M % 256 == 0 && N % 256 == 0 && tiles(256, 256) >= 192) return TILE_256;
   if (M % 256 == 0 && N % 128 == 0 && tiles(256, 128) >= (epi == EPI_SWIGLU_BWD ? 256 : 192)) return TILE_256x128;
-  if (reads && t64 > 512 && t64 <= 768 && K <= 3072) return TILE_64;
+  if (reads && t64 > 512 && t64 <= 768 && K <= (epi == EPI_SWIGLU_BWD ? 1024 : 1536)) return TILE_64;
+  if (epi == EPI_F32_ACC && !mn && !whole && t64 > 768 && t64 <= 1024 && K <= 256) return TILE_64;
   if (!whole && t128 > 256 && t128 <= 320 && K <= 1536) return TILE_64;
   if (!whole && epi == EPI_RESID && t128 > 512 && t128 <= 640) return TILE_128x64;
   if (t128 >= 176) {
-    const bool four = mn && !reads && (epi == EPI_H16 || layout != GEMM_NN || K <= 1024);
+    const bool four = mn && epi == EPI_H16 && K <= 512;
     return whole && (t128 > 256 || four) ? TILE_128 : TILE_128W8;
   }
   if (t64 > 256) {
