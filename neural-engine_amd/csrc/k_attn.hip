@@ -115,12 +115,13 @@ struct TileCopy {
 // of that order instead, so that the blocks of one (head, sequence), which read the same
 // Q / K / V / dO rows, share an L2 (with consecutive blocks on different XCDs every XCD
 // fetched every tile: the backward read 3.0 GB per layer at batch 8 x seq 2048).
+__device__ __forceinline__ int xcd_order(int pid, int n) {
+  const int x = pid % 8, q = n / 8, rem = n % 8;
+  return x * q + min(x, rem) + pid / 8;  // a bijection of [0, n)
+}
 __device__ __forceinline__ void xcd_block(int &bx, int &by, int &bz) {
   const int gx = gridDim.x, gy = gridDim.y;
-  const int n = gx * gy * gridDim.z;
-  const int pid = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-  const int x = pid % 8, q = n / 8, rem = n % 8;
-  const int u = x * q + min(x, rem) + pid / 8;  // a bijection of [0, n)
+  const int u = xcd_order(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), gx * gy * gridDim.z);
   bx = u % gx;
   by = (u / gx) % gy;
   bz = u / (gx * gy);
@@ -741,7 +742,25 @@ __global__ __launch_bounds__(HG * NW * 64)
   __shared__ __attribute__((aligned(16))) h16_t lds[HG][2][2 * BLK * (HD + 16)];
   __shared__ __attribute__((aligned(16))) float lse_s[HG][2][BLK], ndl_s[HG][2][BLK];
   int bx, by, bz;
-  xcd_block(bx, by, bz);
+  if constexpr (HG == 1) {
+    xcd_block(bx, by, bz);
+  } else {
+    // One row of the blocks that have work, a KV head's together.  A block of two groups fills a CU, so they
+    // all run at once only if every XCD and shader engine gets its share; with a grid row per query head, empty
+    // for dK / dV beyond the KV heads, some got twice the others'.  256 blocks: 4 / 2 heads of 128, 32 x 64
+    // 15.6 -> 10.4 us; 16 / 8 heads of 128, 2 x 256 26.0 -> 17.6; of 64, 4 x 128 12.2 -> 9.2.  (Blocks of one
+    // group, two a CU, go either way by it: 32 / 8 heads of 128, 4 x 2048 900 -> 652 us, 8 x 256 51.6 -> 63.5.)
+    constexpr uint32_t QROWS = 16 * NW * HG * RGQ;
+    const uint32_t nq = (a.S + QROWS - 1) / QROWS, ratio = a.NH / nky, group = nkv + ratio * nq;
+    const uint32_t u = xcd_order(blockIdx.x, gridDim.x), row = u / group, r = u % group;
+    bz = row / nky;
+    by = row % nky;
+    bx = r;
+    if (r >= (uint32_t)nkv) {
+      by = by * ratio + (r - nkv) / nq;
+      bx = nkv + (r - nkv) % nq;
+    }
+  }
   if (bx < nkv) {
     if (by < nky) dkdv_block<HT, HD, NW, 1, SPLIT, HG>(a, bx, by, bz, lds, lse_s, ndl_s);
   } else {
@@ -754,7 +773,8 @@ int bwd_hd(const AttnArgs &a, hipStream_t s) {
   constexpr int QROWS = 16 * NW * HG * RGQ;
   const int nblk = a.S / (16 * NW);              // key blocks of dK / dV
   const int nq = (a.S + QROWS - 1) / QROWS;  // query blocks of dQ
-  const dim3 grid(nblk + nq, a.NH, a.B), block(HG * NW * 64);
+  const dim3 grid = HG > 1 ? dim3((nblk * a.NKV + nq * a.NH) * a.B) : dim3(nblk + nq, a.NH, a.B);
+  const dim3 block(HG * NW * 64);
   if constexpr (HG == 1)
     if (a.part && a.NH != a.NKV) {
       hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, true, 1>), grid, block, 0, s, a, nblk, a.NH);
@@ -794,8 +814,8 @@ template <typename HT, int HD>
 int bwd_shape(const AttnArgs &a, hipStream_t s) {
   if (pick_shape(a) == SHAPE_2x1) {
     // Two head groups a dK / dV block (one block a CU: 150 KB of LDS at heads of 128) while all
-    // blocks run at once.  256 tokens, 16 / 8
-    // heads of 128 (128 blocks): 21.5 -> 16.2 us.
+    // blocks run at once.  16 / 8 heads, 256 tokens (128 blocks): heads of 128 22.7 -> 17.4 us, of 64 14.6 ->
+    // 11.2; 4 / 2 heads of 64, 1 x 2048 80 -> 54; bf16 the same.
     const long blocks = (long)a.B * (a.S / 32 * a.NKV + a.S / 64 * a.NH);
     if (!a.part && a.NH / a.NKV % 2 == 0 && blocks <= 256) return bwd_hd<HT, HD, 2, 1, 2>(a, s);
     return bwd_hd<HT, HD, 2, 1>(a, s);
