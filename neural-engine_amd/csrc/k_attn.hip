@@ -731,14 +731,16 @@ int fwd_t(const AttnArgs &a, hipStream_t s) {
 // side: at short sequences each alone leaves half the CUs idle.
 // RGQ: 16-query groups per wave of the dQ blocks (the dK / dV blocks have one of 16 keys).  HG: head
 // groups of the dK / dV blocks, NW waves each; the dQ blocks have HG * NW waves.
-// bf16 heads of 64 on 4 waves keep three waves per SIMD (168 VGPRs): left to itself the compiler took 172
-// for the wider dQ blocks and two waves (batch 4 x 1024, 10 / 5 heads: 73 us on blocks of 64 queries, 84 at
-// two waves, 75 at three, with 36 bytes of spills).  fp16 takes two: at three, with more blocks beside each
-// other on a CU, a launch of one round is slower (12 heads, 1 x 2048: 58 us at two, 68 at three).
-template <typename HT, int HD, int NW, int RGQ, bool SPLIT, int HG>
-__global__ __launch_bounds__(HG * NW * 64)
-    __attribute__((amdgpu_waves_per_eu(HD == 64 && NW == 4 && HT::id == H16B::id ? 3 : 2))) void attn_bwd_kernel(
-        AttnArgs a, int nkv, int nky) {
+// WPE: waves per SIMD to fit.  bf16 heads of 64 on 4 waves keep three (168 VGPRs): left to itself the compiler
+// took 172 for the wider dQ blocks and two waves (batch 4 x 1024, 10 / 5 heads: 73 us on blocks of 64 queries,
+// 84 at two waves, 75 at three, with 36 bytes of spills).  fp16 takes two: at three, with more blocks beside
+// each other on a CU, a launch of one round is slower (12 heads, 1 x 2048: 58 us at two, 68 at three).  So do
+// the wider bf16 blocks while two of them a CU are all there are (4 / 2 heads, 4 x 2048: 100.7 at two waves,
+// 106.6 at three).
+template <typename HT, int HD, int NW, int RGQ, bool SPLIT, int HG, int WPE>
+__global__ __launch_bounds__(HG * NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) void attn_bwd_kernel(AttnArgs a,
+                                                                                                          int nkv,
+                                                                                                          int nky) {
   __shared__ __attribute__((aligned(16))) h16_t lds[HG][2][2 * BLK * (HD + 16)];
   __shared__ __attribute__((aligned(16))) float lse_s[HG][2][BLK], ndl_s[HG][2][BLK];
   int bx, by, bz;
@@ -768,7 +770,7 @@ __global__ __launch_bounds__(HG * NW * 64)
   }
 }
 
-template <typename HT, int HD, int NW, int RGQ, int HG = 1>
+template <typename HT, int HD, int NW, int RGQ, int HG = 1, int WPE = HD == 64 && NW == 4 && HT::id == H16B::id ? 3 : 2>
 int bwd_hd(const AttnArgs &a, hipStream_t s) {
   constexpr int QROWS = 16 * NW * HG * RGQ;
   const int nblk = a.S / (16 * NW);              // key blocks of dK / dV
@@ -777,7 +779,7 @@ int bwd_hd(const AttnArgs &a, hipStream_t s) {
   const dim3 block(HG * NW * 64);
   if constexpr (HG == 1)
     if (a.part && a.NH != a.NKV) {
-      hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, true, 1>), grid, block, 0, s, a, nblk, a.NH);
+      hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, true, 1, WPE>), grid, block, 0, s, a, nblk, a.NH);
       NE_HIP(hipGetLastError());
       if (!a.defer_gqa) {
         const long n4 = (long)a.B * a.S * a.NKV * HD / 4;
@@ -785,29 +787,37 @@ int bwd_hd(const AttnArgs &a, hipStream_t s) {
       }
       return ne_hip_status(hipGetLastError(), "attn_bwd");
     }
-  hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, false, HG>), grid, block, 0, s, a, nblk, a.NKV);
+  hipLaunchKernelGGL((attn_bwd_kernel<HT, HD, NW, RGQ, false, HG, WPE>), grid, block, 0, s, a, nblk, a.NKV);
   return ne_hip_status(hipGetLastError(), "attn_bwd");
 }
 
-// dQ blocks of 128 queries (two groups a wave) instead of 64: half the LDS reads, but half the blocks, so
-// that a launch of few rounds ends with a nearly empty one.  From the time of both at batch 1 to 8 x 192 to
-// 2048, 8 to 16 heads, fp16 and bf16 (us, 64 -> 128 queries a block):
-//  * at least one such block a CU (256);
-//  * heads of 128: not below 448 tokens (320 with 4 query heads per KV head): 16 / 8 heads 8 x 192 24.3 -> 26.7,
-//    8 x 320 41 -> 45, but 8 x 448 60 -> 57, 3 x 1088 147 -> 137, 8 x 2048 659 -> 594; without GQA the dK / dV
-//    blocks are as many as the dQ blocks and it takes 512: 8 / 8 heads 2 x 2048 106 -> 110, 8 x 1024 117 -> 112.
-//    With 4 query heads per KV head the longer dK / dV blocks decide and it goes either way by size: 16 / 4 heads
-//    8 x 448 70 -> 78, 8 x 512 90 -> 83;
-//  * heads of 64: fp16 12 heads 8 x 2048 297 -> 278.  In bf16 the wider block spills a few registers at three
-//    waves per SIMD: not without GQA (12 heads 4 x 1344 78 -> 87), otherwise up to 512 blocks (10 / 5 heads
-//    3 x 1088 79 -> 61, 16 / 4 heads 4 x 1024 137 -> 115; 10 / 5 heads 8 x 1024, 640 blocks, 78 -> 84).
+// dQ blocks of 128 queries (two groups a wave) instead of 64: half the LDS reads, but half the blocks, the
+// one with the first queries half empty where S is an odd multiple of 64.  From the time of both at some 3600
+// shapes of 64 to 2048 tokens, 4 to 32 heads, fp16 and bf16 (us, 64 -> 128 queries a block), of which this rule
+// leaves 125 more than 5% behind the better one:
+//  * at least one such block a CU (256), and S >= 128 (16 / 8 heads of 128, 128 x 64 59.7 -> 63.9);
+//  * fp16, and heads of 128: 8 x 2048 666 -> 611, 20 x 256 78 -> 68, 40 x 128 51.8 -> 47.7, but 320 tokens, of
+//    three blocks one half empty, only with 4 query heads per KV head and few blocks (16 / 8 heads 8 x 320 39.7 ->
+//    43.5, 16 / 4 heads 6 x 320 58.9 -> 52.4, 17 x 320 89.7 -> 96.1), 192 tokens and no GQA just above one a CU at
+//    least (8 x 192 24.1 -> 26.0, 10 x 192 32.2 -> 30.4; 8 / 8 heads of 128 32 x 128 even, 40 x 128 -11%);
+//    without GQA a bf16 head of 128 takes two a CU on longer ones (12 heads 3 x 1088 even, 5 x 1088 120 -> 116);
+//    few KV heads with 2 query heads each leave shader engines uneven (4 / 2 heads 160 x 128 34.3 -> 35.7);
+//  * bf16 heads of 64: the wider block spills a few registers at three waves per SIMD: not without GQA (12
+//    heads 4 x 1344 78 -> 87), otherwise up to 512 blocks (10 / 5 heads 3 x 1088 79 -> 61, 16 / 4 heads 4 x 1024
+//    137 -> 115; 10 / 5 heads 8 x 1024, 640 blocks, 78 -> 84) or, with 4 query heads per KV head, any number of
+//    long ones (16 / 4 heads 8 x 1088 155 -> 128).
 template <typename HT, int HD>
 bool two_query_groups(const AttnArgs &a) {
   const long blocks = (long)((a.S + 127) / 128) * a.NH * a.B;
   const int ratio = a.NH / a.NKV;
-  if (HD == 128) return a.S >= (ratio >= 4 ? 320 : 448) && blocks >= (ratio == 1 ? 512 : 256);
-  if (HT::id == H16F::id) return blocks >= 256;
-  return ratio > 1 && blocks >= 256 && blocks <= 512;
+  const bool bf16 = HT::id == H16B::id, half = a.S == 192 || a.S == 320;
+  if (a.S < 128 || blocks < 256) return false;
+  if (HD == 64 && bf16) return ratio >= 4 ? blocks <= 512 || a.S >= 1024 : ratio > 1 && blocks <= 512 && !half;
+  if (ratio == 2 && a.NKV < 4 && a.S < 256) return false;
+  if (a.S == 192) return (ratio > 1 || HD == 64) && blocks > 256;
+  if (a.S == 320) return ratio >= 4 && blocks <= 400;
+  if (ratio == 1) return blocks >= (HD == 128 && bf16 && a.S >= 448 ? 512 : 257);
+  return true;
 }
 
 template <typename HT, int HD>
@@ -820,7 +830,12 @@ int bwd_shape(const AttnArgs &a, hipStream_t s) {
     if (!a.part && a.NH / a.NKV % 2 == 0 && blocks <= 256) return bwd_hd<HT, HD, 2, 1, 2>(a, s);
     return bwd_hd<HT, HD, 2, 1>(a, s);
   }
-  return two_query_groups<HT, HD>(a) ? bwd_hd<HT, HD, 4, 2>(a, s) : bwd_hd<HT, HD, 4, 1>(a, s);
+  if (!two_query_groups<HT, HD>(a)) return bwd_hd<HT, HD, 4, 1>(a, s);
+  if constexpr (HD == 64 && HT::id == H16B::id) {
+    const long blocks = (long)a.B * (a.S / 64 * (a.part ? a.NH : a.NKV) + (a.S + 127) / 128 * a.NH);
+    if (blocks <= 512) return bwd_hd<HT, HD, 4, 2, 1, 2>(a, s);
+  }
+  return bwd_hd<HT, HD, 4, 2>(a, s);
 }
 
 template <typename HT>

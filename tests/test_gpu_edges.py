@@ -267,11 +267,13 @@ def test_gemm_tiles(M, N, K, layout, epi, fmt):
 
 # dQ blocks of 128 queries: S a multiple of 64 only, so that the block with the first queries is half
 # outside; dK / dV blocks of two head groups (short sequences, 2 or 4 query heads per KV head, up to
-# 256 blocks in all and one more; exactly 256, 240 in rows that the XCDs share unevenly); against float64 autograd.  P and dS are rounded to 16 bits: a few roundings deep.
+# 256 blocks in all and one more; exactly 256, 240 in rows that the XCDs share unevenly); bf16 heads of 64 with
+# 352 and 570 blocks (two and three waves per SIMD); against float64 autograd.  P and dS are rounded to 16 bits: a few roundings deep.
 @pytest.mark.parametrize("B,S,NH,NKV,HD", [(8, 192, 16, 4, 64), (8, 192, 16, 8, 128), (2, 576, 26, 13, 128),
                                            (8, 256, 16, 16, 64), (1, 64, 2, 1, 128), (1, 128, 8, 2, 64),
                                            (2, 192, 6, 3, 128), (1, 512, 16, 8, 128), (1, 576, 16, 8, 64),
-                                           (32, 64, 4, 2, 64), (2, 256, 16, 8, 128), (10, 64, 16, 4, 64)])
+                                           (32, 64, 4, 2, 64), (2, 256, 16, 8, 128), (10, 64, 16, 4, 64),
+                                           (6, 576, 10, 5, 64)])
 @pytest.mark.parametrize("fmt", ["fp16", "bf16"])
 def test_attn_bwd_two_groups(fmt, B, S, NH, NKV, HD):
     dt, tdt, _, u = FMT[fmt]
