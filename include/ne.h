@@ -292,8 +292,7 @@ int ne_k_qk_prep_fwd(int dtype, const void *qkv, int64_t ld, const float *cosb,
                      void *stream);
 /* Backward of ne_k_qk_prep_fwd: dq [T,NH*HD], dk [T,NKV*HD] fp32 -> q/k column blocks of
  * dqkv; gain grads (times dg_scale) accumulate into dgq/dgk.  TD/cpu_ops.h:510-537.  Any
- * even ld and 4-byte aligned qkv, dqkv (8-byte dq, dk) will do; with ld % 8 == 0 and all
- * 16-byte aligned a faster form runs, with the same dqkv bits. */
+ * even ld and 4-byte aligned qkv, dqkv (8-byte dq, dk) will do. */
 int ne_k_qk_prep_bwd(int dtype, const float *dq, const float *dk, const void *qkv, int64_t ld,
                      const float *cosb, const float *sinb, const float *gq, const float *gk,
                      const float *rq, const float *rk, void *dqkv, float *dgq, float *dgk,

@@ -661,18 +661,29 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_kernel(
   }
 }
 
+struct Rows16 {
+  typedef f32x4 f4;
+  typedef u16x8 h8;
+};
+struct Rows4 {
+  typedef f32x4 f4 __attribute__((aligned(4)));
+  typedef u16x8 h8 __attribute__((aligned(4)));
+};
+
 // The same backward where there are no partials to write or read (the kernel entry point: it has no
-// scratch) and every access can be 16 bytes (the launcher checks).  HBM-bound: reads dq, dk (fp32) and
+// scratch).  ROWS: the vector types' alignment, 16 bytes where every row starts on 16 (the launcher checks), else
+// 4.  HBM-bound: reads dq, dk (fp32) and
 // the q and k columns of qkv, writes their columns of dqkv.  A head slot (one head of one token) is
 // HD/8 consecutive lanes owning 8 elements each; a block takes tok_per_block tokens and its slots run
 // over the (token, head) items of those, so a lane meets the same 8 columns of a head every time and
 // keeps their q- and k-gain sums in registers for the whole block: they meet in LDS once, at its end,
 // and leave as one atomic per channel and block.  The kernel above (one head per block, 4- and 8-byte
 // accesses, the atomics of every head's blocks on the same lines, about 22 ns each, one after the other)
-// takes 171 us for 16,384 tokens of 16 + 8 heads of 128, 698 us for 3264 and 52 us for 256; this one 95
-// (408 MB: 4.3 TB/s), 25 and 7.6 us.  The same products in the same order of sums as that kernel (a lane's
-// 4 pairs are the butterfly's first two strides; fused multiply-adds written out): the same dqkv bits.
-template <typename HT, bool QKN, int HD>
+// takes 171 us for 16,384 tokens of 16 + 8 heads of 128, 698 us for 3264 and 52 us for 256; this one 94
+// (408 MB: 4.3 TB/s), 24.5 and 7.9 us, and 95, 24.5 and 7.8 on rows of 2 elements more.  The same products in
+// the same order of sums as that kernel (a lane's 4 pairs are the butterfly's first two strides; fused
+// multiply-adds written out): the same dqkv bits.
+template <typename HT, bool QKN, int HD, typename ROWS>
 __global__ __launch_bounds__(256) void qk_prep_bwd_wide_kernel(
     const float *__restrict__ dq, const float *__restrict__ dk, const h16_t *__restrict__ qkv, long ld,
     const float *__restrict__ cosb, const float *__restrict__ sinb, const float *__restrict__ gq,
@@ -680,6 +691,8 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_wide_kernel(
     h16_t *__restrict__ dqkv, float *__restrict__ dgq, float *__restrict__ dgk, float dg_scale, int T,
     int S, int NH, int NKV, int tok_per_block, int *ovf) {
   constexpr int TPH = HD / 8, HALF = HD / 2, SPB = 256 / TPH;  // lanes per slot, slots per block
+  typedef typename ROWS::f4 f4;
+  typedef typename ROWS::h8 h8;
   const int j = threadIdx.x % TPH;
   const int slots = NH + NKV;
   const int t0 = blockIdx.x * tok_per_block, nt = min(tok_per_block, T - t0);
@@ -693,7 +706,7 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_wide_kernel(
   }
   // An item's loads are issued before the item before it is worked on: two items are in flight per lane.
   struct Item {
-    float4 d[2], c4, s4;
+    f32x4 d[2], c4, s4;
     u16x8 pr;
     float r;
   };
@@ -703,13 +716,13 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_wide_kernel(
     const int h = w % slots;
     const bool isq = h < NH;
     const float *p = isq ? dq + (t * NH + h) * HD + 8 * j : dk + (t * NKV + h - NH) * HD + 8 * j;
-    it.d[0] = *(const float4 *)p;
-    it.d[1] = *(const float4 *)(p + 4);
+    it.d[0] = *(const f4 *)p;
+    it.d[1] = *(const f4 *)(p + 4);
     const long pos = t % S;
-    it.c4 = *(const float4 *)(cosb + pos * HALF + 4 * j);
-    it.s4 = *(const float4 *)(sinb + pos * HALF + 4 * j);
+    it.c4 = *(const f4 *)(cosb + pos * HALF + 4 * j);
+    it.s4 = *(const f4 *)(sinb + pos * HALF + 4 * j);
     if (QKN) {
-      it.pr = *(const u16x8 *)(qkv + t * ld + (long)h * HD + 8 * j);  // the k heads follow the q heads
+      it.pr = *(const h8 *)(qkv + t * ld + (long)h * HD + 8 * j);  // the k heads follow the q heads
       it.r = isq ? rq[t * NH + h] : rk[t * NKV + h - NH];
     }
   };
@@ -718,8 +731,8 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_wide_kernel(
     const long t = t0 + w / slots;
     const int h = w % slots;
     const bool isq = h < NH;
-    const float cv[4] = {it.c4.x, it.c4.y, it.c4.z, it.c4.w}, sv[4] = {it.s4.x, it.s4.y, it.s4.z, it.s4.w};
-    const float in[8] = {it.d[0].x, it.d[0].y, it.d[0].z, it.d[0].w, it.d[1].x, it.d[1].y, it.d[1].z, it.d[1].w};
+    const f32x4 &cv = it.c4, &sv = it.s4;
+    const float in[8] = {it.d[0][0], it.d[0][1], it.d[0][2], it.d[0][3], it.d[1][0], it.d[1][1], it.d[1][2], it.d[1][3]};
     u16x8 o;
     if (!QKN) {
 #pragma unroll
@@ -757,7 +770,7 @@ __global__ __launch_bounds__(256) void qk_prep_bwd_wide_kernel(
     }
 #pragma unroll
     for (int e = 0; e < 8; e++) bad |= HT::bad(o[e]);
-    *(u16x8 *)(dqkv + t * ld + (long)h * HD + 8 * j) = o;
+    *(h8 *)(dqkv + t * ld + (long)h * HD + 8 * j) = o;
   };
   int w = threadIdx.x / TPH;
   Item ia, ib;
@@ -928,24 +941,29 @@ int launch_qk_prep_bwd(int dt, const float *dq, const float *dk, const h16_t *qk
   if (HD != 64 && HD != 128) return ne_fail(NE_ERR_ARG, "qk_prep: head_dim %d not in {64,128}", HD);
   if (T <= 0) return ne_fail(NE_ERR_ARG, "qk_prep: T = %d", T);
   if (kvpart && (ld % 2 || NH % NKV)) return ne_fail(NE_ERR_ARG, "qk_prep: bad layout for the dK/dV partials");
-  // The wide form: no partials, 16-byte rows, and enough tokens: without gains (no atomics to save) 192
+  // The wide form: no partials, even rows, and enough tokens: without gains (no atomics to save) 192
   // tokens of 16 + 8 heads of 128 take 3.7 us on one head a block and 2.9 on this, 2048 tokens 17.2 and
   // 7.1, but 64 tokens 2.8 and 3.5.
   const uintptr_t align = (uintptr_t)dq | (uintptr_t)dk | (uintptr_t)qkv | (uintptr_t)dqkv | (uintptr_t)cosb | (uintptr_t)sinb;
-  if (!part && !kvpart && ld % 8 == 0 && !(align & 15) && (gq || T >= 192)) {
+  if (!part && !kvpart && ld % 2 == 0 && !(align & 3) && (gq || T >= 192)) {
     const int tpb = qk_tpb_wide(T, gq != nullptr);
     return DISPATCH_H16(dt, [&] {
       auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((T + tpb - 1) / tpb), dim3(256), 0, s, dq, dk, qkv, ld, cosb, sinb, gq, gk, rq,
                            rk, dqkv, dgq, dgk, dg_scale, T, S, NH, NKV, tpb, ovf);
       };
-      if (HD == 128) {
-        if (gq) go(qk_prep_bwd_wide_kernel<HT, true, 128>);
-        else go(qk_prep_bwd_wide_kernel<HT, false, 128>);
-      } else {
-        if (gq) go(qk_prep_bwd_wide_kernel<HT, true, 64>);
-        else go(qk_prep_bwd_wide_kernel<HT, false, 64>);
-      }
+      auto form = [&](auto rows) {
+        typedef decltype(rows) R;
+        if (HD == 128) {
+          if (gq) go(qk_prep_bwd_wide_kernel<HT, true, 128, R>);
+          else go(qk_prep_bwd_wide_kernel<HT, false, 128, R>);
+        } else {
+          if (gq) go(qk_prep_bwd_wide_kernel<HT, true, 64, R>);
+          else go(qk_prep_bwd_wide_kernel<HT, false, 64, R>);
+        }
+      };
+      if (ld % 8 == 0 && !(align & 15)) form(Rows16{});
+      else form(Rows4{});
       return ne_hip_status(hipGetLastError(), "qk_prep_bwd");
     }());
   }

@@ -80,9 +80,9 @@ def test_qk_prep_bwd_edges(fmt, T, S, NH, NKV, HD, pad, qk):
         assert rel_l2(host(dgq), 1 + 2 * dgqr) < 1e-4 and rel_l2(host(dgk), 1 + 2 * dgkr) < 1e-4
 
 
-# The sums behind dqkv have one order, whichever form runs (16-byte rows: the wide one; a pitch or a base that
-# is not: one head a block, which the training step uses too): a head's products by pairs, the pairs in a
-# butterfly of strides 1, 2, 4 ..., fused multiply-adds where written here.  Restated in numpy (a float64
+# The sums behind dqkv have one order, whichever form runs (the wide one, on 16-byte rows or on a pitch or a base
+# that is not; one head a block for few tokens without gains, which the training step uses too): a head's
+# products by pairs, the pairs in a butterfly of strides 1, 2, 4 ..., fused multiply-adds where written here.  Restated in numpy (a float64
 # product of two float32 values is exact), so every element has the same bits; the two forms' borders
 # (191 / 192 tokens without gains), one token, and an empty last pass.
 @pytest.mark.parametrize("fmt", ["fp16", "bf16"])
