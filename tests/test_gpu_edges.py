@@ -137,11 +137,12 @@ def test_qk_prep_bwd_bits(fmt, T, NH, NKV, HD, qk):
 
 
 # Sampling runs a row of logits in chunks of at least 1024 columns: one chunk, two, a last chunk shorter
-# than the others; peaked (gain 8) and flat (gain 1) distributions, with and without the top-p mask.
+# than the others, and without the mask up to 2048 columns in one block; peaked (gain 8) and flat (gain 1) distributions, with and without the top-p mask.
 # A pick may differ from the oracle's only where its uniform lies within 1e-5 of the boundary between
 # the two in cumulative probability (the fp32 logits and their softmax, 32k terms of rounding 6e-8).
 @pytest.mark.parametrize("V,B,gain,top_p", [(512, 1, 8.0, 0.9), (1024, 3, 1.0, 1.0), (2112, 5, 8.0, 0.95),
-                                            (2112, 2, 1.0, 0.5), (32064, 1, 8.0, 0.9), (32064, 6, 1.0, 1.0)])
+                                            (2112, 2, 1.0, 0.5), (2048, 2, 1.0, 1.0), (2112, 3, 1.0, 1.0),
+                                            (32064, 1, 8.0, 0.9), (32064, 6, 1.0, 1.0)])
 def test_decode_sampling_chunks(V, B, gain, top_p):
     cfg = om.tiny(vocab=V)
     P = {k: om.round_bf16(v) for k, v in om.init_params(cfg, seed=V).items()}
